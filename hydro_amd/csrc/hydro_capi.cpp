@@ -80,7 +80,7 @@ struct hydro_amd_grid {
   long state_ver = 1;
   long cour_ver = 0;     // state version whose CFL maxima the slots hold (0: none)
   bool cour_dirty = false;
-  SweepTune tune = {64, 1, 4, 8};  // set by precision at creation
+  SweepTune tune = {0, 1, 4, 8};  // set by precision at creation
   // host mirror of the run control, valid between calls
   double t = 0, dt = 0;
   int nstep = 0;
@@ -259,7 +259,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   g->esz = dbl(g) ? sizeof(double) : sizeof(float);
   // the 4-wave LDS x form in both precisions (FP64: within 2 % of the DPP
   // form at 8192^2 and faster on small grids; mixed: its fastest form)
-  g->tune = dbl(g) ? SweepTune{64, 1, 4, 8} : SweepTune{64, 4, 4, 16};
+  g->tune = dbl(g) ? SweepTune{0, 1, 4, 8} : SweepTune{0, 4, 4, 16};
   g->geom.nx = p->nx;
   g->geom.ny = p->ny;
   g->geom.pitch = ((long) p->nx + 4 + 31) / 32 * 32;
@@ -860,8 +860,11 @@ extern "C" int hydro_amd_grid_autotune(hydro_amd_grid* g, int reps, int* best) {
   // Candidates are timed in two passes, in opposite orders, and scored by
   // the sum, so a clock that drifts during tuning favours none of them.
   std::vector<SweepTune> ys;
-  for (int yseg : {16, 32, 64, 128, 256, 512}) {
+  const long ncb = (g->p.nx + 63) / 64;
+  for (int yseg : {1, 2, 4, 8, 16, 32, 64, 128, 256, 512}) {
     if (yseg > 4 * g->p.ny && yseg != 16) continue;
+    // short segments are for grids with few columns (y_rows, hydro_kernels.hip)
+    if (yseg < 16 && ncb * ((g->p.ny + yseg - 1) / yseg) > 16384) continue;
     for (int yw : {1, 2, 4}) {
       SweepTune t = cur;
       t.yseg = yseg;

@@ -234,6 +234,26 @@ void launch_boundary(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S
                      ph.bd, ph.bu, src, dst2, has2, ctl);
 }
 
+// Rows each y-sweep wave marches when the caller has not said.  A wave of n
+// rows starts with work worth about one more row (four rows' loads and
+// primitives, one flux), so long segments waste less; but the launch lasts as
+// long as its longest wave, and a wave's rows follow one another, so short
+// ones end earlier and spread more evenly.  With W = column blocks x rows wave
+// rows on a fixed number of SIMDs the two costs, W / n and n, balance at n
+// proportional to sqrt(W); the measured best lengths lie at sqrt(W) / 32 from
+// 250x125 (1 row) to 8192x8192 (32).  Time of a step, FP64 / fast / mixed
+// forms, against the 64 rows (16 on small grids) that every size took before:
+// 250x125 34 / 28 / 25 us against 85 / 52 / 46; 1021x767 84 / 57 / 46 against
+// 108 / 71 / 59; 4099x3001 595 / 376 / 227 against 653 / 382 / 263.  Past
+// `most` rows nothing is won: 8192x8192, fast form, 1.81-1.83 ms at 32 rows,
+// 1.83-1.85 at 64; 16384x12000, FP64 form, 8.13 at 32, 8.09 at 64, 8.16 at 128.
+static int y_rows(long ncolblk, long ny, int most) {
+  int n = 1;
+  while (n < most && 1024L * (n + 1) * (n + 1) <= ncolblk * ny) n++;
+  const long nseg = cdiv(ny, n);  // even segments: none ends the launch alone
+  return (int) cdiv(ny, nseg);
+}
+
 // The sweep launch for one arithmetic form FD (shapes as in launch_sweep).
 template <typename S, int FD>
 static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, double dx,
@@ -276,13 +296,16 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     DISPATCH(HX);
 #undef HX
   } else {
-    int yseg = tune.yseg > 0 ? tune.yseg : 64;
     const int yw = tune.ywaves > 0 ? tune.ywaves : 1;
     const int ncolblk = (int) cdiv(g.nx, 64);
-    // a narrow or short grid has few columns to march: shorten the segments
-    // (down to 16 rows; each adds a 4-row halo) until there are about two
-    // waves per SIMD, rather than leave most of the GPU idle
-    while (yseg > 16 && (long) ncolblk * cdiv(g.ny, yseg) < 2048) yseg >>= 1;
+    int yseg = tune.yseg;
+    if (yseg <= 0) {
+      yseg = y_rows(ncolblk, g.ny, FD == kFast ? 32 : 64);
+    } else {
+      // a given length: shortened (down to 16 rows) until there are about two
+      // waves per SIMD, rather than leave most of the GPU idle
+      while (yseg > 16 && (long) ncolblk * cdiv(g.ny, yseg) < 2048) yseg >>= 1;
+    }
     const int nsg = (int) cdiv(g.ny, (long) yseg * yw);
 #define HY(A, B)                                                                             \
   hipLaunchKernelGGL((k_sweep_y<S, A, B, FD>), dim3((unsigned) ncolblk * nsg), dim3(64 * yw), \

@@ -50,7 +50,7 @@ constexpr int kCourSlots = 1024;
 constexpr int kXSeg = 60;
 
 struct SweepTune {
-  int yseg;     // rows per y-sweep thread (column march length)
+  int yseg;     // rows per y-sweep thread (column march length); 0: by the grid's size
   int ywaves;   // waves per y-sweep workgroup (1..4)
   int xwaves;   // waves per x-sweep workgroup (1..4)
   int xiter;    // row segments each x-sweep wave walks
