@@ -415,6 +415,11 @@ static int inst_yseg(const hydro_amd_batch* b, int ny) {
   return (int) ((ny + W * nrg - 1) / (W * nrg));
 }
 
+// The sweeps form the ghosts of all but very narrow instances.
+static bool folds_ghosts(const Inst& in) {
+  return in.p.nx >= kGhostMin && in.p.ny >= kGhostMin;
+}
+
 template <typename S>
 static InstDev<S> inst_dev(hydro_amd_batch* b, int id) {
   const Inst& in = b->inst[id];
@@ -433,6 +438,7 @@ static InstDev<S> inst_dev(hydro_amd_batch* b, int id) {
   d.br = in.p.boundary_right;
   d.bd = in.p.boundary_down;
   d.bu = in.p.boundary_up;
+  d.fold = folds_ghosts(in);
   d.nseg = (in.p.nx + kXSeg - 1) / kXSeg;
   d.yseg = inst_yseg(b, in.p.ny);
   return d;
@@ -454,11 +460,12 @@ static void tasks_of(const hydro_amd_batch* b, int id, int kind, std::vector<BTa
   }
 }
 
-// Ghost fills of one instance in direction idim, kBoundaryChunk (line, var)
+// Ghost fills of one narrow instance in direction idim, kBoundaryChunk (line, var)
 // pairs per task so a large instance spreads over many workgroups.
 static void boundary_tasks_of(const hydro_amd_batch* b, int id, int idim,
                               std::vector<BTask>& out) {
   const Inst& in = b->inst[id];
+  if (folds_ghosts(in)) return;
   const int nl = idim == 1 ? in.p.ny : in.p.nx;
   for (int a = 0; a < 4 * nl; a += kBoundaryChunk) out.push_back(BTask{id, idim, a, 0});
 }
@@ -539,27 +546,27 @@ static int rebuild(hydro_amd_batch* b) {
 // reading buffer `phase`; q: the list's two task-queue counters.
 template <typename S>
 static void sweep_list(hydro_amd_batch* b, int kind, const InstDev<S>* I, int k, int phase,
-                       int nblk, uint64_t* q) {
+                       bool ghosts, int nblk, uint64_t* q) {
   if constexpr (sizeof(S) == 8) {
     if (b->prec == HYDRO_AMD_FP64_FAST) {
-      launch_batch_sweep_fast(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, b->tune,
-                              nblk, q, b->st);
+      launch_batch_sweep_fast(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
+                              b->tune, nblk, q, b->st);
       return;
     }
   }
-  launch_batch_sweep<S>(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, b->tune, nblk,
-                        q, b->st);
+  launch_batch_sweep<S>(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
+                        b->tune, nblk, q, b->st);
 }
 
-// One phase: its ghost fills, then its x tasks and its y tasks.
+// One phase: the ghost fills of its narrow instances, then its x tasks and its y tasks.
 template <typename S>
 static void enq_phase(hydro_amd_batch* b, int which, int phase) {
   const InstDev<S>* I = (const InstDev<S>*) b->idev;
   const int x = which == 0 ? 0 : 2, y = x + 1, bd = which == 0 ? 4 : 5;
   launch_batch_boundary<S>(I, b->tasks + b->off[bd], b->n[bd], phase, b->nblk_y, b->st);
   uint64_t* q = b->qctr + 4 * phase;  // x: q[0..1], y: q[2..3]
-  sweep_list<S>(b, 1, I, x, phase, b->nblk_x, q);
-  sweep_list<S>(b, 2, I, y, phase, b->nblk_y, q + 2);
+  sweep_list<S>(b, 1, I, x, phase, true, b->nblk_x, q);
+  sweep_list<S>(b, 2, I, y, phase, true, b->nblk_y, q + 2);
 }
 
 template <typename S>
@@ -725,10 +732,10 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
             const int kind = (k % 2 == 0) ? 1 : 2;
             const int nb = kind == 1 ? b->nblk_x : b->nblk_y;
             if (dbl(b))
-              sweep_list<double>(b, kind, (const InstDev<double>*) b->idev, k, 0, nb,
+              sweep_list<double>(b, kind, (const InstDev<double>*) b->idev, k, 0, false, nb,
                                  b->qctr + 2 * k);
             else
-              sweep_list<float>(b, kind, (const InstDev<float>*) b->idev, k, 0, nb,
+              sweep_list<float>(b, kind, (const InstDev<float>*) b->idev, k, 0, false, nb,
                                 b->qctr + 2 * k);
           }
         }

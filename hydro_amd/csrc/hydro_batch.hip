@@ -41,6 +41,15 @@ __device__ __forceinline__ int next_task(uint64_t* qnext) {
   return t;
 }
 
+// The ghosts of one instance's sweep in direction idim (GhostFill).
+template <typename S>
+__device__ __forceinline__ GhostFill inst_ghosts(const InstDev<S>& d, int idim, int phase,
+                                                 int ghosts) {
+  if (!d.fold) return GhostFill{0, 0, 0};
+  const int to = ghosts ? 1 + phase : 0;  // buffer 0: read in phase 0, written in phase 1
+  return idim == 1 ? GhostFill{d.bl, d.br, to} : GhostFill{d.bd, d.bu, to};
+}
+
 // x tasks of one phase (every task's kind is 1).  ST1: every listed
 // instance has slope_type == 1 (the host splits each phase's lists), so the
 // limiter's multiply/divide by slope_type is compiled out as in single grids.
@@ -51,7 +60,7 @@ __device__ __forceinline__ int next_task(uint64_t* qnext) {
 template <typename S, bool ST1, int FD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_batch_sweep_x(
     const InstDev<S>* __restrict__ inst, const BTask* __restrict__ tasks, int ntask, int phase,
-    int xiter, uint64_t* qnext) {
+    int ghosts, int xiter, uint64_t* qnext) {
   const int wpb = blockDim.x >> 6;
   const int wave = wave_id();
   for (;;) {
@@ -63,6 +72,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     const double dtdx = d.ctl->dt / d.dx;
     const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
     const GridView<S> in = d.buf[phase], out = d.buf[1 - phase];
+    const GhostFill gf = inst_ghosts(d, 1, phase, ghosts);
     // the second sweep of an odd step is an x sweep; it produces the CFL
     // maxima the next (even) step's dt needs
     const bool cour = phase == 1;
@@ -71,9 +81,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
     SegWalk w(tk.a + wave, d.nseg);
     for (int it = 0; it < xiter && w.row < d.g.ny; it++) {
       if (cour)
-        x_segment<S, ST1, true, FD>(d.g, d.ph, tr, dtdx, in, out, w.row, w.seg, cx, cy);
+        x_segment<S, ST1, true, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
       else
-        x_segment<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, w.row, w.seg, cx, cy);
+        x_segment<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
       w.advance(wpb, d.nseg);
     }
     if (cour) commit_courant(cx, cy, d.cour, kInstSlots, t % kInstSlots);
@@ -85,7 +95,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 template <typename S, bool ST1, int FD>
 __global__ __launch_bounds__(256) void k_batch_sweep_y(const InstDev<S>* __restrict__ inst,
                                                        const BTask* __restrict__ tasks,
-                                                       int ntask, int phase, int yseg,
+                                                       int ntask, int phase, int ghosts,
                                                        uint64_t* qnext) {
   const int wpb = blockDim.x >> 6;
   const int wave = wave_id();
@@ -107,12 +117,14 @@ __global__ __launch_bounds__(256) void k_batch_sweep_y(const InstDev<S>* __restr
       const int j1 = min(j0 + d.yseg, d.g.ny + 2);
       extern __shared__ __attribute__((aligned(16))) unsigned char ylds[];
       YStash<S>* ys = reinterpret_cast<YStash<S>*>(ylds) + wave;
-      y_march<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, colok, i, j0, j1, ys, cx, cy);
+      y_march<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, inst_ghosts(d, 2, phase, ghosts),
+                                 colok, i, j0, j1, ys, cx, cy);
     }
   }
 }
 
-// Ghost fills (kind = direction) of (line, var) pairs [a, a + kBoundaryChunk)
+// Ghost fills of the instances too narrow for the sweeps to form theirs
+// (kind = direction): of (line, var) pairs [a, a + kBoundaryChunk)
 // of one instance per task, from buffer `phase` into both buffers.
 template <typename S>
 __global__ __launch_bounds__(256) void k_batch_boundary(const InstDev<S>* inst,
@@ -259,25 +271,26 @@ static int occupancy_fd(int kind, int waves) {
 
 template <typename S, bool ST1, int FD>
 static void launch_sweep_part(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                              int phase, const BatchTune& tn, int nblocks, uint64_t* q,
-                              hipStream_t st) {
+                              int phase, bool ghosts, const BatchTune& tn, int nblocks,
+                              uint64_t* q, hipStream_t st) {
   if (ntask <= 0) return;
   const int nb = ntask < nblocks ? ntask : nblocks;
   if (kind == 1)
     hipLaunchKernelGGL((k_batch_sweep_x<S, ST1, FD>), dim3(nb), dim3(64 * tn.waves), 0, st, inst,
-                       tasks, ntask, phase, tn.xiter, q);
+                       tasks, ntask, phase, (int) ghosts, tn.xiter, q);
   else
     hipLaunchKernelGGL((k_batch_sweep_y<S, ST1, FD>), dim3(nb), dim3(64 * tn.waves),
-                       tn.waves * sizeof(YStash<S>), st, inst, tasks, ntask, phase, tn.yseg, q);
+                       tn.waves * sizeof(YStash<S>), st, inst, tasks, ntask, phase, (int) ghosts, q);
 }
 
 template <typename S, int FD>
 static void launch_batch_sweep_fd(int kind, const InstDev<S>* inst, const BTask* tasks,
-                                  int ntask, int nst1, int phase, const BatchTune& tn,
-                                  int nblocks, uint64_t* q, hipStream_t st) {
-  launch_sweep_part<S, true, FD>(kind, inst, tasks, nst1, phase, tn, nblocks, q, st);
-  launch_sweep_part<S, false, FD>(kind, inst, tasks + nst1, ntask - nst1, phase, tn, nblocks,
-                                  q + 1, st);
+                                  int ntask, int nst1, int phase, bool ghosts,
+                                  const BatchTune& tn, int nblocks, uint64_t* q,
+                                  hipStream_t st) {
+  launch_sweep_part<S, true, FD>(kind, inst, tasks, nst1, phase, ghosts, tn, nblocks, q, st);
+  launch_sweep_part<S, false, FD>(kind, inst, tasks + nst1, ntask - nst1, phase, ghosts, tn,
+                                  nblocks, q + 1, st);
 }
 
 #ifndef HYDRO_FAST_UNIT
@@ -288,10 +301,10 @@ int batch_sweep_occupancy(int kind, int waves) {
 
 template <typename S>
 void launch_batch_sweep(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                        int nst1, int phase, const BatchTune& tn, int nblocks, uint64_t* q,
-                        hipStream_t st) {
-  launch_batch_sweep_fd<S, unit_form<S>()>(kind, inst, tasks, ntask, nst1, phase, tn, nblocks, q,
-                                           st);
+                        int nst1, int phase, bool ghosts, const BatchTune& tn, int nblocks,
+                        uint64_t* q, hipStream_t st) {
+  launch_batch_sweep_fd<S, unit_form<S>()>(kind, inst, tasks, ntask, nst1, phase, ghosts, tn,
+                                           nblocks, q, st);
 }
 #ifdef HYDRO_BASE_UNIT
 template int batch_sweep_occupancy<double>(int, int);
@@ -304,9 +317,10 @@ int batch_sweep_occupancy_fast(int kind, int waves) {
 }
 
 void launch_batch_sweep_fast(int kind, const InstDev<double>* inst, const BTask* tasks,
-                             int ntask, int nst1, int phase, const BatchTune& tn, int nblocks,
-                             uint64_t* q, hipStream_t st) {
-  launch_batch_sweep_fd<double, kFast>(kind, inst, tasks, ntask, nst1, phase, tn, nblocks, q, st);
+                             int ntask, int nst1, int phase, bool ghosts, const BatchTune& tn,
+                             int nblocks, uint64_t* q, hipStream_t st) {
+  launch_batch_sweep_fd<double, kFast>(kind, inst, tasks, ntask, nst1, phase, ghosts, tn, nblocks,
+                                       q, st);
 }
 #endif
 
@@ -341,7 +355,7 @@ void launch_batch_ctl(const InstDev<S>* inst, const int* ids, int nids, bool beg
 
 #define INST_ARITH(S)                                                                            \
   template void launch_batch_sweep<S>(int, const InstDev<S>*, const BTask*, int, int, int,      \
-                                      const BatchTune&, int, uint64_t*, hipStream_t);             \
+                                      bool, const BatchTune&, int, uint64_t*, hipStream_t);       \
   template void launch_batch_courant<S>(const InstDev<S>*, const int*, int, hipStream_t);
 #define INST_MOVE(S)                                                                             \
   template void launch_batch_boundary<S>(const InstDev<S>*, const BTask*, int, int, int,        \

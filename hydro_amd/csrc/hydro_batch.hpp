@@ -21,6 +21,7 @@ struct InstDev {
   RunCtl* ctl;
   uint64_t* cour;         // 2 * kInstSlots
   int bl, br, bd, bu;     // boundary types
+  int fold;               // the sweeps form the ghosts (else k_batch_boundary does)
   int nseg;               // 60-cell segments per row
   int yseg;               // rows each wave marches in this instance's y tasks
 };
@@ -39,12 +40,13 @@ struct BatchTune {
 };
 
 // kind 1: x tasks, 2: y tasks (a phase launches both, on their own tables).
-// The first nst1 tasks belong to instances with slope_type == 1.  q: the two
+// The first nst1 tasks belong to instances with slope_type == 1.  ghosts: the
+// ghost values formed on the way are stored in buffer 0.  q: the two
 // task-queue counters of this list (zero at launch).
 template <typename S>
 void launch_batch_sweep(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                        int nst1, int phase, const BatchTune& tn, int nblocks, uint64_t* q,
-                        hipStream_t st);
+                        int nst1, int phase, bool ghosts, const BatchTune& tn, int nblocks,
+                        uint64_t* q, hipStream_t st);
 template <typename S>
 void launch_batch_boundary(const InstDev<S>* inst, const BTask* tasks, int ntask, int phase,
                            int nblocks, hipStream_t st);
@@ -63,8 +65,8 @@ int batch_sweep_occupancy(int kind, int waves);  // resident workgroups per CU
 // launch_batch_sweep / batch_sweep_occupancy for double, with the kFast
 // arithmetic.
 void launch_batch_sweep_fast(int kind, const InstDev<double>* inst, const BTask* tasks,
-                             int ntask, int nst1, int phase, const BatchTune& tn, int nblocks,
-                             uint64_t* q, hipStream_t st);
+                             int ntask, int nst1, int phase, bool ghosts, const BatchTune& tn,
+                             int nblocks, uint64_t* q, hipStream_t st);
 int batch_sweep_occupancy_fast(int kind, int waves);
 
 }  // namespace hydro

@@ -421,19 +421,28 @@ static void enq_boundary(hydro_amd_grid* g, int idim, int src, const RunCtl* ctl
   });
 }
 
+// The sweeps form their own ghosts, unless the grid is too narrow for that.
+static bool folds_ghosts(const hydro_amd_grid* g) {
+  return g->p.nx >= kGhostMin && g->p.ny >= kGhostMin;
+}
+
+// One sweep with its ghosts, reading buffer `src` and writing the other; the
+// ghost values are left in buffer 0, the state between steps.
 static void enq_sweep(hydro_amd_grid* g, int idim, int src, double dt, const RunCtl* ctl,
                       bool cour) {
   uint64_t* c = cour ? g->cour : nullptr;
+  const int fill = folds_ghosts(g) ? (src == 0 ? 1 : 2) : -1;
+  if (fill < 0) enq_boundary(g, idim, src, ctl);
   timed(g, idim == 1 ? 0 : 1, [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
       launch_sweep_fast(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, c, g->tune,
-                        g->st);
+                        fill, g->st);
     else if (g->prec == HYDRO_AMD_FP64)
       launch_sweep<double>(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, c,
-                           g->tune, g->st);
+                           g->tune, fill, g->st);
     else
       launch_sweep<float>(idim, g->geom, g->ph, g->vf[src], g->vf[1 - src], dt, ctl, c,
-                          g->tune, g->st);
+                          g->tune, fill, g->st);
   });
 }
 
@@ -451,9 +460,7 @@ static void enq_courant(hydro_amd_grid* g, const RunCtl* ctl) {
 static void enq_godunov(hydro_amd_grid* g, int idim_start, double dt, const RunCtl* ctl,
                         bool cour) {
   const int d1 = idim_start == 1 ? 1 : 2, d2 = 3 - d1;
-  enq_boundary(g, d1, 0, ctl);
   enq_sweep(g, d1, 0, dt, ctl, false);
-  enq_boundary(g, d2, 1, ctl);
   enq_sweep(g, d2, 1, dt, ctl, cour);
 }
 
@@ -726,16 +733,17 @@ static double time_sweep(hydro_amd_grid* g, int idim, const SweepTune& t, int re
     (void) hipEventDestroy(a);
     return 1e30;
   }
+  const int fill = folds_ghosts(g) ? 0 : -1;
   auto launch = [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
       launch_sweep_fast(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, cour, t,
-                        g->st);
+                        fill, g->st);
     else if (g->prec == HYDRO_AMD_FP64)
       launch_sweep<double>(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, cour, t,
-                           g->st);
+                           fill, g->st);
     else
       launch_sweep<float>(idim, g->geom, g->ph, g->vf[0], g->vf[1], 1e-12, nullptr, cour, t,
-                          g->st);
+                          fill, g->st);
   };
   launch();  // warm
   (void) hipEventRecord(a, g->st);

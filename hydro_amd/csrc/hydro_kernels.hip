@@ -24,7 +24,7 @@ namespace hydro {
 template <typename S, bool ST1, bool COUR, int FD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_sweep_x(GridGeom g, Phys<S> ph, double dx,
                                                  double dt_val, const RunCtl* ctl,
-                                                 GridView<S> in, GridView<S> out,
+                                                 GridView<S> in, GridView<S> out, GhostFill gf,
                                                  uint64_t* cour, int nseg, int xiter) {
   double dt = dt_val;
   if (ctl) {
@@ -38,7 +38,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
   // segments (blockIdx.x * xiter + it) * wpb + wave, it = 0 .. xiter-1
   SegWalk w((int) blockIdx.x * xiter * wpb + wave_id(), nseg);
   for (int it = 0; it < xiter && w.row < g.ny; it++) {
-    x_segment<S, ST1, COUR, FD>(g, ph, tk, dtdx, in, out, w.row, w.seg, cx, cy);
+    x_segment<S, ST1, COUR, FD>(g, ph, tk, dtdx, in, out, gf, w.row, w.seg, cx, cy);
     w.advance(wpb, nseg);
   }
   if (COUR) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
@@ -50,7 +50,8 @@ template <typename S, bool ST1, bool COUR, int W, int FD>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(5))) void k_sweep_xb(GridGeom g, Phys<S> ph, double dx,
                                                      double dt_val, const RunCtl* ctl,
                                                      GridView<S> in, GridView<S> out,
-                                                     uint64_t* cour, int nseg, int xiter) {
+                                                     GhostFill gf, uint64_t* cour, int nseg,
+                                                     int xiter) {
   __shared__ XLds<S, W> sh;
   double dt = dt_val;
   if (ctl) {
@@ -60,8 +61,8 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(5))) voi
   const double dtdx = dt / dx;  // hydro_godunov.c:101
   const TraceK<S> tk = make_tracek<S>((S) dtdx, ph.scheme);
   double cx = 0.0, cy = 0.0;
-  x_blocks<S, ST1, COUR, W, FD>(g, ph, tk, dtdx, in, out, (int) blockIdx.x * xiter, xiter, nseg,
-                                sh, cx, cy);
+  x_blocks<S, ST1, COUR, W, FD>(g, ph, tk, dtdx, in, out, gf, (int) blockIdx.x * xiter, xiter,
+                                nseg, sh, cx, cy);
   if (COUR) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
 }
 
@@ -72,7 +73,7 @@ __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(5))) voi
 template <typename S, bool ST1, bool COUR, int FD>
 __global__ __launch_bounds__(256) void k_sweep_y(GridGeom g, Phys<S> ph, double dx,
                                                  double dt_val, const RunCtl* ctl,
-                                                 GridView<S> in, GridView<S> out,
+                                                 GridView<S> in, GridView<S> out, GhostFill gf,
                                                  uint64_t* cour, int yseg, int ncolblk) {
   double dt = dt_val;
   if (ctl) {
@@ -92,7 +93,7 @@ __global__ __launch_bounds__(256) void k_sweep_y(GridGeom g, Phys<S> ph, double 
     const int j1 = min(j0 + yseg, g.ny + 2);  // rows [j0, j1) are updated
     extern __shared__ __attribute__((aligned(16))) unsigned char ylds[];
     YStash<S>* ys = reinterpret_cast<YStash<S>*>(ylds) + wave_id();
-    y_march<S, ST1, COUR, FD>(g, ph, tk, dtdx, in, out, colok, i, j0, j1, ys, cx, cy);
+    y_march<S, ST1, COUR, FD>(g, ph, tk, dtdx, in, out, gf, colok, i, j0, j1, ys, cx, cy);
   }
   if (COUR) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
 }
@@ -257,8 +258,9 @@ static int y_rows(long ncolblk, long ny, int most) {
 // The sweep launch for one arithmetic form FD (shapes as in launch_sweep).
 template <typename S, int FD>
 static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, double dx,
-                            GridView<S> in, GridView<S> out, double dt_val, const RunCtl* ctl,
-                            uint64_t* cour, const SweepTune& tune, bool st1, hipStream_t st) {
+                            GridView<S> in, GridView<S> out, const GhostFill& gf, double dt_val,
+                            const RunCtl* ctl, uint64_t* cour, const SweepTune& tune, bool st1,
+                            hipStream_t st) {
   const bool c = cour != nullptr;
 #define DISPATCH(F)                         \
   do {                                      \
@@ -277,7 +279,7 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     const dim3 grid(cdiv(pieces, xiter)), blk(64 * W);
 #define HXB(A, B, WW) \
   hipLaunchKernelGGL((k_sweep_xb<S, A, B, WW, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, \
-                     in, out, cour, nseg, xiter)
+                     in, out, gf, cour, nseg, xiter)
 #define HXW(A, B) do { if (W == 2) HXB(A, B, 2); else HXB(A, B, 4); } while (0)
     DISPATCH(HXW);
 #undef HXW
@@ -292,7 +294,7 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     const dim3 grid(cdiv(waves, (long) xw * xiter)), blk(64 * xw);
 #define HX(A, B) \
   hipLaunchKernelGGL((k_sweep_x<S, A, B, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, in, \
-                     out, cour, nseg, xiter)
+                     out, gf, cour, nseg, xiter)
     DISPATCH(HX);
 #undef HX
   } else {
@@ -309,19 +311,27 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     const int nsg = (int) cdiv(g.ny, (long) yseg * yw);
 #define HY(A, B)                                                                             \
   hipLaunchKernelGGL((k_sweep_y<S, A, B, FD>), dim3((unsigned) ncolblk * nsg), dim3(64 * yw), \
-                     yw * sizeof(YStash<S>), st, g, ph, dx, dt_val, ctl, in, out, cour, yseg,  \
-                     ncolblk)
+                     yw * sizeof(YStash<S>), st, g, ph, dx, dt_val, ctl, in, out, gf, cour,    \
+                     yseg, ncolblk)
     DISPATCH(HY);
 #undef HY
   }
 #undef DISPATCH
 }
 
+// The ghosts of one sweep: formed by it (fill 0..2, see GhostFill::to), or in
+// memory already (fill < 0).
+static GhostFill ghost_fill(int idim, const PhysArgs& pa, int fill) {
+  if (fill < 0) return GhostFill{0, 0, 0};
+  return idim == 1 ? GhostFill{pa.bl, pa.br, fill} : GhostFill{pa.bd, pa.bu, fill};
+}
+
 #ifndef HYDRO_FAST_UNIT
 template <typename S>
 void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> in,
                   GridView<S> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                  const SweepTune& tune, hipStream_t st) {
+                  const SweepTune& tune, int fill, hipStream_t st) {
+  const GhostFill gf = ghost_fill(idim, pa, fill);
   const Phys<S> ph = make_phys<S>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type, pa.niter,
                                   pa.iorder, pa.scheme);
   const bool st1 = pa.slope_type == 1.0;
@@ -336,21 +346,24 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
                     (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny
                                : (long) cdiv(g.nx, 64) * cdiv(g.ny, 16)) >= kFastDivWaves;
     if (fd)
-      launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, dt_val, ctl, cour, tune, st1, st);
+      launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
+                                 st);
     else
-      launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, dt_val, ctl, cour, tune, st1, st);
+      launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
+                                 st);
   } else {
-    launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, dt_val, ctl, cour, tune, st1, st);
+    launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
+                                 st);
   }
 }
 #else
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,
                        GridView<double> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                       const SweepTune& tune, hipStream_t st) {
+                       const SweepTune& tune, int fill, hipStream_t st) {
   const Phys<double> ph = make_phys<double>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type,
                                             pa.niter, pa.iorder, pa.scheme);
-  launch_sweep_fd<double, kFast>(idim, g, ph, pa.dx, in, out, dt_val, ctl, cour, tune,
-                                 pa.slope_type == 1.0, st);
+  launch_sweep_fd<double, kFast>(idim, g, ph, pa.dx, in, out, ghost_fill(idim, pa, fill), dt_val,
+                                 ctl, cour, tune, pa.slope_type == 1.0, st);
 }
 #endif
 
@@ -404,13 +417,13 @@ template void launch_boundary<float>(int, const GridGeom&, const PhysArgs&, Grid
                                      GridView<float>, const RunCtl*, hipStream_t);
 template void launch_sweep<double>(int, const GridGeom&, const PhysArgs&, GridView<double>,
                                    GridView<double>, double, const RunCtl*, uint64_t*,
-                                   const SweepTune&, hipStream_t);
+                                   const SweepTune&, int, hipStream_t);
 template void launch_courant<double>(const GridGeom&, const PhysArgs&, GridView<double>,
                                      uint64_t*, const RunCtl*, hipStream_t);
 #elif defined(HYDRO_MIXED_UNIT)
 template void launch_sweep<float>(int, const GridGeom&, const PhysArgs&, GridView<float>,
                                   GridView<float>, double, const RunCtl*, uint64_t*,
-                                  const SweepTune&, hipStream_t);
+                                  const SweepTune&, int, hipStream_t);
 template void launch_courant<float>(const GridGeom&, const PhysArgs&, GridView<float>,
                                     uint64_t*, const RunCtl*, hipStream_t);
 #endif

@@ -38,6 +38,13 @@ struct GridGeom {
   long pitch;
 };
 
+// The ghost cells of one sweep's direction: the boundary types of its low and
+// high side (<= 0: the ghosts in memory), and where the ghost values go --
+// 1 the buffer that the sweep reads, 2 the one it writes, 0 nowhere.
+struct GhostFill {
+  int lo, hi, to;
+};
+
 struct PhysArgs {
   double gamma, smallr, smallc, slope_type, courant_factor, dx;
   int niter, iorder, scheme;
@@ -49,6 +56,11 @@ constexpr int kCourSlots = 1024;
 // x sweep: one 64-lane wave updates 60 cells of a row.
 constexpr int kXSeg = 60;
 
+// Narrowest grid whose ghosts' sources are all interior cells (but for the
+// high-x source nx+2 of the absorbing type, which nothing rewrites), so that
+// each ghost can be formed on its own.
+constexpr int kGhostMin = 3;
+
 struct SweepTune {
   int yseg;     // rows per y-sweep thread (column march length); 0: by the grid's size
   int ywaves;   // waves per y-sweep workgroup (1..4)
@@ -57,6 +69,10 @@ struct SweepTune {
 };
 
 // ---- launchers (hydro_kernels.hip) -----------------------------------------
+// Ghost cells: launch_sweep fills those of its direction itself (fill_ghosts
+// says where to: 1 the input, 2 the output, 0 nowhere; -1: the ghosts are in
+// memory already, put there by launch_boundary).  It may be asked to on grids
+// of at least kGhostMin cells each way.
 // dt handling: if ctl != nullptr the kernels read dt and the active flag from
 // it; otherwise dt_val is used.  cour (2*kCourSlots uint64, zeroed) receives
 // the CFL maxima of the written state when non-null.
@@ -67,13 +83,13 @@ void launch_boundary(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S
 template <typename S>
 void launch_sweep(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> in,
                   GridView<S> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                  const SweepTune& tune, hipStream_t st);
+                  const SweepTune& tune, int fill_ghosts, hipStream_t st);
 
 // The FP64 fast form's sweeps (hydro_kernels.hip, fast unit): as
 // launch_sweep, with the kFast arithmetic.
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView<double> in,
                        GridView<double> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                       const SweepTune& tune, hipStream_t st);
+                       const SweepTune& tune, int fill_ghosts, hipStream_t st);
 
 template <typename S>
 void launch_courant(const GridGeom& g, const PhysArgs& ph, GridView<S> in, uint64_t* cour,

@@ -151,6 +151,65 @@ struct SegWalk {
   }
 };
 
+// ---- ghost cells in the sweeps ----------------------------------------------
+//
+// A sweep forms the ghost cells of its direction where it loads them, from
+// their interior source cells (make_boundary.c:237-289, 381-433), instead of
+// reading them after a kernel of their own: that launch cost 4.7-8 us before
+// every sweep, as much as the sweep itself on a small grid (250x125, FP64: x
+// sweep 8 us).  The values are also stored (GhostFill::to), since the state
+// that a caller sees includes them; cells that only read ghosts as they are
+// (type <= 0, and the absorbing high-x source) are not written, so no cell is
+// both written by one workgroup and read by another.
+
+// The cell that ghost cell gi (0, 1, n+2 or n+3) of a line of n interior cells
+// takes its value from, in direction idim; gi itself where it
+// keeps its own.  neg: the normal momentum changes sign (reflecting walls).
+__device__ __forceinline__ int ghost_source(int idim, int n, int lo, int hi, int gi, bool& neg) {
+  const bool low = gi < 2;
+  const int typ = low ? lo : hi;
+  neg = typ == 1;
+  if (typ <= 0) return gi;
+  if (typ == 1) return low ? 3 - gi : 2 * n + 3 - gi;
+  // absorbing: the reference's source cells (left 2, right nx+2, down 4, up ny+1)
+  if (typ == 2) return idim == 1 ? (low ? 2 : n + 2) : (low ? 4 : n + 1);
+  return low ? n + gi : gi - n;
+}
+
+// The conserved values at padded column i (at most nx+3 is read) of the row
+// at `base`, ghosts formed; o: where the cell was read (its own place for an
+// interior cell).  edge: the row piece touches ghost columns (wave-uniform).
+template <typename S>
+__device__ __forceinline__ void load_x(const GridGeom& g, const GridView<S>& in,
+                                       const GridView<S>& out, const GhostFill& gf, long base,
+                                       int i, bool edge, long& o, S& U0, S& U1, S& U2, S& U3) {
+  const int ic = i < g.nx + 4 ? i : g.nx + 3;
+  if (!edge) {
+    o = base + ic;
+    U0 = in.p[0][o];
+    U1 = in.p[1][o];
+    U2 = in.p[2][o];
+    U3 = in.p[3][o];
+    return;
+  }
+  bool neg = false;
+  const bool ghost = ic < 2 || ic >= g.nx + 2;
+  const int is = ghost ? ghost_source(1, g.nx, gf.lo, gf.hi, ic, neg) : ic;
+  o = base + is;
+  U0 = in.p[0][o];
+  U1 = in.p[1][o];
+  U2 = in.p[2][o];
+  U3 = in.p[3][o];
+  if (neg) U1 = -U1;
+  if (is != i && i == ic && gf.to != 0) {
+    const GridView<S>& d = gf.to == 1 ? in : out;
+    d.p[0][base + i] = U0;
+    d.p[1][base + i] = U1;
+    d.p[2][base + i] = U2;
+    d.p[3][base + i] = U3;
+  }
+}
+
 // FD, the arithmetic form (hydro_numerics.hpp): kGated -- the range-gated
 // FP64 divisions may be used (FP64 launches with enough waves to keep the
 // SIMDs busy); kIeee -- the IEEE code alone; kFast -- the FP64 fast form.
@@ -158,14 +217,15 @@ template <typename S, bool ST1, bool COUR, int FD>
 __device__ __forceinline__ void x_segment(const GridGeom& g, const Phys<S>& ph,
                                           const TraceK<S>& tk, double dtdx,
                                           const GridView<S>& in, const GridView<S>& out,
-                                          long jrow, int seg, double& cx, double& cy) {
+                                          const GhostFill& gf, long jrow, int seg, double& cx,
+                                          double& cy) {
   const int lane = threadIdx.x & 63;
   const long j = jrow + 2;
   const int i = kXSeg * seg + lane;  // padded column of this lane
-  const int ic = i < g.nx + 4 ? i : g.nx + 3;
-  const long o = j * g.pitch + ic;
-
-  const S U0 = in.p[0][o], U1 = in.p[1][o], U2 = in.p[2][o], U3 = in.p[3][o];
+  const bool edge = seg == 0 || kXSeg * seg + 63 >= g.nx + 2;
+  long o;
+  S U0, U1, U2, U3;
+  load_x<S>(g, in, out, gf, j * g.pitch, i, edge, o, U0, U1, U2, U3);
   Prim<S> pc;
   bool fc = false;
   if constexpr (FD == kFast) {
@@ -270,8 +330,8 @@ template <typename S, bool ST1, bool COUR, int W, int FD>
 __device__ __forceinline__ void x_blocks(const GridGeom& g, const Phys<S>& ph,
                                          const TraceK<S>& tk, double dtdx,
                                          const GridView<S>& in, const GridView<S>& out,
-                                         int first, int npieces, int nseg, XLds<S, W>& sh,
-                                         double& cx, double& cy) {
+                                         const GhostFill& gf, int first, int npieces, int nseg,
+                                         XLds<S, W>& sh, double& cx, double& cy) {
   constexpr int N = 64 * W;
   // the FP64 form's range-gated code has no registers to spare for it
   constexpr bool kPrefetch = FD == kFast || sizeof(S) == 4;
@@ -282,12 +342,9 @@ __device__ __forceinline__ void x_blocks(const GridGeom& g, const Phys<S>& ph,
   auto fetch = [&](const SegWalk& ww) {
     XCell<S> c;
     c.i = (N - 4) * ww.seg + t;
-    const int ic = c.i < g.nx + 4 ? c.i : g.nx + 3;
-    c.o = ((long) ww.row + 2) * g.pitch + ic;
-    c.U0 = in.p[0][c.o];
-    c.U1 = in.p[1][c.o];
-    c.U2 = in.p[2][c.o];
-    c.U3 = in.p[3][c.o];
+    const bool edge = ww.seg == 0 || (N - 4) * ww.seg + N > g.nx + 2;
+    load_x<S>(g, in, out, gf, ((long) ww.row + 2) * g.pitch, c.i, edge, c.o, c.U0, c.U1, c.U2,
+              c.U3);
     return c;
   };
   auto prims = [&](XCell<S>& c) {
@@ -428,27 +485,47 @@ __device__ __forceinline__ Cell<S> stash_get_cell(const S (&b)[4][64], int lane)
   return Cell<S>{b[0][lane], b[1][lane], b[2][lane], b[3][lane]};
 }
 
+// Column i of padded row j (wave-uniform), a ghost row formed from its source.
 template <typename S>
-__device__ __forceinline__ Cell<S> load_y(const GridView<S>& in, long o) {
+__device__ __forceinline__ Cell<S> load_y(const GridGeom& g, const GridView<S>& in,
+                                          const GridView<S>& out, const GhostFill& gf, bool colok,
+                                          int j, long i) {
+  const bool ghost = j < 2 || j >= g.ny + 2;
+  bool neg = false;
+  const int js = ghost ? ghost_source(2, g.ny, gf.lo, gf.hi, j, neg) : j;
+  const long o = (long) js * g.pitch + i;
   // gather with the IU/IV swap of conservar.c:106-109
-  return Cell<S>{in.p[0][o], in.p[2][o], in.p[1][o], in.p[3][o]};
+  Cell<S> u{in.p[0][o], in.p[2][o], in.p[1][o], in.p[3][o]};
+  if (ghost) {  // wave-uniform
+    if (neg) u.u1 = -u.u1;
+    if (js != j && gf.to != 0 && colok) {
+      const GridView<S>& d = gf.to == 1 ? in : out;
+      const long od = (long) j * g.pitch + i;
+      d.p[0][od] = u.u0;
+      d.p[2][od] = u.u1;
+      d.p[1][od] = u.u2;
+      d.p[3][od] = u.u3;
+    }
+  }
+  return u;
 }
 
 template <typename S, bool ST1, bool COUR, int FD>
 __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
                                         const TraceK<S>& tk, double dtdx,
                                         const GridView<S>& in, const GridView<S>& out,
-                                        bool colok, long i, int j0, int j1, YStash<S>* ys,
-                                        double& cx, double& cy) {
+                                        const GhostFill& gf, bool colok, long i, int j0, int j1,
+                                        YStash<S>* ys, double& cx, double& cy) {
   const long P = g.pitch;
   const int lane = threadIdx.x & 63;
   const bool o1 = ph.iorder == 1;
 
   // prologue: cells j0-2 .. j0+1
-  Cell<S> ua = load_y(in, (long) (j0 - 2) * P + i);
-  Cell<S> ub = load_y(in, (long) (j0 - 1) * P + i);
-  Cell<S> uc = load_y(in, (long) j0 * P + i);
-  Cell<S> ud = load_y(in, (long) (j0 + 1) * P + i);
+  auto load = [&](int j) { return load_y<S>(g, in, out, gf, colok, j, i); };
+  Cell<S> ua = load(j0 - 2);
+  Cell<S> ub = load(j0 - 1);
+  Cell<S> uc = load(j0);
+  Cell<S> ud = load(j0 + 1);
   // rows j0 and j0+1 await their updates
   stash_put_cell(ys->u[j0 % 3], lane, uc);
   stash_put_cell(ys->u[(j0 + 1) % 3], lane, ud);
@@ -492,7 +569,7 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
   Q4<S> qC = pcc.q, qD = pd.q;
   S cD = pd.c, rD = pd.rinv, iD = pd.cinv;
   // the next row's loads are issued one row ahead of their use
-  Cell<S> uN = load_y(in, (long) (j0 + 2) * P + i);
+  Cell<S> uN = load(j0 + 2);
   // One row of the march: take row j, prefetch row j+1, update row j-2,
   // shift the window.
   auto row = [&](int j) {
@@ -504,7 +581,7 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
     const int sj = j % 3;  // wave-uniform
     stash_put_cell(ys->u[sj], lane, uE);
     const int jn = j + 1 <= j1 + 1 ? j + 1 : j1 + 1;  // last row: a harmless reload
-    uN = load_y(in, (long) jn * P + i);
+    uN = load(jn);
     const bool fE = cell_ok(uE);
     const Prim<S> pE = prim(uE, fE);
     Q4<S> qxmD, qxpD;
@@ -574,22 +651,13 @@ __device__ __forceinline__ void boundary_line(int idim, const GridGeom& g, int b
   const int normal = (idim == 1) ? 1 : 2;
   const long line = k + 2;
   for (int gp = 0; gp < 4; gp++) {
-    const int lo = gp < 2;
-    const int typ = (idim == 1) ? (lo ? bl : br) : (lo ? bd : bu);
+    const int typ = (idim == 1) ? (gp < 2 ? bl : br) : (gp < 2 ? bd : bu);
     if (typ <= 0) continue;
-    const int gidx = lo ? gp : nn + gp;  // 0, 1, nn+2, nn+3
-    int sidx;
-    S sign = (S) 1;
-    if (typ == 1) {
-      sidx = lo ? 3 - gidx : 2 * nn + 3 - gidx;
-      if (v == normal) sign = (S) -1;
-    } else if (typ == 2) {
-      // reference source cells: left 2, right nn+2, down 4, up ny+1
-      if (idim == 1) sidx = lo ? 2 : nn + 2;
-      else sidx = lo ? 4 : nn + 1;
-    } else {
-      sidx = lo ? nn + gidx : gidx - nn;
-    }
+    const int gidx = gp < 2 ? gp : nn + gp;  // 0, 1, nn+2, nn+3
+    bool neg;
+    const int sidx = idim == 1 ? ghost_source(1, nn, bl, br, gidx, neg)
+                               : ghost_source(2, nn, bd, bu, gidx, neg);
+    const S sign = neg && v == normal ? (S) -1 : (S) 1;
     long od, os;
     if (idim == 1) {
       od = line * g.pitch + gidx;
