@@ -575,7 +575,16 @@ static void enq_step_t(hydro_amd_batch* b, bool flip) {
   launch_batch_ctl<S>(I, b->ids, b->nids, true, b->qctr, b->st);
   enq_phase<S>(b, flip ? 1 : 0, 0);
   enq_phase<S>(b, flip ? 0 : 1, 1);
-  launch_batch_ctl<S>(I, b->ids, b->nids, false, b->qctr, b->st);
+}
+
+// Closes the last step of a run (each step closes the one before it).
+static void enq_close(hydro_amd_batch* b) {
+  if (dbl(b))
+    launch_batch_ctl<double>((const InstDev<double>*) b->idev, b->ids, b->nids, false, b->qctr,
+                             b->st);
+  else
+    launch_batch_ctl<float>((const InstDev<float>*) b->idev, b->ids, b->nids, false, b->qctr,
+                            b->st);
 }
 
 static void enq_step(hydro_amd_batch* b, bool flip) {
@@ -640,6 +649,7 @@ extern "C" int hydro_amd_batch_run_async(hydro_amd_batch* b, int steps) {
     enq_step(b, b->flip);
     b->flip = !b->flip;
   }
+  enq_close(b);
   BCHK(hipGetLastError());
   return 0;
 }

@@ -167,7 +167,9 @@ __global__ __launch_bounds__(256) void k_batch_courant(const InstDev<S>* inst, c
   }
 }
 
-// main.c:244-260 for every listed instance: one wave per instance.  A batch
+// main.c:297-298 and 244-260 for every listed instance, one wave each: closes
+// the step that is open (so that only the last step of a run needs
+// k_batch_ctl_end: one launch of 4.3 us a step less), opens the next.  A batch
 // also stops an instance at its first dt that is not positive and finite
 // (the reference would go on; this only differs for runs that have already
 // broken down) and flags it, so one bad run cannot stall the others.
@@ -179,8 +181,9 @@ __global__ __launch_bounds__(64) void k_batch_ctl_begin(const InstDev<S>* inst, 
   for (int k = blockIdx.x; k < nids; k += gridDim.x) {
     const InstDev<S>& d = inst[ids[k]];
     RunCtl* c = d.ctl;
-    const double t = c->t, tend = c->tend;
-    const int nstep = c->nstep, nstepmax = c->nstepmax;
+    const int open = c->active;
+    const double t = open ? c->t + c->dt : c->t, tend = c->tend;
+    const int nstep = c->nstep + (open ? 1 : 0), nstepmax = c->nstepmax;
     bool act = (t < tend) && (nstep < nstepmax) && !c->fault;
     bool bad = false;
     if (act && (nstep % 2) == 0) {
@@ -190,13 +193,15 @@ __global__ __launch_bounds__(64) void k_batch_ctl_begin(const InstDev<S>* inst, 
       if (threadIdx.x == 0 && !bad) c->dt = dt;
     }
     if (threadIdx.x == 0) {
+      c->t = t;
+      c->nstep = nstep;
       if (bad) c->fault = 1;
       c->active = (act && !bad) ? 1 : 0;
     }
   }
 }
 
-// main.c:297-298
+// main.c:297-298 for the last step of a run
 template <typename S>
 __global__ void k_batch_ctl_end(const InstDev<S>* inst, const int* ids, int nids) {
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -205,6 +210,7 @@ __global__ void k_batch_ctl_end(const InstDev<S>* inst, const int* ids, int nids
   if (!c->active) return;
   c->nstep += 1;
   c->t += c->dt;
+  c->active = 0;
 }
 
 [[maybe_unused]] static inline unsigned cdivu(long a, long b) {

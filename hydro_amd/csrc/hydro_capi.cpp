@@ -71,8 +71,8 @@ struct hydro_amd_grid {
   GridView<double> vd[2];
   GridView<float> vf[2];
   uint64_t* cour = nullptr;
-  RunCtl* ctl = nullptr;
-  RunCtl* hctl = nullptr;   // pinned host copy: every RunCtl / dt transfer goes through it
+  RunCtl* ctl = nullptr;    // [2]: even and odd steps (hydro_kernels.hpp)
+  RunCtl* hctl = nullptr;   // [2], pinned host copy: every RunCtl / dt transfer goes through it
   double* dscal = nullptr;  // device scalar for dt
   double* dlog = nullptr;
   int dlog_cap = 0;
@@ -84,6 +84,7 @@ struct hydro_amd_grid {
   // host mirror of the run control, valid between calls
   double t = 0, dt = 0;
   int nstep = 0;
+  bool queued = false;  // steps were queued that the mirror does not show yet
   // cached two-step graph
   hipGraphExec_t gexec = nullptr;
   bool gexec_cour = false;
@@ -251,6 +252,22 @@ static int validate(const hydro_amd_params* p) {
   return 0;
 }
 
+// The mirror's run control to the device, no step open.
+static int write_ctl(hydro_amd_grid* g) {
+  HIPCHK(hipStreamSynchronize(g->st));  // the pinned copy may still feed a queued copy
+  RunCtl c{};
+  c.t = g->t;
+  c.dt = g->dt;
+  c.tend = g->p.tend;
+  c.nstep = g->nstep;
+  c.nstepmax = g->p.nstepmax;
+  g->hctl[0] = g->hctl[1] = c;
+  g->queued = false;
+  HIPCHK(hipMemcpyAsync(g->ctl, g->hctl, 2 * sizeof(RunCtl), hipMemcpyHostToDevice, g->st));
+  HIPCHK(hipStreamSynchronize(g->st));
+  return 0;
+}
+
 extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   if (validate(p)) return nullptr;
   hydro_amd_grid* g = new hydro_amd_grid();
@@ -271,20 +288,15 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   if (hipStreamCreateWithFlags(&g->st, hipStreamNonBlocking) != hipSuccess ||
       alloc_buffer(g, 0) || alloc_buffer(g, 1) ||
       hipMalloc(&g->cour, 2 * kCourSlots * sizeof(uint64_t)) != hipSuccess ||
-      hipMalloc(&g->ctl, sizeof(RunCtl)) != hipSuccess ||
-      hipHostMalloc(&g->hctl, sizeof(RunCtl), hipHostMallocDefault) != hipSuccess ||
+      hipMalloc(&g->ctl, 2 * sizeof(RunCtl)) != hipSuccess ||
+      hipHostMalloc(&g->hctl, 2 * sizeof(RunCtl), hipHostMallocDefault) != hipSuccess ||
       hipMalloc(&g->dscal, sizeof(double)) != hipSuccess) {
     if (g_err.empty()) fail("device allocation failed");
     hydro_amd_grid_destroy(g);
     return nullptr;
   }
   launch_clear_slots(g->cour, g->st);
-  *g->hctl = RunCtl{};
-  g->hctl->tend = p->tend;
-  g->hctl->nstepmax = p->nstepmax;
-  if (hipMemcpyAsync(g->ctl, g->hctl, sizeof(RunCtl), hipMemcpyHostToDevice, g->st) !=
-          hipSuccess ||
-      hipStreamSynchronize(g->st) != hipSuccess) {
+  if (write_ctl(g)) {
     fail("grid setup failed");
     hydro_amd_grid_destroy(g);
     return nullptr;
@@ -294,25 +306,9 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
 
 extern "C" long long hydro_amd_grid_bytes(const hydro_amd_grid* g) {
   return g ? (long long) (2 * (4 * g->plane + kOrigin + 64) * g->esz +
-                          2 * kCourSlots * sizeof(uint64_t) + sizeof(RunCtl) + 8 +
+                          2 * kCourSlots * sizeof(uint64_t) + 2 * sizeof(RunCtl) + 8 +
                           g->dlog_cap * 8)
            : 0;
-}
-
-static int write_ctl(hydro_amd_grid* g) {
-  HIPCHK(hipStreamSynchronize(g->st));  // the pinned copy may still feed a queued copy
-  RunCtl& c = *g->hctl;
-  c = RunCtl{};
-  c.t = g->t;
-  c.dt = g->dt;
-  c.tend = g->p.tend;
-  c.nstep = g->nstep;
-  c.nstepmax = g->p.nstepmax;
-  c.active = 0;
-  c.log = nullptr;
-  HIPCHK(hipMemcpyAsync(g->ctl, g->hctl, sizeof(RunCtl), hipMemcpyHostToDevice, g->st));
-  HIPCHK(hipStreamSynchronize(g->st));
-  return 0;
 }
 
 static void bump(hydro_amd_grid* g) { g->state_ver++; }
@@ -429,19 +425,19 @@ static bool folds_ghosts(const hydro_amd_grid* g) {
 // One sweep with its ghosts, reading buffer `src` and writing the other; the
 // ghost values are left in buffer 0, the state between steps.
 static void enq_sweep(hydro_amd_grid* g, int idim, int src, double dt, const RunCtl* ctl,
-                      bool cour) {
+                      RunCtl* nxt, bool cour) {
   uint64_t* c = cour ? g->cour : nullptr;
   const int fill = folds_ghosts(g) ? (src == 0 ? 1 : 2) : -1;
   if (fill < 0) enq_boundary(g, idim, src, ctl);
   timed(g, idim == 1 ? 0 : 1, [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
-      launch_sweep_fast(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, c, g->tune,
+      launch_sweep_fast(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, nxt, c, g->tune,
                         fill, g->st);
     else if (g->prec == HYDRO_AMD_FP64)
-      launch_sweep<double>(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, c,
+      launch_sweep<double>(idim, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, nxt, c,
                            g->tune, fill, g->st);
     else
-      launch_sweep<float>(idim, g->geom, g->ph, g->vf[src], g->vf[1 - src], dt, ctl, c,
+      launch_sweep<float>(idim, g->geom, g->ph, g->vf[src], g->vf[1 - src], dt, ctl, nxt, c,
                           g->tune, fill, g->st);
   });
 }
@@ -458,10 +454,10 @@ static void enq_courant(hydro_amd_grid* g, const RunCtl* ctl) {
 // hydro_godunov.c:98-237: boundary + sweep for both directions, state back in
 // buffer 0.  `cour` folds the CFL maxima of the result into the second sweep.
 static void enq_godunov(hydro_amd_grid* g, int idim_start, double dt, const RunCtl* ctl,
-                        bool cour) {
+                        RunCtl* nxt, bool cour) {
   const int d1 = idim_start == 1 ? 1 : 2, d2 = 3 - d1;
-  enq_sweep(g, d1, 0, dt, ctl, false);
-  enq_sweep(g, d2, 1, dt, ctl, cour);
+  enq_sweep(g, d1, 0, dt, ctl, nxt, false);
+  enq_sweep(g, d2, 1, dt, ctl, nullptr, cour);
 }
 
 static void prepare_slots(hydro_amd_grid* g) {
@@ -473,7 +469,7 @@ static void prepare_slots(hydro_amd_grid* g) {
 static int godunov_impl(hydro_amd_grid* g, int idim, double dt, bool want_cour) {
   if (idim != 1 && idim != 2) return fail("idim must be 1 or 2 (got %d)", idim);
   if (want_cour) prepare_slots(g);
-  enq_godunov(g, idim, dt, nullptr, want_cour);
+  enq_godunov(g, idim, dt, nullptr, nullptr, want_cour);
   HIPCHK(hipGetLastError());
   bump(g);
   if (want_cour) {
@@ -524,14 +520,17 @@ extern "C" int hydro_amd_grid_compute_deltat(hydro_amd_grid* g, double* dt) {
 // ---- device time loop ------------------------------------------------------------------
 
 // One step of main.c:244-298 with run control on the device; `n` is the step
-// number the host expects (its parity fixes the sweep order).
+// number the host expects (its parity fixes the sweep order and the control).
 static void enq_step(hydro_amd_grid* g, int n) {
-  launch_ctl_begin(g->ctl, g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, g->st);
-  const bool even = (n % 2) == 0;
-  enq_godunov(g, even ? 1 : 2, 0.0, g->ctl, !even);
-  launch_ctl_end(g->ctl, g->st);
+  if (n % 2 == 0) {
+    launch_ctl_begin(g->ctl, g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, g->st);
+    enq_godunov(g, 1, 0.0, g->ctl, g->ctl + 1, false);
+  } else {
+    enq_godunov(g, 2, 0.0, g->ctl + 1, nullptr, true);
+  }
 }
 
+// The outcome of the queued steps (ctl[0]).
 static int read_ctl(hydro_amd_grid* g, RunCtl* c) {
   HIPCHK(hipMemcpyAsync(g->hctl, g->ctl, sizeof(RunCtl), hipMemcpyDeviceToHost, g->st));
   HIPCHK(hipStreamSynchronize(g->st));
@@ -557,48 +556,10 @@ static int get_graph(hydro_amd_grid* g) {
   return 0;
 }
 
-// `start`, when given, is recorded on the stream right before the first step
-// (the autotuner's clock, which the run control's set-up stays outside of).
-static int run_enqueue(hydro_amd_grid* g, int max_steps, int log_cap,
-                       hipEvent_t start = nullptr) {
-  if (max_steps <= 0) return 0;
-  // dt of an even step comes from the CFL maxima of the current state
-  if (g->nstep % 2 == 0) ensure_cour(g);
-  // log setup + limits
-  RunCtl c;
-  if (read_ctl(g, &c)) return -1;
-  c.tend = g->p.tend;
-  c.nstepmax = g->p.nstepmax;
-  c.log_base = g->nstep;
-  c.log_cap = log_cap;
-  c.log = log_cap > 0 ? g->dlog : nullptr;
-  // read_ctl left the stream idle, so the pinned copy is free; nothing
-  // rewrites it before the next synchronising call
-  *g->hctl = c;
-  HIPCHK(hipMemcpyAsync(g->ctl, g->hctl, sizeof(RunCtl), hipMemcpyHostToDevice, g->st));
-  if (start) HIPCHK(hipEventRecord(start, g->st));
-  int n = g->nstep, left = max_steps;
-  if (n % 2 == 1) {  // finish the odd step first so the graph starts even
-    enq_step(g, n);
-    n++;
-    left--;
-  }
-  if (left >= 2 && !g->prof) {
-    if (get_graph(g)) return -1;
-    for (; left >= 2; left -= 2, n += 2) HIPCHK(hipGraphLaunch(g->gexec, g->st));
-  }
-  for (; left >= 2; left--, n++) enq_step(g, n);
-  if (left == 1) {
-    enq_step(g, n);
-    n++;
-  }
-  HIPCHK(hipGetLastError());
-  return 0;
-}
-
 static int run_finish(hydro_amd_grid* g, int* steps_done) {
   RunCtl c;
   if (read_ctl(g, &c)) return -1;
+  g->queued = false;
   if (g->prof) prof_collect(g);
   const int done = c.nstep - g->nstep;
   if (done > 0) {
@@ -617,6 +578,53 @@ static int run_finish(hydro_amd_grid* g, int* steps_done) {
   g->dt = c.dt;
   g->nstep = c.nstep;
   if (steps_done) *steps_done = done;
+  return 0;
+}
+
+// `start`, when given, is recorded on the stream right before the first step
+// (the autotuner's clock, which the run control's set-up stays outside of).
+static int run_enqueue(hydro_amd_grid* g, int max_steps, int log_cap,
+                       hipEvent_t start = nullptr) {
+  if (max_steps <= 0) return 0;
+  if (g->queued && run_finish(g, nullptr)) return -1;  // the step parity below is the mirror's
+  // dt of an even step comes from the CFL maxima of the current state
+  if (g->nstep % 2 == 0) ensure_cour(g);
+  // control, log setup + limits
+  HIPCHK(hipStreamSynchronize(g->st));  // the pinned copy may still feed a queued copy
+  RunCtl c{};
+  c.t = g->t;
+  c.dt = g->dt;
+  c.nstep = g->nstep;
+  c.tend = g->p.tend;
+  c.nstepmax = g->p.nstepmax;
+  c.log_base = g->nstep;
+  c.log_cap = log_cap;
+  c.log = log_cap > 0 ? g->dlog : nullptr;
+  g->hctl[0] = c;
+  // an odd step to begin with is open from the start
+  c.active = g->nstep % 2 == 1 && (c.t < c.tend) && (c.nstep < c.nstepmax);
+  g->hctl[1] = c;
+  // nothing rewrites the pinned copy before the next synchronising call
+  HIPCHK(hipMemcpyAsync(g->ctl, g->hctl, 2 * sizeof(RunCtl), hipMemcpyHostToDevice, g->st));
+  g->queued = true;
+  if (start) HIPCHK(hipEventRecord(start, g->st));
+  int n = g->nstep, left = max_steps;
+  if (n % 2 == 1) {  // finish the odd step first so the graph starts even
+    enq_step(g, n);
+    n++;
+    left--;
+  }
+  if (left >= 2 && !g->prof) {
+    if (get_graph(g)) return -1;
+    for (; left >= 2; left -= 2, n += 2) HIPCHK(hipGraphLaunch(g->gexec, g->st));
+  }
+  for (; left >= 2; left--, n++) enq_step(g, n);
+  if (left == 1) {
+    enq_step(g, n);
+    n++;
+  }
+  launch_ctl_end(g->ctl, n % 2 == 0, g->st);  // (n: the next step)
+  HIPCHK(hipGetLastError());
   return 0;
 }
 
@@ -736,13 +744,13 @@ static double time_sweep(hydro_amd_grid* g, int idim, const SweepTune& t, int re
   const int fill = folds_ghosts(g) ? 0 : -1;
   auto launch = [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
-      launch_sweep_fast(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, cour, t,
+      launch_sweep_fast(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, nullptr, cour, t,
                         fill, g->st);
     else if (g->prec == HYDRO_AMD_FP64)
-      launch_sweep<double>(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, cour, t,
+      launch_sweep<double>(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, nullptr, cour, t,
                            fill, g->st);
     else
-      launch_sweep<float>(idim, g->geom, g->ph, g->vf[0], g->vf[1], 1e-12, nullptr, cour, t,
+      launch_sweep<float>(idim, g->geom, g->ph, g->vf[0], g->vf[1], 1e-12, nullptr, nullptr, cour, t,
                           fill, g->st);
   };
   launch();  // warm

@@ -18,16 +18,44 @@
 
 namespace hydro {
 
+// ---- run control ---------------------------------------------------------------
+
+// main.c:297-298: the step of c is done (if it ran at all).  Called by one thread.
+__device__ __forceinline__ void close_step(RunCtl& c) {
+  if (!c.active) return;
+  const int k = c.nstep - c.log_base;
+  if (c.log && k >= 0 && k < c.log_cap) c.log[k] = c.dt;
+  c.nstep += 1;
+  c.t += c.dt;
+  c.active = 0;
+}
+
+// The even step's x sweep, workgroup 0: the odd step that follows takes the
+// same dt, so its control is known before the step has run.  Nothing reads
+// *nxt in this launch.  (In a kernel of their own, closing a step and opening
+// the next one took 4.3 + 4.5 us a step, 2 x 5 launches in the two-step graph
+// beside its sweeps; now 1 launch.)
+__device__ __forceinline__ void open_odd_step(const RunCtl* ctl, RunCtl* nxt) {
+  if (!nxt || blockIdx.x != 0 || threadIdx.x != 0) return;
+  RunCtl c = *ctl;
+  if (c.active) {
+    close_step(c);
+    c.active = (c.t < c.tend) && (c.nstep < c.nstepmax);
+  }
+  *nxt = c;
+}
+
 // ---- x sweep ---------------------------------------------------------------
 
 // A workgroup walks wpb * xiter consecutive row segments, wpb at a time.
 template <typename S, bool ST1, bool COUR, int FD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_sweep_x(GridGeom g, Phys<S> ph, double dx,
                                                  double dt_val, const RunCtl* ctl,
-                                                 GridView<S> in, GridView<S> out, GhostFill gf,
-                                                 uint64_t* cour, int nseg, int xiter) {
+                                                 RunCtl* nxt, GridView<S> in, GridView<S> out,
+                                                 GhostFill gf, uint64_t* cour, int nseg, int xiter) {
   double dt = dt_val;
   if (ctl) {
+    open_odd_step(ctl, nxt);
     if (!ctl->active) return;  // grid-uniform
     dt = ctl->dt;
   }
@@ -49,12 +77,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k
 template <typename S, bool ST1, bool COUR, int W, int FD>
 __global__ __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(5))) void k_sweep_xb(GridGeom g, Phys<S> ph, double dx,
                                                      double dt_val, const RunCtl* ctl,
-                                                     GridView<S> in, GridView<S> out,
-                                                     GhostFill gf, uint64_t* cour, int nseg,
+                                                     RunCtl* nxt, GridView<S> in,
+                                                     GridView<S> out, GhostFill gf, uint64_t* cour, int nseg,
                                                      int xiter) {
   __shared__ XLds<S, W> sh;
   double dt = dt_val;
   if (ctl) {
+    open_odd_step(ctl, nxt);
     if (!ctl->active) return;  // grid-uniform
     dt = ctl->dt;
   }
@@ -144,32 +173,30 @@ __global__ __launch_bounds__(64) void k_dt_finalize(uint64_t* cour, double cf, d
   if (threadIdx.x == 0) *dt_out = dt;
 }
 
-// main.c:244-260: open a step.
+// main.c:244-260: open an even step (ctl[0]), after closing the odd one before
+// it if that is open (ctl[1], which holds the run's latest state either way).
 __global__ __launch_bounds__(64) void k_ctl_begin(RunCtl* ctl, uint64_t* cour, double cf,
                                                   double dx, double smallc) {
-  const double t = ctl->t, tend = ctl->tend;
-  const int nstep = ctl->nstep, nstepmax = ctl->nstepmax;
-  const bool act = (t < tend) && (nstep < nstepmax);
-  if (!act) {
-    if (threadIdx.x == 0) ctl->active = 0;
-    return;  // wave-uniform
+  RunCtl c = ctl[1];
+  if (threadIdx.x != 0) c.log = nullptr;  // one thread logs
+  close_step(c);
+  if ((c.t < c.tend) && (c.nstep < c.nstepmax)) {  // wave-uniform
+    c.dt = wave_reduce_dt(cour, kCourSlots, cf, dx, smallc);
+    if (c.nstep == 0) c.dt = c.dt / 2.0;
+    c.active = 1;
   }
-  if ((nstep % 2) == 0) {
-    double dt = wave_reduce_dt(cour, kCourSlots, cf, dx, smallc);
-    if (nstep == 0) dt = dt / 2.0;
-    if (threadIdx.x == 0) ctl->dt = dt;
-  }
-  if (threadIdx.x == 0) ctl->active = 1;
+  if (threadIdx.x == 0) ctl[0] = c;
 }
 
-// main.c:297-298: close a step.
-__global__ void k_ctl_end(RunCtl* ctl) {
-  if (threadIdx.x != 0 || !ctl->active) return;
-  const int n = ctl->nstep;
-  const int k = n - ctl->log_base;
-  if (ctl->log && k >= 0 && k < ctl->log_cap) ctl->log[k] = ctl->dt;
-  ctl->nstep = n + 1;
-  ctl->t += ctl->dt;
+// The run's last step was odd (open in ctl[1]) or even (closed by its x sweep,
+// an odd step opened in ctl[1] that will not run now): the outcome to ctl[0].
+__global__ void k_ctl_end(RunCtl* ctl, int odd) {
+  if (threadIdx.x != 0) return;
+  RunCtl c = ctl[1];
+  if (odd) close_step(c);
+  c.active = 0;
+  ctl[0] = c;
+  ctl[1].active = 0;
 }
 
 __global__ void k_clear_slots(uint64_t* cour) {
@@ -259,8 +286,8 @@ static int y_rows(long ncolblk, long ny, int most) {
 template <typename S, int FD>
 static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, double dx,
                             GridView<S> in, GridView<S> out, const GhostFill& gf, double dt_val,
-                            const RunCtl* ctl, uint64_t* cour, const SweepTune& tune, bool st1,
-                            hipStream_t st) {
+                            const RunCtl* ctl, RunCtl* nxt, uint64_t* cour,
+                            const SweepTune& tune, bool st1, hipStream_t st) {
   const bool c = cour != nullptr;
 #define DISPATCH(F)                         \
   do {                                      \
@@ -279,7 +306,7 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     const dim3 grid(cdiv(pieces, xiter)), blk(64 * W);
 #define HXB(A, B, WW) \
   hipLaunchKernelGGL((k_sweep_xb<S, A, B, WW, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, \
-                     in, out, gf, cour, nseg, xiter)
+                     nxt, in, out, gf, cour, nseg, xiter)
 #define HXW(A, B) do { if (W == 2) HXB(A, B, 2); else HXB(A, B, 4); } while (0)
     DISPATCH(HXW);
 #undef HXW
@@ -293,8 +320,8 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
     while (xiter > 1 && cdiv(waves, (long) xw * xiter) < 1024) xiter >>= 1;
     const dim3 grid(cdiv(waves, (long) xw * xiter)), blk(64 * xw);
 #define HX(A, B) \
-  hipLaunchKernelGGL((k_sweep_x<S, A, B, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, in, \
-                     out, gf, cour, nseg, xiter)
+  hipLaunchKernelGGL((k_sweep_x<S, A, B, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, nxt, \
+                     in, out, gf, cour, nseg, xiter)
     DISPATCH(HX);
 #undef HX
   } else {
@@ -329,8 +356,8 @@ static GhostFill ghost_fill(int idim, const PhysArgs& pa, int fill) {
 #ifndef HYDRO_FAST_UNIT
 template <typename S>
 void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> in,
-                  GridView<S> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                  const SweepTune& tune, int fill, hipStream_t st) {
+                  GridView<S> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                  uint64_t* cour, const SweepTune& tune, int fill, hipStream_t st) {
   const GhostFill gf = ghost_fill(idim, pa, fill);
   const Phys<S> ph = make_phys<S>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type, pa.niter,
                                   pa.iorder, pa.scheme);
@@ -346,24 +373,24 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
                     (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny
                                : (long) cdiv(g.nx, 64) * cdiv(g.ny, 16)) >= kFastDivWaves;
     if (fd)
-      launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
-                                 st);
+      launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, nxt, cour, tune,
+                                 st1, st);
     else
-      launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
-                                 st);
+      launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, nxt, cour, tune,
+                                 st1, st);
   } else {
-    launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, cour, tune, st1,
-                                 st);
+    launch_sweep_fd<S, kIeee>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, nxt, cour, tune,
+                                 st1, st);
   }
 }
 #else
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,
-                       GridView<double> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                       const SweepTune& tune, int fill, hipStream_t st) {
+                       GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                       uint64_t* cour, const SweepTune& tune, int fill, hipStream_t st) {
   const Phys<double> ph = make_phys<double>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type,
                                             pa.niter, pa.iorder, pa.scheme);
   launch_sweep_fd<double, kFast>(idim, g, ph, pa.dx, in, out, ghost_fill(idim, pa, fill), dt_val,
-                                 ctl, cour, tune, pa.slope_type == 1.0, st);
+                                 ctl, nxt, cour, tune, pa.slope_type == 1.0, st);
 }
 #endif
 
@@ -390,8 +417,8 @@ void launch_ctl_begin(RunCtl* ctl, uint64_t* cour, double cf, double dx, double 
   hipLaunchKernelGGL(k_ctl_begin, dim3(1), dim3(64), 0, st, ctl, cour, cf, dx, smallc);
 }
 
-void launch_ctl_end(RunCtl* ctl, hipStream_t st) {
-  hipLaunchKernelGGL(k_ctl_end, dim3(1), dim3(64), 0, st, ctl);
+void launch_ctl_end(RunCtl* ctl, bool odd, hipStream_t st) {
+  hipLaunchKernelGGL(k_ctl_end, dim3(1), dim3(64), 0, st, ctl, (int) odd);
 }
 
 void launch_clear_slots(uint64_t* cour, hipStream_t st) {
@@ -416,13 +443,13 @@ template void launch_boundary<double>(int, const GridGeom&, const PhysArgs&, Gri
 template void launch_boundary<float>(int, const GridGeom&, const PhysArgs&, GridView<float>,
                                      GridView<float>, const RunCtl*, hipStream_t);
 template void launch_sweep<double>(int, const GridGeom&, const PhysArgs&, GridView<double>,
-                                   GridView<double>, double, const RunCtl*, uint64_t*,
+                                   GridView<double>, double, const RunCtl*, RunCtl*, uint64_t*,
                                    const SweepTune&, int, hipStream_t);
 template void launch_courant<double>(const GridGeom&, const PhysArgs&, GridView<double>,
                                      uint64_t*, const RunCtl*, hipStream_t);
 #elif defined(HYDRO_MIXED_UNIT)
 template void launch_sweep<float>(int, const GridGeom&, const PhysArgs&, GridView<float>,
-                                  GridView<float>, double, const RunCtl*, uint64_t*,
+                                  GridView<float>, double, const RunCtl*, RunCtl*, uint64_t*,
                                   const SweepTune&, int, hipStream_t);
 template void launch_courant<float>(const GridGeom&, const PhysArgs&, GridView<float>,
                                     uint64_t*, const RunCtl*, hipStream_t);

@@ -14,7 +14,9 @@ namespace hydro {
 
 // Device-resident time-loop state (HydroC99_2DMpi/Src/main.c:244-298 moved
 // onto the GPU so whole runs can be queued or graph-captured without host
-// round trips).
+// round trips).  A grid has two, one for its even steps and one for its odd
+// ones, so that a sweep can read the open step's while one workgroup of it
+// already writes the next step's.
 struct RunCtl {
   double t, dt, tend;
   int nstep, nstepmax;
@@ -74,7 +76,9 @@ struct SweepTune {
 // memory already, put there by launch_boundary).  It may be asked to on grids
 // of at least kGhostMin cells each way.
 // dt handling: if ctl != nullptr the kernels read dt and the active flag from
-// it; otherwise dt_val is used.  cour (2*kCourSlots uint64, zeroed) receives
+// it; otherwise dt_val is used.  nxt (x sweeps that open an even step): the
+// sweep also closes the step in *nxt, which becomes the odd step's control.
+// cour (2*kCourSlots uint64, zeroed) receives
 // the CFL maxima of the written state when non-null.
 template <typename S>
 void launch_boundary(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> src,
@@ -82,29 +86,32 @@ void launch_boundary(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S
 
 template <typename S>
 void launch_sweep(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> in,
-                  GridView<S> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                  const SweepTune& tune, int fill_ghosts, hipStream_t st);
+                  GridView<S> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                  uint64_t* cour, const SweepTune& tune, int fill_ghosts, hipStream_t st);
 
 // The FP64 fast form's sweeps (hydro_kernels.hip, fast unit): as
 // launch_sweep, with the kFast arithmetic.
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView<double> in,
-                       GridView<double> out, double dt_val, const RunCtl* ctl, uint64_t* cour,
-                       const SweepTune& tune, int fill_ghosts, hipStream_t st);
+                       GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                       uint64_t* cour, const SweepTune& tune, int fill_ghosts, hipStream_t st);
 
 template <typename S>
 void launch_courant(const GridGeom& g, const PhysArgs& ph, GridView<S> in, uint64_t* cour,
                     const RunCtl* ctl, hipStream_t st);
 
 // dt_finalize reduces the CFL slots (clearing them) into
-// dt = cfl*dx / max(cx, cy, smallc) at *dt_out.  ctl_begin opens a step of the
-// device time loop: active = (t < tend && nstep < nstepmax); on even steps dt
-// comes from the slots (halved at step 0).  ctl_end logs dt and advances
-// nstep and t.
+// dt = cfl*dx / max(cx, cy, smallc) at *dt_out.  The device time loop's
+// control, ctl[0] for even steps and ctl[1] for odd ones: ctl_begin closes the
+// odd step before (if one is open) and opens an even step, active = (t < tend
+// && nstep < nstepmax), dt from the slots (halved at step 0); the even step's
+// x sweep closes it and opens the odd one (launch_sweep's nxt); ctl_end closes
+// the last step of a run and leaves the outcome in ctl[0].  Closing a step
+// logs dt and advances nstep and t.
 void launch_dt_finalize(uint64_t* cour, double cf, double dx, double smallc, double* dt_out,
                         hipStream_t st);
 void launch_ctl_begin(RunCtl* ctl, uint64_t* cour, double cf, double dx, double smallc,
                       hipStream_t st);
-void launch_ctl_end(RunCtl* ctl, hipStream_t st);
+void launch_ctl_end(RunCtl* ctl, bool odd, hipStream_t st);
 void launch_clear_slots(uint64_t* cour, hipStream_t st);
 
 // Initial state (hydro_funcs.c:79-146): interior rho=1, u=v=0, E=1e-5, ghosts
