@@ -116,6 +116,7 @@ extern "C" void hydro_amd_batch_destroy(hydro_amd_batch* b) {
   if (b->hctl) (void) hipHostFree(b->hctl);
   if (b->hidev) (void) hipHostFree(b->hidev);
   if (b->st) (void) hipStreamDestroy(b->st);
+  stage_handles(-1);
   delete b;
 }
 
@@ -126,6 +127,7 @@ extern "C" hydro_amd_batch* hydro_amd_batch_create(int precision, long long budg
     return nullptr;
   }
   hydro_amd_batch* b = new hydro_amd_batch();
+  stage_handles(+1);
   b->prec = precision;
   b->esz = dbl(b) ? 8 : 4;
   // defaults (the serving loop runs with them): FP64 (2, 8, 32), what the
@@ -382,21 +384,10 @@ extern "C" int hydro_amd_batch_upload(hydro_amd_batch* b, int id, const double* 
   Inst* in = live(b, id);
   if (!in || !u) return in ? hydro_amd_set_error("null argument") : -1;
   const long nxt = in->p.nx + 4, rows = 4L * (in->p.ny + 4);
-  std::vector<float> tmp;
-  const void* srcp = u;
-  size_t w = 8;
-  if (!dbl(b)) {
-    tmp.resize((size_t) nxt * rows);
-    for (size_t k = 0; k < tmp.size(); k++) tmp[k] = (float) u[k];
-    srcp = tmp.data();
-    w = 4;
-  }
-  for (int k = 0; k < 2; k++) {
-    void* dst = (char*) in->mem[k] + kOrigin * b->esz;
-    BCHK(hipMemcpy2DAsync(dst, in->g.pitch * w, srcp, nxt * w, nxt * w, rows,
-                          hipMemcpyHostToDevice, b->st));
-  }
-  BCHK(hipStreamSynchronize(b->st));
+  void* dst = (char*) in->mem[0] + kOrigin * b->esz;
+  if (stage_h2d(dst, (int) b->esz, in->g.pitch, u, 8, nxt, rows, b->st)) return -1;
+  BCHK(hipMemcpyAsync(in->mem[1], in->mem[0], (size_t) in->bytes / 2, hipMemcpyDeviceToDevice,
+                      b->st));
   launch_zero_u64(b->cour + (size_t) id * 2 * kInstSlots, 2 * kInstSlots, b->st);
   launch_batch_set_ctl(b->ctl + id, 0.0, 0.0, in->p.tend, 0, in->p.nstepmax, 0, b->st);
   in->need_cour = true;

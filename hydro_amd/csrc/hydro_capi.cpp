@@ -218,6 +218,7 @@ extern "C" void hydro_amd_grid_destroy(hydro_amd_grid* g) {
   if (g->dlog) (void) hipFree(g->dlog);
   if (g->hctl) (void) hipHostFree(g->hctl);
   if (g->st) (void) hipStreamDestroy(g->st);
+  stage_handles(-1);
   delete g;
 }
 
@@ -252,9 +253,10 @@ static int validate(const hydro_amd_params* p) {
   return 0;
 }
 
-// The mirror's run control to the device, no step open.
-static int write_ctl(hydro_amd_grid* g) {
-  HIPCHK(hipStreamSynchronize(g->st));  // the pinned copy may still feed a queued copy
+// The mirror's run control to the device, no step open.  fresh: the pinned
+// copy was never used.
+static int write_ctl(hydro_amd_grid* g, bool fresh = false) {
+  if (!fresh) HIPCHK(hipStreamSynchronize(g->st));  // it may still feed a queued copy
   RunCtl c{};
   c.t = g->t;
   c.dt = g->dt;
@@ -271,6 +273,7 @@ static int write_ctl(hydro_amd_grid* g) {
 extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   if (validate(p)) return nullptr;
   hydro_amd_grid* g = new hydro_amd_grid();
+  stage_handles(+1);
   g->p = *p;
   g->prec = p->precision;
   g->esz = dbl(g) ? sizeof(double) : sizeof(float);
@@ -296,7 +299,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
     return nullptr;
   }
   launch_clear_slots(g->cour, g->st);
-  if (write_ctl(g)) {
+  if (write_ctl(g, true)) {
     fail("grid setup failed");
     hydro_amd_grid_destroy(g);
     return nullptr;
@@ -349,21 +352,11 @@ extern "C" int hydro_amd_grid_upload(hydro_amd_grid* g, const double* u) {
   if (!g || !u) return fail("null argument");
   const long nxt = g->p.nx + 4, rows = 4L * (g->p.ny + 4);
   void* dst = (char*) g->mem[0] + kOrigin * g->esz;
-  if (dbl(g)) {
-    HIPCHK(hipMemcpy2DAsync(dst, g->geom.pitch * 8, u, nxt * 8, nxt * 8, rows,
-                            hipMemcpyHostToDevice, g->st));
-  } else {
-    std::vector<float> tmp((size_t) nxt * rows);
-    for (size_t k = 0; k < tmp.size(); k++) tmp[k] = (float) u[k];
-    HIPCHK(hipMemcpy2DAsync(dst, g->geom.pitch * 4, tmp.data(), nxt * 4, nxt * 4, rows,
-                            hipMemcpyHostToDevice, g->st));
-    HIPCHK(hipStreamSynchronize(g->st));
-  }
+  if (stage_h2d(dst, (int) g->esz, g->geom.pitch, u, 8, nxt, rows, g->st)) return -1;
   // the second buffer carries the same ghosts (they are refreshed into both)
   const long total = 4 * g->plane + kOrigin + 64;
   HIPCHK(hipMemcpyAsync(g->mem[1], g->mem[0], (size_t) total * g->esz,
                         hipMemcpyDeviceToDevice, g->st));
-  HIPCHK(hipStreamSynchronize(g->st));
   bump(g);
   return 0;
 }

@@ -139,5 +139,13 @@ void launch_image(const GridGeom& g, const S* rho, int shrink, int w, int h,
 // (hydro_stage.cpp); dst_esz == src_esz, or 8 with src_esz == 4 (widening).
 int stage_d2h(void* dst, int dst_esz, const void* src, int src_esz, long src_pitch, long width,
               long rows, hipStream_t st);
+// Contiguous host rows -> pitched device rows; dst_esz == src_esz, or 4 with
+// src_esz == 8 (rounding).
+int stage_h2d(void* dst, int dst_esz, long dst_pitch, const void* src, int src_esz, long width,
+              long rows, hipStream_t st);
+// Host memory to host memory, converting (4 <-> 8 bytes an element).
+void host_copy(void* dst, int dst_esz, const void* src, int src_esz, size_t n);
+// Live grids and batches, +1 / -1: staging memory is held for them.
+void stage_handles(int d);
 
 }  // namespace hydro

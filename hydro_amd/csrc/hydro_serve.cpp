@@ -31,6 +31,9 @@
 #include <vector>
 
 #include "../../include/hydro_amd.h"
+#include "hydro_kernels.hpp"
+
+using namespace hydro;
 
 extern "C" int hydro_amd_set_error(const char* fmt, ...);  // hydro_capi.cpp
 int hydro_amd_batch_download_raw(hydro_amd_batch* b, int id, void* dst, int* elem_size,
@@ -479,14 +482,7 @@ extern "C" int hydro_amd_server_result(hydro_amd_server* s, int rid, double* uol
   Request& r = s->req[rid];
   const unsigned char* src = r.data(s->arena);
   if (r.state != DONE || !src) return hydro_amd_set_error("no result for %d", rid);
-  const size_t n = r.result_bytes / r.esz;
-  if (r.esz == 8) {
-    const double* d = (const double*) src;
-    for (size_t k = 0; k < n; k++) uold[k] = d[k];
-  } else {
-    const float* f = (const float*) src;
-    for (size_t k = 0; k < n; k++) uold[k] = f[k];
-  }
+  host_copy(uold, 8, src, r.esz, r.result_bytes / r.esz);
   return 0;
 }
 

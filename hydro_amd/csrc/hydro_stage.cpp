@@ -1,14 +1,25 @@
-// Device -> host copies of pitched state through pinned staging buffers.
+// Copies of pitched state between host and device through pinned staging
+// buffers.
 //
-// A hipMemcpy2D into pageable host memory runs at a few GB/s; into pinned
-// memory it runs at the link's rate.  Results are copied here in slabs of rows
-// into two process-wide pinned buffers, alternating, so the DMA of one slab
-// overlaps the host copy (and FP32 -> FP64 widening) of the previous one.
+// A hipMemcpy2D to or from pageable host memory goes row by row (a 1021x767
+// upload ran at 0.9 GB/s); between pinned memory and the device it runs at the
+// link's rate (55-57 GB/s at every row length from 2 to 64 KB).  What is left
+// is the host's own copy between the pinned buffers and the caller's array,
+// with the FP32 <-> FP64 conversion on the way: one thread does 14 GB/s into
+// fresh pages (5 GB/s where they are 4 KB ones), eight 30, so a large state is
+// cut into slabs of rows that up to kLanes threads carry, each through two
+// buffers of its own, the DMA of one beside the host copy of the other.
+// 8192x8192 FP64 download: 153 ms with one thread, 46 with eight; 1021x767
+// upload 28.4 ms through hipMemcpy2D, 0.8 so.
 #include <hip/hip_runtime.h>
 
 #include <string.h>
 
+#include <algorithm>
+#include <atomic>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 #include "hydro_kernels.hpp"
 
@@ -16,36 +27,176 @@ extern "C" int hydro_amd_set_error(const char* fmt, ...);  // hydro_capi.cpp
 
 namespace hydro {
 namespace {
-constexpr size_t kStageBytes = 16u << 20;  // per buffer
+// Per buffer.  The link idles about 10 us between two DMA calls: 8192x8192
+// FP64 in 72 ms with slabs of 1 MB, 54 with 2, 46 with 4 (twelve threads).
+constexpr size_t kSlabBytes = 4u << 20;
+constexpr int kLanes = 8;      // threads, two buffers each
+constexpr int kLanesKept = 4;  // whose buffers stay when no grid or batch is left
+// Host bytes that are worth a thread (starting one takes about 17 us; 0.4 to
+// 1.5 MB measured alike from 700x500 up).
+constexpr size_t kThreadBytes = 3u << 19;
 
-struct Stage {
-  std::mutex mu;  // one staged copy at a time per process
+struct Lane {
   void* buf[2] = {nullptr, nullptr};
   hipEvent_t ev[2] = {nullptr, nullptr};
-  bool ready = false;
+};
+struct Stage {
+  std::mutex mu;  // one staged copy at a time per process
+  Lane lane[kLanes];
+  int ready = 0;    // lanes that have their buffers
+  int handles = 0;  // live grids and batches
 };
 Stage g_stage;
 
-int stage_init() {
-  if (g_stage.ready) return 0;
-  for (int k = 0; k < 2; k++) {
-    if (hipHostMalloc(&g_stage.buf[k], kStageBytes, hipHostMallocDefault) != hipSuccess)
-      return hydro_amd_set_error("pinned staging allocation failed");
-    if (hipEventCreateWithFlags(&g_stage.ev[k], hipEventDisableTiming) != hipSuccess)
-      return hydro_amd_set_error("staging event creation failed");
-  }
-  g_stage.ready = true;
-  return 0;
+void lane_free(Lane& l) {
+  if (l.buf[0]) (void) hipHostFree(l.buf[0]);  // one allocation
+  for (hipEvent_t e : l.ev)
+    if (e) (void) hipEventDestroy(e);
+  l = Lane();
 }
 
-void widen_rows(void* dst, int dst_esz, const void* src, int src_esz, size_t n) {
-  if (dst_esz == src_esz) {
-    memcpy(dst, src, n * (size_t) src_esz);
-  } else {  // float -> double
+// At least one lane, up to n; how many there are.
+int lanes_for(int n) {
+  for (; g_stage.ready < n; g_stage.ready++) {
+    Lane& l = g_stage.lane[g_stage.ready];
+    if (hipHostMalloc(&l.buf[0], 2 * kSlabBytes, hipHostMallocDefault) != hipSuccess ||
+        hipEventCreateWithFlags(&l.ev[0], hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&l.ev[1], hipEventDisableTiming) != hipSuccess) {
+      (void) hipGetLastError();
+      lane_free(l);
+      break;
+    }
+    l.buf[1] = (char*) l.buf[0] + kSlabBytes;
+  }
+  return std::min(n, g_stage.ready);
+}
+
+// n elements of sesz bytes to desz bytes (4 or 8 each).
+void convert(void* dst, int desz, const void* src, int sesz, size_t n) {
+  if (desz == sesz) {
+    memcpy(dst, src, n * (size_t) sesz);
+  } else if (desz == 8) {
     const float* s = (const float*) src;
     double* d = (double*) dst;
     for (size_t k = 0; k < n; k++) d[k] = s[k];
+  } else {
+    const double* s = (const double*) src;
+    float* d = (float*) dst;
+    for (size_t k = 0; k < n; k++) d[k] = (float) s[k];
   }
+}
+
+// Runs work(k) for k = 0..n-1, k = 0 on the calling thread and the others on
+// threads of their own, where they can be had.
+template <typename F>
+void on_threads(int n, const F& work) {
+  std::thread th[kLanes];
+  int started = 0;
+  for (int k = 1; k < n; k++) {
+    try {
+      th[k] = std::thread([&work, k] { work(k); });
+      started = k;
+    } catch (const std::system_error&) {
+      break;
+    }
+  }
+  work(0);
+  for (int k = started + 1; k < n; k++) work(k);
+  for (int k = 1; k <= started; k++) th[k].join();
+}
+
+int thread_count(size_t bytes) {
+  static const int cpus = std::max(1, (int) std::thread::hardware_concurrency());
+  const size_t want = std::max<size_t>(1, bytes / kThreadBytes);
+  return (int) std::min<size_t>(want, (size_t) std::min(cpus, kLanes));
+}
+
+// One block of columns, at most a slab wide: `rows` rows of `width` elements;
+// host rows hpitch elements apart, device rows dpitch.
+struct Block {
+  char* host;
+  int hesz;
+  long hpitch;
+  char* dev;
+  int desz;
+  long dpitch, width, rows;
+  hipStream_t st;
+};
+
+int copy_block(const Block& b, bool up) {
+  const size_t row_bytes = (size_t) b.width * b.desz;
+  int n = lanes_for(thread_count((size_t) b.width * b.rows * b.hesz));
+  if (n < 1) return hydro_amd_set_error("pinned staging allocation failed");
+  // slabs small enough that every thread has two or more
+  const long per = std::max(1L, std::min((long) (kSlabBytes / row_bytes),
+                                         (b.rows + 2L * n - 1) / (2L * n)));
+  const long nslab = (b.rows + per - 1) / per;
+  n = (int) std::min<long>(n, nslab);
+  int dev = 0;
+  (void) hipGetDevice(&dev);
+  std::atomic<int> bad{0};
+  auto host_copy = [&](void* buf, long r0, long nr) {
+    char* h = b.host + (size_t) r0 * b.hpitch * b.hesz;
+    if (b.hpitch == b.width) {
+      const size_t m = (size_t) nr * b.width;
+      if (up) convert(buf, b.desz, h, b.hesz, m);
+      else convert(h, b.hesz, buf, b.desz, m);
+      return;
+    }
+    for (long r = 0; r < nr; r++) {
+      char* hr = h + (size_t) r * b.hpitch * b.hesz;
+      char* br = (char*) buf + (size_t) r * row_bytes;
+      if (up) convert(br, b.desz, hr, b.hesz, b.width);
+      else convert(hr, b.hesz, br, b.desz, b.width);
+    }
+  };
+  auto work = [&](int k) {
+    Lane& l = g_stage.lane[k];
+    if (hipSetDevice(dev) != hipSuccess) {
+      bad = 1;
+      return;
+    }
+    auto dma = [&](int q, long c) {
+      const long r0 = c * per, nr = std::min(per, b.rows - r0);
+      char* d = b.dev + (size_t) r0 * b.dpitch * b.desz;
+      const hipError_t e =
+          up ? hipMemcpy2DAsync(d, (size_t) b.dpitch * b.desz, l.buf[q], row_bytes, row_bytes, nr,
+                                hipMemcpyHostToDevice, b.st)
+             : hipMemcpy2DAsync(l.buf[q], row_bytes, d, (size_t) b.dpitch * b.desz, row_bytes, nr,
+                                hipMemcpyDeviceToHost, b.st);
+      if (e != hipSuccess || hipEventRecord(l.ev[q], b.st) != hipSuccess) bad = 1;
+    };
+    int q = 0;
+    if (!up && k < nslab) dma(0, k);
+    for (long c = k; c < nslab && !bad; c += n, q ^= 1) {
+      const long r0 = c * per, nr = std::min(per, b.rows - r0);
+      if (up) {
+        if (c >= k + 2L * n && hipEventSynchronize(l.ev[q]) != hipSuccess) bad = 1;
+        host_copy(l.buf[q], r0, nr);
+        if (!bad) dma(q, c);
+      } else {
+        if (c + n < nslab) dma(q ^ 1, c + n);  // its buffer was emptied a slab ago
+        if (hipEventSynchronize(l.ev[q]) != hipSuccess) bad = 1;
+        if (!bad) host_copy(l.buf[q], r0, nr);
+      }
+    }
+  };
+  on_threads(n, work);
+  // (the buffers are free again once the stream is past the copies)
+  if ((up || bad) && hipStreamSynchronize(b.st) != hipSuccess) bad = 1;
+  return bad ? hydro_amd_set_error("%s copy failed", up ? "host-to-device" : "device-to-host") : 0;
+}
+
+int staged(char* host, int hesz, char* dev, int desz, long pitch, long width, long rows,
+           hipStream_t st, bool up) {
+  std::lock_guard<std::mutex> lk(g_stage.mu);
+  const long most = (long) (kSlabBytes / desz);  // columns at a time
+  for (long c = 0; c < width; c += most) {
+    const Block b{host + (size_t) c * hesz, hesz, width, dev + (size_t) c * desz, desz, pitch,
+                  std::min(most, width - c), rows, st};
+    if (copy_block(b, up)) return -1;
+  }
+  return 0;
 }
 }  // namespace
 
@@ -55,37 +206,34 @@ void widen_rows(void* dst, int dst_esz, const void* src, int src_esz, size_t n) 
 // Ordered after earlier work on `st`; returns when the data is in dst.
 int stage_d2h(void* dst, int dst_esz, const void* src, int src_esz, long src_pitch, long width,
               long rows, hipStream_t st) {
+  return staged((char*) dst, dst_esz, (char*) src, src_esz, src_pitch, width, rows, st, false);
+}
+
+// The way back: contiguous host rows of src_esz-byte elements to pitched rows
+// on the device (dst_esz == src_esz, or 4 with src_esz == 8, rounded).
+// Ordered after earlier work on `st`; returns when the data is on the device.
+int stage_h2d(void* dst, int dst_esz, long dst_pitch, const void* src, int src_esz, long width,
+              long rows, hipStream_t st) {
+  return staged((char*) src, src_esz, (char*) dst, dst_esz, dst_pitch, width, rows, st, true);
+}
+
+// dst = src, n elements, on as many threads as that is worth (both in host memory).
+void host_copy(void* dst, int dst_esz, const void* src, int src_esz, size_t n) {
+  const int t = thread_count(n * (size_t) std::max(dst_esz, src_esz));
+  const size_t per = (n + t - 1) / t;
+  on_threads(t, [&](int k) {
+    const size_t a = std::min(n, per * k), m = std::min(n, a + per) - a;
+    convert((char*) dst + a * dst_esz, dst_esz, (const char*) src + a * src_esz, src_esz, m);
+  });
+}
+
+// A grid or batch is made (+1) or destroyed (-1): with the last one most of the
+// staging memory goes back.
+void stage_handles(int d) {
   std::lock_guard<std::mutex> lk(g_stage.mu);
-  const size_t row_bytes = (size_t) width * src_esz;
-  if (stage_init() != 0 || row_bytes > kStageBytes) {  // direct (pageable) copy
-    if (dst_esz != src_esz) return hydro_amd_set_error("row too wide for staged widening");
-    if (hipMemcpy2DAsync(dst, row_bytes, src, (size_t) src_pitch * src_esz, row_bytes, rows,
-                         hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipStreamSynchronize(st) != hipSuccess)
-      return hydro_amd_set_error("device-to-host copy failed");
-    return 0;
-  }
-  const long per = (long) (kStageBytes / row_bytes);
-  const long nchunk = (rows + per - 1) / per;
-  auto issue = [&](long c) -> int {
-    const long r0 = c * per, nr = rows - r0 < per ? rows - r0 : per;
-    const char* s = (const char*) src + (size_t) r0 * src_pitch * src_esz;
-    if (hipMemcpy2DAsync(g_stage.buf[c & 1], row_bytes, s, (size_t) src_pitch * src_esz,
-                         row_bytes, nr, hipMemcpyDeviceToHost, st) != hipSuccess ||
-        hipEventRecord(g_stage.ev[c & 1], st) != hipSuccess)
-      return hydro_amd_set_error("device-to-host copy failed");
-    return 0;
-  };
-  if (nchunk > 0 && issue(0)) return -1;
-  for (long c = 0; c < nchunk; c++) {
-    if (c + 1 < nchunk && issue(c + 1)) return -1;  // its buffer was drained at c-1
-    if (hipEventSynchronize(g_stage.ev[c & 1]) != hipSuccess)
-      return hydro_amd_set_error("device-to-host copy failed");
-    const long r0 = c * per, nr = rows - r0 < per ? rows - r0 : per;
-    widen_rows((char*) dst + (size_t) r0 * width * dst_esz, dst_esz, g_stage.buf[c & 1],
-               src_esz, (size_t) nr * width);
-  }
-  return 0;
+  g_stage.handles += d;
+  if (g_stage.handles > 0) return;
+  while (g_stage.ready > kLanesKept) lane_free(g_stage.lane[--g_stage.ready]);
 }
 
 }  // namespace hydro
