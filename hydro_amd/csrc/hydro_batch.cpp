@@ -65,14 +65,14 @@ struct hydro_amd_batch {
   int n[6] = {0, 0, 0, 0, 0, 0}; // Px Py Qx Qy PB QB
   int off[6] = {0, 0, 0, 0, 0, 0};
   int n1[6] = {0, 0, 0, 0, 0, 0};  // leading tasks of slope_type == 1 instances
-  uint64_t* qctr = nullptr;        // kQueues task-queue counters (device)
+  BList* lists = nullptr;          // what the task tables are written from (device)
   int nids = 0;
   int maxid = -1;                // highest live id
   bool dirty = true;
   bool flip = false;             // next step runs Q before P
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
-  BatchTune tune = {2, 8, 32};  // set by precision at creation
-  int nblk_x = 1024, nblk_y = 1024, cus = 256;
+  BatchTune tune = {1, 0, 0};
+  int xiter = 1, yseg = 1;       // the shape in use (rebuild)
   std::vector<int> live_ids;
   RunCtl* hctl = nullptr;        // pinned host copy of the run controls
   void* hidev = nullptr;         // pinned host copy of the instance array
@@ -80,20 +80,6 @@ struct hydro_amd_batch {
 
 // FP64 storage (the FP64 and FP64 fast forms) rather than FP32.
 static bool dbl(const hydro_amd_batch* b) { return b->prec != HYDRO_AMD_MIXED; }
-
-static void size_grids(hydro_amd_batch* b) {
-  const int w = b->tune.waves;
-  if (b->prec == HYDRO_AMD_FP64_FAST) {
-    b->nblk_x = b->cus * batch_sweep_occupancy_fast(1, w);
-    b->nblk_y = b->cus * batch_sweep_occupancy_fast(2, w);
-  } else if (b->prec == HYDRO_AMD_FP64) {
-    b->nblk_x = b->cus * batch_sweep_occupancy<double>(1, w);
-    b->nblk_y = b->cus * batch_sweep_occupancy<double>(2, w);
-  } else {
-    b->nblk_x = b->cus * batch_sweep_occupancy<float>(1, w);
-    b->nblk_y = b->cus * batch_sweep_occupancy<float>(2, w);
-  }
-}
 
 static void drop_graphs(hydro_amd_batch* b) {
   for (auto& g : b->gexec)
@@ -111,7 +97,7 @@ extern "C" void hydro_amd_batch_destroy(hydro_amd_batch* b) {
     for (auto& m : in.mem)
       if (m) (void) hipFree(m);
   for (void* p : {(void*) b->ctl, (void*) b->cour, b->idev, (void*) b->tasks, (void*) b->ids,
-                  (void*) b->cids, (void*) b->qctr})
+                  (void*) b->cids, (void*) b->lists})
     if (p) (void) hipFree(p);
   if (b->hctl) (void) hipHostFree(b->hctl);
   if (b->hidev) (void) hipHostFree(b->hidev);
@@ -130,11 +116,6 @@ extern "C" hydro_amd_batch* hydro_amd_batch_create(int precision, long long budg
   stage_handles(+1);
   b->prec = precision;
   b->esz = dbl(b) ? 8 : 4;
-  // defaults (the serving loop runs with them): FP64 (2, 8, 32), what the
-  // autotuner picks for the 512-instance mix; mixed (4, 32, 64), the fastest
-  // measured on the serving mix (sides 128-4096: 48.4 solves/s against 45.0
-  // for (4, 8, 16) at 1000 arrivals/s)
-  b->tune = precision == HYDRO_AMD_MIXED ? BatchTune{4, 32, 64} : BatchTune{2, 8, 32};
   b->budget = budget_bytes > 0 ? budget_bytes : (1LL << 62);
   b->inst.resize(kMaxInst);
   const size_t isz = dbl(b) ? sizeof(InstDev<double>) : sizeof(InstDev<float>);
@@ -144,7 +125,7 @@ extern "C" hydro_amd_batch* hydro_amd_batch_create(int precision, long long budg
             hipMalloc(&b->idev, isz * kMaxInst) == hipSuccess &&
             hipMalloc(&b->ids, sizeof(int) * kMaxInst) == hipSuccess &&
             hipMalloc(&b->cids, sizeof(int) * kMaxInst) == hipSuccess &&
-            hipMalloc(&b->qctr, sizeof(uint64_t) * kQueues) == hipSuccess &&
+            hipMalloc(&b->lists, sizeof(BList) * 4 * kMaxInst) == hipSuccess &&
             hipHostMalloc((void**) &b->hctl, sizeof(RunCtl) * kMaxInst) == hipSuccess &&
             hipHostMalloc(&b->hidev, isz * kMaxInst) == hipSuccess;
   if (!ok) {
@@ -160,9 +141,6 @@ extern "C" hydro_amd_batch* hydro_amd_batch_create(int precision, long long budg
     uint64_t thr = ~0ULL;
     (void) hipMemPoolSetAttribute(pool, hipMemPoolAttrReleaseThreshold, &thr);
   }
-  hipDeviceProp_t prop;
-  if (hipGetDeviceProperties(&prop, dev) == hipSuccess) b->cus = prop.multiProcessorCount;
-  size_grids(b);
   if (hipStreamSynchronize(b->st) != hipSuccess) {
     hydro_amd_set_error("batch setup failed");
     hydro_amd_batch_destroy(b);
@@ -397,11 +375,35 @@ extern "C" int hydro_amd_batch_upload(hydro_amd_batch* b, int id, const double* 
 
 // ---- task tables -------------------------------------------------------------------
 
+// Task shape by the load.  As in a single grid's y sweep (y_rows,
+// hydro_kernels.hip), a task's fixed cost and the unevenness that long tasks
+// leave at a launch's end balance at a length proportional to the square root
+// of the work: sqrt(wave rows) / 32 rows, sqrt(segments) / 100 segments.  The
+// best of all shapes tried, x segments / y rows: 12 grids of 64-256 a side
+// 2 / 2; 30 of 150-500 2-4 / 8; 60 of 64-1024 4-8 / 12; 300 of 64-1024 8 / 32;
+// 24 of 128-4096 8-16 / 24-32.  A step took with the fixed shapes before (2
+// or 4 waves of 8 or 32 segments, 32 or 64 rows) and takes with these: 12 small
+// grids, mixed, 138 and 28 us; 30, fast, 156 and 113; 60, FP64, 701 and 650;
+// 24 of up to 4096, mixed, 1.21 and 1.16 ms.
+static void shape_by_load(hydro_amd_batch* b) {
+  long segs = 0, wrows = 0;
+  for (int id : b->live_ids) {
+    const hydro_amd_params& p = b->inst[id].p;
+    segs += (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+    wrows += (long) ((p.nx + 63) / 64) * p.ny;
+  }
+  auto root = [](long n, double by, int most) {
+    return std::max(1, std::min(most, (int) (std::sqrt((double) n) / by + 0.5)));
+  };
+  b->xiter = b->tune.xiter > 0 ? b->tune.xiter : root(segs, 100, 32);
+  b->yseg = b->tune.yseg > 0 ? b->tune.yseg : root(wrows, 32, 32);
+}
+
 // Rows per wave in an instance's y tasks: the instance's rows split evenly
-// over as few row groups (of waves x tune.yseg rows) as cover them, so no
+// over as few row groups (of waves x b->yseg rows) as cover them, so no
 // group ends with a short segment that pays the full halo.
 static int inst_yseg(const hydro_amd_batch* b, int ny) {
-  const long W = b->tune.waves, per = W * b->tune.yseg;
+  const long W = b->tune.waves, per = W * b->yseg;
   const long nrg = (ny + per - 1) / per;
   return (int) ((ny + W * nrg - 1) / (W * nrg));
 }
@@ -435,30 +437,29 @@ static InstDev<S> inst_dev(hydro_amd_batch* b, int id) {
   return d;
 }
 
-static void tasks_of(const hydro_amd_batch* b, int id, int kind, std::vector<BTask>& out) {
-  const Inst& in = b->inst[id];
-  const int W = b->tune.waves;
+// An instance's x (kind 1) or y (kind 2) tasks.
+static BList sweep_tasks(const hydro_amd_batch* b, int id, int kind) {
+  const hydro_amd_params& p = b->inst[id].p;
+  const long W = b->tune.waves;
+  BList l{id, kind, 0, 0, 0, 0};
   if (kind == 1) {
-    const long nseg = (in.p.nx + kXSeg - 1) / kXSeg;
-    const long tot = nseg * in.p.ny, per = (long) W * b->tune.xiter;
-    for (long a = 0; a < tot; a += per) out.push_back(BTask{id, 1, (int) a, 0});
+    const long per = W * b->xiter, tot = (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+    l.per = (int) per;
+    l.count = (int) ((tot + per - 1) / per);
   } else {
-    const int ncb = (in.p.nx + 63) / 64;
-    const long rows = (long) W * inst_yseg(b, in.p.ny);
-    const int nrg = (int) ((in.p.ny + rows - 1) / rows);
-    for (int rg = 0; rg < nrg; rg++)
-      for (int cb = 0; cb < ncb; cb++) out.push_back(BTask{id, 2, cb, rg});
+    const long rows = W * inst_yseg(b, p.ny);
+    l.ncb = (p.nx + 63) / 64;
+    l.count = (int) (l.ncb * ((p.ny + rows - 1) / rows));
   }
+  return l;
 }
 
-// Ghost fills of one narrow instance in direction idim, kBoundaryChunk (line, var)
-// pairs per task so a large instance spreads over many workgroups.
-static void boundary_tasks_of(const hydro_amd_batch* b, int id, int idim,
-                              std::vector<BTask>& out) {
-  const Inst& in = b->inst[id];
-  if (folds_ghosts(in)) return;
-  const int nl = idim == 1 ? in.p.ny : in.p.nx;
-  for (int a = 0; a < 4 * nl; a += kBoundaryChunk) out.push_back(BTask{id, idim, a, 0});
+// Ghost fills of one narrow instance in direction idim, kBoundaryChunk
+// (line, var) pairs per task so a large instance spreads over many workgroups.
+static BList ghost_tasks(const hydro_amd_batch* b, int id, int idim) {
+  const hydro_amd_params& p = b->inst[id].p;
+  const long tot = 4L * (idim == 1 ? p.ny : p.nx);
+  return BList{id, idim, 0, (int) ((tot + kBoundaryChunk - 1) / kBoundaryChunk), kBoundaryChunk, 0};
 }
 
 // Reads the run controls of ids [0, maxid] into the pinned host copy.
@@ -482,39 +483,50 @@ static int rebuild(hydro_amd_batch* b) {
       b->maxid = k;
     }
   if (read_ctl(b)) return -1;
+  shape_by_load(b);
   // each sweep list: tasks of slope_type == 1 instances first (their own
   // kernel variant), then the others
-  std::vector<BTask> L[6], G[6];
+  std::vector<BList> L[6][2];
   for (int id : b->live_ids) {
     const bool even = (b->hctl[id].nstep % 2) == 0;
-    std::vector<BTask>* S = b->inst[id].p.slope_type == 1.0 ? L : G;
-    tasks_of(b, id, 1, even ? S[0] : S[2]);
-    tasks_of(b, id, 2, even ? S[3] : S[1]);
-    boundary_tasks_of(b, id, even ? 1 : 2, L[4]);
-    boundary_tasks_of(b, id, even ? 2 : 1, L[5]);
+    const int gen = b->inst[id].p.slope_type == 1.0 ? 0 : 1;
+    L[even ? 0 : 2][gen].push_back(sweep_tasks(b, id, 1));
+    L[even ? 3 : 1][gen].push_back(sweep_tasks(b, id, 2));
+    if (!folds_ghosts(b->inst[id])) {
+      L[4][0].push_back(ghost_tasks(b, id, even ? 1 : 2));
+      L[5][0].push_back(ghost_tasks(b, id, even ? 2 : 1));
+    }
   }
-  int need = 0;
+  std::vector<BList> all;
+  long need = 0;
   for (int k = 0; k < 6; k++) {
-    b->n1[k] = (int) L[k].size();
-    L[k].insert(L[k].end(), G[k].begin(), G[k].end());
-    b->off[k] = need;
-    b->n[k] = (int) L[k].size();
-    need += b->n[k];
+    b->off[k] = (int) need;
+    for (auto& part : L[k]) {
+      for (BList& l : part) {
+        l.first = (int) need;
+        need += l.count;
+        all.push_back(l);
+      }
+      if (&part == &L[k][0]) b->n1[k] = (int) (need - b->off[k]);
+    }
+    b->n[k] = (int) (need - b->off[k]);
   }
+  if (need > (1L << 30)) return hydro_amd_set_error("batch too large: %ld tasks", need);
   b->nids = (int) b->live_ids.size();
   if (need > b->task_cap) {
     if (b->tasks) BCHK(hipFree(b->tasks));
     b->tasks = nullptr;
     b->task_cap = 0;
-    const int cap = std::max(need, 1024) * 2;
+    const long cap = std::max(need + need / 2, 4096L);
     BCHK(hipMalloc(&b->tasks, sizeof(BTask) * cap));
-    b->task_cap = cap;
+    b->task_cap = (int) cap;
   }
-  std::vector<BTask> all;
-  all.reserve(need);
-  for (auto& l : L) all.insert(all.end(), l.begin(), l.end());
-  if (!all.empty())
-    BCHK(hipMemcpy(b->tasks, all.data(), sizeof(BTask) * all.size(), hipMemcpyHostToDevice));
+  // (the tables are written on the device: a large load has 1e5 tasks)
+  if (!all.empty()) {
+    BCHK(hipMemcpy(b->lists, all.data(), sizeof(BList) * all.size(), hipMemcpyHostToDevice));
+    launch_batch_tasks(b->lists, (int) all.size(), b->tasks, b->st);
+    BCHK(hipGetLastError());
+  }
   if (b->nids)
     BCHK(hipMemcpy(b->ids, b->live_ids.data(), sizeof(int) * b->nids, hipMemcpyHostToDevice));
   if (b->maxid >= 0) {
@@ -534,36 +546,36 @@ static int rebuild(hydro_amd_batch* b) {
 }
 
 // The sweeps of task list k (kind 1: x, 2: y) in the batch's arithmetic form,
-// reading buffer `phase`; q: the list's two task-queue counters.
+// reading buffer `phase`.
 template <typename S>
 static void sweep_list(hydro_amd_batch* b, int kind, const InstDev<S>* I, int k, int phase,
-                       bool ghosts, int nblk, uint64_t* q) {
+                       bool ghosts) {
   if constexpr (sizeof(S) == 8) {
     if (b->prec == HYDRO_AMD_FP64_FAST) {
       launch_batch_sweep_fast(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
-                              b->tune, nblk, q, b->st);
+                              b->tune.waves, b->xiter, b->st);
       return;
     }
   }
   launch_batch_sweep<S>(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
-                        b->tune, nblk, q, b->st);
+                        b->tune.waves, b->xiter, b->st);
 }
 
-// One phase: the ghost fills of its narrow instances, then its x tasks and its y tasks.
+// One phase: the ghost fills of its narrow instances, then its x tasks and its
+// y tasks.
 template <typename S>
 static void enq_phase(hydro_amd_batch* b, int which, int phase) {
   const InstDev<S>* I = (const InstDev<S>*) b->idev;
   const int x = which == 0 ? 0 : 2, y = x + 1, bd = which == 0 ? 4 : 5;
-  launch_batch_boundary<S>(I, b->tasks + b->off[bd], b->n[bd], phase, b->nblk_y, b->st);
-  uint64_t* q = b->qctr + 4 * phase;  // x: q[0..1], y: q[2..3]
-  sweep_list<S>(b, 1, I, x, phase, true, b->nblk_x, q);
-  sweep_list<S>(b, 2, I, y, phase, true, b->nblk_y, q + 2);
+  launch_batch_boundary<S>(I, b->tasks + b->off[bd], b->n[bd], phase, b->st);
+  sweep_list<S>(b, 1, I, x, phase, true);
+  sweep_list<S>(b, 2, I, y, phase, true);
 }
 
 template <typename S>
 static void enq_step_t(hydro_amd_batch* b, bool flip) {
   const InstDev<S>* I = (const InstDev<S>*) b->idev;
-  launch_batch_ctl<S>(I, b->ids, b->nids, true, b->qctr, b->st);
+  launch_batch_ctl<S>(I, b->ids, b->nids, true, b->st);
   enq_phase<S>(b, flip ? 1 : 0, 0);
   enq_phase<S>(b, flip ? 0 : 1, 1);
 }
@@ -571,11 +583,9 @@ static void enq_step_t(hydro_amd_batch* b, bool flip) {
 // Closes the last step of a run (each step closes the one before it).
 static void enq_close(hydro_amd_batch* b) {
   if (dbl(b))
-    launch_batch_ctl<double>((const InstDev<double>*) b->idev, b->ids, b->nids, false, b->qctr,
-                             b->st);
+    launch_batch_ctl<double>((const InstDev<double>*) b->idev, b->ids, b->nids, false, b->st);
   else
-    launch_batch_ctl<float>((const InstDev<float>*) b->idev, b->ids, b->nids, false, b->qctr,
-                            b->st);
+    launch_batch_ctl<float>((const InstDev<float>*) b->idev, b->ids, b->nids, false, b->st);
 }
 
 static void enq_step(hydro_amd_batch* b, bool flip) {
@@ -690,7 +700,6 @@ extern "C" int hydro_amd_batch_set_tune(hydro_amd_batch* b, int waves, int xiter
     return hydro_amd_set_error("tune out of range");
   BCHK(hipStreamSynchronize(b->st));
   b->tune = BatchTune{waves, xiter, yseg};
-  size_grids(b);
   b->dirty = true;
   return 0;
 }
@@ -721,23 +730,21 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
   hipEvent_t e0, e1;
   BCHK(hipEventCreate(&e0));
   BCHK(hipEventCreate(&e1));
-  for (int w : {2, 4})
-    for (int xi : {4, 8, 16, 32})
-      for (int ys : {16, 32, 64, 128}) {
+  // around the shape that goes by the load
+  b->tune = BatchTune{1, 0, 0};
+  shape_by_load(b);
+  const int rx = b->xiter, ry = b->yseg;
+  for (int w : {1, 2, 4})
+    for (int xi : {std::max(1, rx / 2), rx, 2 * rx, 4 * rx})
+      for (int ys : {std::max(1, ry / 2), ry, 2 * ry}) {
         if (hydro_amd_batch_set_tune(b, w, xi, ys) || rebuild(b)) break;
         for (int r = -1; r < reps; r++) {  // r = -1 warms up
           if (r == 0) (void) hipEventRecord(e0, b->st);
           // every x and y list at phase 0: reads buffer 0, writes buffer 1 only
-          launch_zero_u64(b->qctr, kQueues, b->st);
           for (int k = 0; k < 4; k++) {
             const int kind = (k % 2 == 0) ? 1 : 2;
-            const int nb = kind == 1 ? b->nblk_x : b->nblk_y;
-            if (dbl(b))
-              sweep_list<double>(b, kind, (const InstDev<double>*) b->idev, k, 0, false, nb,
-                                 b->qctr + 2 * k);
-            else
-              sweep_list<float>(b, kind, (const InstDev<float>*) b->idev, k, 0, false, nb,
-                                b->qctr + 2 * k);
+            if (dbl(b)) sweep_list<double>(b, kind, (const InstDev<double>*) b->idev, k, 0, false);
+            else sweep_list<float>(b, kind, (const InstDev<float>*) b->idev, k, 0, false);
           }
         }
         (void) hipEventRecord(e1, b->st);
@@ -751,11 +758,16 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
   (void) hipEventDestroy(e0);
   (void) hipEventDestroy(e1);
   BCHK(hipMemcpy(b->ctl, saved.data(), sizeof(RunCtl) * nc, hipMemcpyHostToDevice));
-  if (hydro_amd_batch_set_tune(b, bt.waves, bt.xiter, bt.yseg)) return -1;
+  if (bms == 1e30) {  // nothing could be timed
+    b->tune = keep;
+    b->dirty = true;
+  } else if (hydro_amd_batch_set_tune(b, bt.waves, bt.xiter, bt.yseg)) {
+    return -1;
+  }
   if (best) {
     best[0] = bt.waves;
-    best[1] = bt.xiter;
-    best[2] = bt.yseg;
+    best[1] = bt.xiter > 0 ? bt.xiter : rx;
+    best[2] = bt.yseg > 0 ? bt.yseg : ry;
   }
   return 0;
 }

@@ -8,8 +8,12 @@
 // HydroC99_2DMpi/Src/main.c:285-291), so a phase's task table mixes x tasks
 // of some instances with y tasks of others (the x and y tasks run as separate
 // launches, and each list as two: instances with slope_type == 1 first, in
-// the specialised variant).  Workgroups are persistent: the grid is sized to
-// the GPU, and the workgroups pull task indices from an atomic counter.  A
+// the specialised variant).  One workgroup takes one task, handed out by the
+// hardware's dispatcher: resident workgroups that drew task indices from an
+// atomic counter got at most 86 M of them a second (one address), which held
+// up every launch of small tasks (60 grids of 64-1024 a side, a step: FP64 701
+// against 788 us, fast 434 against 495, mixed 294 against 330 at the same task
+// shapes) and made tasks small enough to balance the load a loss.  A
 // task is one workgroup's worth of one instance:
 //   x task: wpb * xiter consecutive 60-cell row segments (each wave walks xiter)
 //   y task: 64 columns x (wpb * yseg) rows (each wave marches yseg rows; the
@@ -27,20 +31,6 @@
 
 namespace hydro {
 
-// The next task index of a sweep launch for the whole workgroup: persistent
-// workgroups pull tasks from one counter (zeroed before the launch), so a
-// workgroup that drew cheap tasks takes more instead of idling while others
-// finish.  Every index past the table ends the loop of the workgroup that
-// drew it, so the launch drains.
-__device__ __forceinline__ int next_task(uint64_t* qnext) {
-  __shared__ int s_next;
-  if (threadIdx.x == 0) s_next = (int) atomicAdd((unsigned long long*) qnext, 1ULL);
-  __syncthreads();
-  const int t = s_next;
-  __syncthreads();  // every thread has read s_next before it is rewritten
-  return t;
-}
-
 // The ghosts of one instance's sweep in direction idim (GhostFill).
 template <typename S>
 __device__ __forceinline__ GhostFill inst_ghosts(const InstDev<S>& d, int idim, int phase,
@@ -53,73 +43,63 @@ __device__ __forceinline__ GhostFill inst_ghosts(const InstDev<S>& d, int idim, 
 // x tasks of one phase (every task's kind is 1).  ST1: every listed
 // instance has slope_type == 1 (the host splits each phase's lists), so the
 // limiter's multiply/divide by slope_type is compiled out as in single grids.
-// FD: the arithmetic form (persistent workgroups keep the SIMDs busy, so the
-// FP64 batches take the range-gated divisions, kGated, for every instance).
+// FD: the arithmetic form (a batch keeps the SIMDs busy, so the FP64 batches
+// take the range-gated divisions, kGated, for every instance).
 // Built for 5 waves per SIMD, as the single-grid x sweep (the per-task state
 // would otherwise take it to 98 VGPRs and 4 waves; one register spills).
 template <typename S, bool ST1, int FD>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) void k_batch_sweep_x(
-    const InstDev<S>* __restrict__ inst, const BTask* __restrict__ tasks, int ntask, int phase,
-    int ghosts, int xiter, uint64_t* qnext) {
+    const InstDev<S>* __restrict__ inst, const BTask* __restrict__ tasks, int phase, int ghosts,
+    int xiter) {
   const int wpb = blockDim.x >> 6;
-  const int wave = wave_id();
-  for (;;) {
-    const int t = next_task(qnext);
-    if (t >= ntask) break;
-    const BTask tk = tasks[t];
-    const InstDev<S>& d = inst[tk.inst];
-    if (!d.ctl->active) continue;  // workgroup-uniform
-    const double dtdx = d.ctl->dt / d.dx;
-    const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
-    const GridView<S> in = d.buf[phase], out = d.buf[1 - phase];
-    const GhostFill gf = inst_ghosts(d, 1, phase, ghosts);
-    // the second sweep of an odd step is an x sweep; it produces the CFL
-    // maxima the next (even) step's dt needs
-    const bool cour = phase == 1;
-    double cx = 0.0, cy = 0.0;
-    // segments tk.a + it * wpb + wave, it = 0 .. xiter-1
-    SegWalk w(tk.a + wave, d.nseg);
-    for (int it = 0; it < xiter && w.row < d.g.ny; it++) {
-      if (cour)
-        x_segment<S, ST1, true, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
-      else
-        x_segment<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
-      w.advance(wpb, d.nseg);
-    }
-    if (cour) commit_courant(cx, cy, d.cour, kInstSlots, t % kInstSlots);
+  const BTask tk = tasks[blockIdx.x];
+  const InstDev<S>& d = inst[tk.inst];
+  if (!d.ctl->active) return;  // workgroup-uniform
+  const double dtdx = d.ctl->dt / d.dx;
+  const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
+  const GridView<S> in = d.buf[phase], out = d.buf[1 - phase];
+  const GhostFill gf = inst_ghosts(d, 1, phase, ghosts);
+  // the second sweep of an odd step is an x sweep; it produces the CFL
+  // maxima the next (even) step's dt needs
+  const bool cour = phase == 1;
+  double cx = 0.0, cy = 0.0;
+  // segments tk.a + it * wpb + wave, it = 0 .. xiter-1
+  SegWalk w(tk.a + wave_id(), d.nseg);
+  for (int it = 0; it < xiter && w.row < d.g.ny; it++) {
+    if (cour)
+      x_segment<S, ST1, true, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
+    else
+      x_segment<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, gf, w.row, w.seg, cx, cy);
+    w.advance(wpb, d.nseg);
   }
+  if (cour) commit_courant(cx, cy, d.cour, kInstSlots, blockIdx.x % kInstSlots);
 }
 
 // y tasks of one phase (every task's kind is 2); y sweeps never end a step
 // whose successor needs dt, so they fold no CFL maxima.
 template <typename S, bool ST1, int FD>
 __global__ __launch_bounds__(256) void k_batch_sweep_y(const InstDev<S>* __restrict__ inst,
-                                                       const BTask* __restrict__ tasks,
-                                                       int ntask, int phase, int ghosts,
-                                                       uint64_t* qnext) {
+                                                       const BTask* __restrict__ tasks, int phase,
+                                                       int ghosts) {
   const int wpb = blockDim.x >> 6;
   const int wave = wave_id();
-  for (;;) {
-    const int t = next_task(qnext);
-    if (t >= ntask) break;
-    const BTask tk = tasks[t];
-    const InstDev<S>& d = inst[tk.inst];
-    if (!d.ctl->active) continue;
-    const double dtdx = d.ctl->dt / d.dx;
-    const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
-    const GridView<S> in = d.buf[phase], out = d.buf[1 - phase];
-    const int col = tk.a * 64 + (threadIdx.x & 63);
-    const bool colok = col < d.g.nx;
-    const long i = 2 + (colok ? col : d.g.nx - 1);
-    const int j0 = 2 + (tk.b * wpb + wave) * d.yseg;
-    double cx = 0.0, cy = 0.0;
-    if (j0 < d.g.ny + 2) {  // wave-uniform
-      const int j1 = min(j0 + d.yseg, d.g.ny + 2);
-      extern __shared__ __attribute__((aligned(16))) unsigned char ylds[];
-      YStash<S>* ys = reinterpret_cast<YStash<S>*>(ylds) + wave;
-      y_march<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, inst_ghosts(d, 2, phase, ghosts),
-                                 colok, i, j0, j1, ys, cx, cy);
-    }
+  const BTask tk = tasks[blockIdx.x];
+  const InstDev<S>& d = inst[tk.inst];
+  if (!d.ctl->active) return;
+  const double dtdx = d.ctl->dt / d.dx;
+  const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
+  const GridView<S> in = d.buf[phase], out = d.buf[1 - phase];
+  const int col = tk.a * 64 + (threadIdx.x & 63);
+  const bool colok = col < d.g.nx;
+  const long i = 2 + (colok ? col : d.g.nx - 1);
+  const int j0 = 2 + (tk.b * wpb + wave) * d.yseg;
+  double cx = 0.0, cy = 0.0;
+  if (j0 < d.g.ny + 2) {  // wave-uniform
+    const int j1 = min(j0 + d.yseg, d.g.ny + 2);
+    extern __shared__ __attribute__((aligned(16))) unsigned char ylds[];
+    YStash<S>* ys = reinterpret_cast<YStash<S>*>(ylds) + wave;
+    y_march<S, ST1, false, FD>(d.g, d.ph, tr, dtdx, in, out, inst_ghosts(d, 2, phase, ghosts),
+                               colok, i, j0, j1, ys, cx, cy);
   }
 }
 
@@ -128,20 +108,17 @@ __global__ __launch_bounds__(256) void k_batch_sweep_y(const InstDev<S>* __restr
 // of one instance per task, from buffer `phase` into both buffers.
 template <typename S>
 __global__ __launch_bounds__(256) void k_batch_boundary(const InstDev<S>* inst,
-                                                        const BTask* tasks, int ntask,
-                                                        int phase) {
-  for (int t = blockIdx.x; t < ntask; t += gridDim.x) {
-    const BTask tk = tasks[t];
-    const InstDev<S>& d = inst[tk.inst];
-    if (!d.ctl->active) continue;
-    const int idim = tk.kind;
-    const int nl = (idim == 1) ? d.g.ny : d.g.nx;
-    const GridView<S> src = d.buf[phase], dst = d.buf[1 - phase];
-    const int kend = min(tk.a + kBoundaryChunk, 4 * nl);
-    for (int k = tk.a + threadIdx.x; k < kend; k += blockDim.x) {
-      const int line = k % nl, v = k / nl;
-      boundary_line<S>(idim, d.g, d.bl, d.br, d.bd, d.bu, src.p[v], dst.p[v], v, line);
-    }
+                                                        const BTask* tasks, int phase) {
+  const BTask tk = tasks[blockIdx.x];
+  const InstDev<S>& d = inst[tk.inst];
+  if (!d.ctl->active) return;
+  const int idim = tk.kind;
+  const int nl = (idim == 1) ? d.g.ny : d.g.nx;
+  const GridView<S> src = d.buf[phase], dst = d.buf[1 - phase];
+  const int kend = min(tk.a + kBoundaryChunk, 4 * nl);
+  for (int k = tk.a + threadIdx.x; k < kend; k += blockDim.x) {
+    const int line = k % nl, v = k / nl;
+    boundary_line<S>(idim, d.g, d.bl, d.br, d.bd, d.bu, src.p[v], dst.p[v], v, line);
   }
 }
 
@@ -175,9 +152,7 @@ __global__ __launch_bounds__(256) void k_batch_courant(const InstDev<S>* inst, c
 // broken down) and flags it, so one bad run cannot stall the others.
 template <typename S>
 __global__ __launch_bounds__(64) void k_batch_ctl_begin(const InstDev<S>* inst, const int* ids,
-                                                        int nids, uint64_t* qctr) {
-  // the step's sweep launches start their task queues from 0
-  if (blockIdx.x == 0 && threadIdx.x < kQueues) qctr[threadIdx.x] = 0;
+                                                        int nids) {
   for (int k = blockIdx.x; k < nids; k += gridDim.x) {
     const InstDev<S>& d = inst[ids[k]];
     RunCtl* c = d.ctl;
@@ -233,6 +208,20 @@ __global__ void k_batch_set_ctl(RunCtl* c, double t, double dt, double tend, int
   c->fault = 0;
 }
 
+// The tasks of one list entry (an instance's share of a phase) per blockIdx.x.
+__global__ __launch_bounds__(256) void k_batch_tasks(const BList* __restrict__ lists,
+                                                     BTask* __restrict__ tasks) {
+  const BList l = lists[blockIdx.x];
+  for (int k = blockIdx.y * 256 + threadIdx.x; k < l.count; k += 256 * gridDim.y)
+    tasks[l.first + k] = l.ncb > 0 ? BTask{l.inst, l.kind, k % l.ncb, k / l.ncb}
+                                   : BTask{l.inst, l.kind, k * l.per, 0};
+}
+
+void launch_batch_tasks(const BList* lists, int n, BTask* tasks, hipStream_t st) {
+  if (n <= 0) return;
+  hipLaunchKernelGGL(k_batch_tasks, dim3(n, 8), dim3(256), 0, st, lists, tasks);
+}
+
 __global__ void k_fill_u64(uint64_t* p, long n) {
   for (long k = (long) blockIdx.x * blockDim.x + threadIdx.x; k < n;
        k += (long) gridDim.x * blockDim.x)
@@ -263,79 +252,48 @@ constexpr int unit_form() {
 #endif
 }
 
-template <typename S, int FD>
-static int occupancy_fd(int kind, int waves) {
-  int nb = 0;
-  const hipError_t e =
-      kind == 1 ? hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                      &nb, k_batch_sweep_x<S, true, FD>, 64 * waves, 0)
-                : hipOccupancyMaxActiveBlocksPerMultiprocessor(
-                      &nb, k_batch_sweep_y<S, true, FD>, 64 * waves, waves * sizeof(YStash<S>));
-  if (e != hipSuccess) return 2;
-  return nb > 0 ? nb : 1;
-}
-
 template <typename S, bool ST1, int FD>
 static void launch_sweep_part(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                              int phase, bool ghosts, const BatchTune& tn, int nblocks,
-                              uint64_t* q, hipStream_t st) {
+                              int phase, bool ghosts, int waves, int xiter, hipStream_t st) {
   if (ntask <= 0) return;
-  const int nb = ntask < nblocks ? ntask : nblocks;
   if (kind == 1)
-    hipLaunchKernelGGL((k_batch_sweep_x<S, ST1, FD>), dim3(nb), dim3(64 * tn.waves), 0, st, inst,
-                       tasks, ntask, phase, (int) ghosts, tn.xiter, q);
+    hipLaunchKernelGGL((k_batch_sweep_x<S, ST1, FD>), dim3(ntask), dim3(64 * waves), 0, st, inst,
+                       tasks, phase, (int) ghosts, xiter);
   else
-    hipLaunchKernelGGL((k_batch_sweep_y<S, ST1, FD>), dim3(nb), dim3(64 * tn.waves),
-                       tn.waves * sizeof(YStash<S>), st, inst, tasks, ntask, phase, (int) ghosts, q);
+    hipLaunchKernelGGL((k_batch_sweep_y<S, ST1, FD>), dim3(ntask), dim3(64 * waves),
+                       waves * sizeof(YStash<S>), st, inst, tasks, phase, (int) ghosts);
 }
 
 template <typename S, int FD>
 static void launch_batch_sweep_fd(int kind, const InstDev<S>* inst, const BTask* tasks,
-                                  int ntask, int nst1, int phase, bool ghosts,
-                                  const BatchTune& tn, int nblocks, uint64_t* q,
-                                  hipStream_t st) {
-  launch_sweep_part<S, true, FD>(kind, inst, tasks, nst1, phase, ghosts, tn, nblocks, q, st);
-  launch_sweep_part<S, false, FD>(kind, inst, tasks + nst1, ntask - nst1, phase, ghosts, tn,
-                                  nblocks, q + 1, st);
+                                  int ntask, int nst1, int phase, bool ghosts, int waves,
+                                  int xiter, hipStream_t st) {
+  launch_sweep_part<S, true, FD>(kind, inst, tasks, nst1, phase, ghosts, waves, xiter, st);
+  launch_sweep_part<S, false, FD>(kind, inst, tasks + nst1, ntask - nst1, phase, ghosts, waves,
+                                  xiter, st);
 }
 
 #ifndef HYDRO_FAST_UNIT
 template <typename S>
-int batch_sweep_occupancy(int kind, int waves) {
-  return occupancy_fd<S, unit_form<S>()>(kind, waves);
-}
-
-template <typename S>
 void launch_batch_sweep(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                        int nst1, int phase, bool ghosts, const BatchTune& tn, int nblocks,
-                        uint64_t* q, hipStream_t st) {
-  launch_batch_sweep_fd<S, unit_form<S>()>(kind, inst, tasks, ntask, nst1, phase, ghosts, tn,
-                                           nblocks, q, st);
+                        int nst1, int phase, bool ghosts, int waves, int xiter, hipStream_t st) {
+  launch_batch_sweep_fd<S, unit_form<S>()>(kind, inst, tasks, ntask, nst1, phase, ghosts, waves,
+                                           xiter, st);
 }
-#ifdef HYDRO_BASE_UNIT
-template int batch_sweep_occupancy<double>(int, int);
 #else
-template int batch_sweep_occupancy<float>(int, int);
-#endif
-#else
-int batch_sweep_occupancy_fast(int kind, int waves) {
-  return occupancy_fd<double, kFast>(kind, waves);
-}
-
 void launch_batch_sweep_fast(int kind, const InstDev<double>* inst, const BTask* tasks,
-                             int ntask, int nst1, int phase, bool ghosts, const BatchTune& tn,
-                             int nblocks, uint64_t* q, hipStream_t st) {
-  launch_batch_sweep_fd<double, kFast>(kind, inst, tasks, ntask, nst1, phase, ghosts, tn, nblocks,
-                                       q, st);
+                             int ntask, int nst1, int phase, bool ghosts, int waves, int xiter,
+                             hipStream_t st) {
+  launch_batch_sweep_fd<double, kFast>(kind, inst, tasks, ntask, nst1, phase, ghosts, waves, xiter,
+                                       st);
 }
 #endif
 
 template <typename S>
 void launch_batch_boundary(const InstDev<S>* inst, const BTask* tasks, int ntask, int phase,
-                           int nblocks, hipStream_t st) {
+                           hipStream_t st) {
   if (ntask <= 0) return;
-  const int nb = ntask < nblocks ? ntask : nblocks;
-  hipLaunchKernelGGL(k_batch_boundary<S>, dim3(nb), dim3(256), 0, st, inst, tasks, ntask, phase);
+  hipLaunchKernelGGL(k_batch_boundary<S>, dim3(ntask), dim3(256), 0, st, inst, tasks, phase);
 }
 
 template <typename S>
@@ -348,11 +306,11 @@ void launch_batch_courant(const InstDev<S>* inst, const int* ids, int nids, hipS
 
 template <typename S>
 void launch_batch_ctl(const InstDev<S>* inst, const int* ids, int nids, bool begin,
-                      uint64_t* qctr, hipStream_t st) {
+                      hipStream_t st) {
   if (nids <= 0) return;
   if (begin) {
     const int nb = nids < 1024 ? nids : 1024;
-    hipLaunchKernelGGL(k_batch_ctl_begin<S>, dim3(nb), dim3(64), 0, st, inst, ids, nids, qctr);
+    hipLaunchKernelGGL(k_batch_ctl_begin<S>, dim3(nb), dim3(64), 0, st, inst, ids, nids);
   } else {
     hipLaunchKernelGGL(k_batch_ctl_end<S>, dim3(cdivu(nids, 256)), dim3(256), 0, st, inst, ids,
                        nids);
@@ -360,14 +318,12 @@ void launch_batch_ctl(const InstDev<S>* inst, const int* ids, int nids, bool beg
 }
 
 #define INST_ARITH(S)                                                                            \
-  template void launch_batch_sweep<S>(int, const InstDev<S>*, const BTask*, int, int, int,      \
-                                      bool, const BatchTune&, int, uint64_t*, hipStream_t);       \
+  template void launch_batch_sweep<S>(int, const InstDev<S>*, const BTask*, int, int, int, bool, \
+                                      int, int, hipStream_t);                                    \
   template void launch_batch_courant<S>(const InstDev<S>*, const int*, int, hipStream_t);
 #define INST_MOVE(S)                                                                             \
-  template void launch_batch_boundary<S>(const InstDev<S>*, const BTask*, int, int, int,        \
-                                         hipStream_t);                                           \
-  template void launch_batch_ctl<S>(const InstDev<S>*, const int*, int, bool, uint64_t*,      \
-                                    hipStream_t);
+  template void launch_batch_boundary<S>(const InstDev<S>*, const BTask*, int, int, hipStream_t); \
+  template void launch_batch_ctl<S>(const InstDev<S>*, const int*, int, bool, hipStream_t);
 #if defined(HYDRO_BASE_UNIT)
 INST_ARITH(double)
 INST_MOVE(double)

@@ -7,8 +7,6 @@ namespace hydro {
 
 constexpr int kInstSlots = 64;        // CFL max slots per instance
 constexpr int kBoundaryChunk = 1024;  // (line, var) ghost fills per boundary task
-// Task-queue counters: [phase][x, y][slope_type == 1 variant, other]
-constexpr int kQueues = 8;
 
 // One instance as the batched kernels see it (device array, rebuilt by the
 // host whenever the set of instances changes).
@@ -32,41 +30,44 @@ struct BTask {
   int inst, kind, a, b;
 };
 
+// An instance's share of one task list: `count` tasks from tasks[first] on;
+// task k has a = k * per, b = 0, or with ncb > 0 a = k % ncb, b = k / ncb.
+struct BList {
+  int inst, kind, first, count, per, ncb;
+};
+
 struct BatchTune {
   int waves;  // waves per workgroup (1..4)
-  int xiter;  // segments each wave walks in an x task
+  int xiter;  // segments each wave walks in an x task; 0: by the load
   int yseg;   // at most this many rows per wave in a y task (each instance
-              // splits its rows evenly into row groups of waves x yseg)
+              // splits its rows evenly into row groups of waves x yseg); 0:
+              // by the load
 };
 
 // kind 1: x tasks, 2: y tasks (a phase launches both, on their own tables).
 // The first nst1 tasks belong to instances with slope_type == 1.  ghosts: the
-// ghost values formed on the way are stored in buffer 0.  q: the two
-// task-queue counters of this list (zero at launch).
+// ghost values formed on the way are stored in buffer 0.  waves per
+// workgroup, xiter segments per wave in x tasks.
 template <typename S>
 void launch_batch_sweep(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
-                        int nst1, int phase, bool ghosts, const BatchTune& tn, int nblocks,
-                        uint64_t* q, hipStream_t st);
+                        int nst1, int phase, bool ghosts, int waves, int xiter, hipStream_t st);
 template <typename S>
 void launch_batch_boundary(const InstDev<S>* inst, const BTask* tasks, int ntask, int phase,
-                           int nblocks, hipStream_t st);
+                           hipStream_t st);
 template <typename S>
 void launch_batch_courant(const InstDev<S>* inst, const int* ids, int nids, hipStream_t st);
 template <typename S>
 void launch_batch_ctl(const InstDev<S>* inst, const int* ids, int nids, bool begin,
-                      uint64_t* qctr, hipStream_t st);  // begin also zeroes qctr[0..kQueues)
+                      hipStream_t st);
+void launch_batch_tasks(const BList* lists, int n, BTask* tasks, hipStream_t st);
 
 void launch_batch_set_ctl(RunCtl* c, double t, double dt, double tend, int nstep, int nstepmax,
                           int active, hipStream_t st);
 void launch_zero_u64(uint64_t* p, long n, hipStream_t st);
-template <typename S>
-int batch_sweep_occupancy(int kind, int waves);  // resident workgroups per CU
 // The FP64 fast form's batched sweeps (hydro_batch.hip, fast unit): as
-// launch_batch_sweep / batch_sweep_occupancy for double, with the kFast
-// arithmetic.
+// launch_batch_sweep for double, with the kFast arithmetic.
 void launch_batch_sweep_fast(int kind, const InstDev<double>* inst, const BTask* tasks,
-                             int ntask, int nst1, int phase, bool ghosts, const BatchTune& tn,
-                             int nblocks, uint64_t* q, hipStream_t st);
-int batch_sweep_occupancy_fast(int kind, int waves);
+                             int ntask, int nst1, int phase, bool ghosts, int waves, int xiter,
+                             hipStream_t st);
 
 }  // namespace hydro

@@ -127,8 +127,8 @@ long long hydro_amd_grid_bytes(const hydro_amd_grid *g);
 /* ---- batches: many independent grids advanced per launch ----------------
  * Each instance is a separate run of the reference time loop (own size,
  * gamma, blast, dt, t, nstep, tend/nstepmax), bit-identical to running it
- * alone with hydro_amd_grid_run.  One persistent workgroup grid per phase
- * walks a task table mixing the instances' x and y sweeps; two steps are
+ * alone with hydro_amd_grid_run.  A phase's launches take their work from task
+ * tables mixing the instances' x and y sweeps; two steps are
  * replayed as a HIP graph.  Instances are admitted against an HBM budget
  * (state buffers only) with the stream-ordered allocator, so admission and
  * retirement never synchronise the device.  All instances share one
@@ -161,8 +161,10 @@ int hydro_amd_batch_sync(hydro_amd_batch *b);
 int hydro_amd_batch_query(hydro_amd_batch *b, int *ids, double *t, int *nstep, double *dt,
                           int *active, int cap);
 /* Task shape (waves per workgroup 1..4, segments per wave in x tasks, rows per
- * wave in y tasks) and its autotuner (times the shapes on the live set; state
- * unchanged).  best[3] receives waves, xiter, yseg. */
+ * wave in y tasks; without a call 1 wave, and lengths by the live set: the
+ * square roots of its segments over 100 and of its 64-column rows over 32)
+ * and its autotuner (times the shapes on the live set; state unchanged).
+ * best[3] receives waves, xiter, yseg. */
 int hydro_amd_batch_set_tune(hydro_amd_batch *b, int waves, int xiter, int yseg);
 int hydro_amd_batch_autotune(hydro_amd_batch *b, int reps, int *best);
 
