@@ -102,7 +102,6 @@ extern "C" void hydro_amd_batch_destroy(hydro_amd_batch* b) {
   if (b->hctl) (void) hipHostFree(b->hctl);
   if (b->hidev) (void) hipHostFree(b->hidev);
   if (b->st) (void) hipStreamDestroy(b->st);
-  stage_handles(-1);
   delete b;
 }
 
@@ -113,7 +112,6 @@ extern "C" hydro_amd_batch* hydro_amd_batch_create(int precision, long long budg
     return nullptr;
   }
   hydro_amd_batch* b = new hydro_amd_batch();
-  stage_handles(+1);
   b->prec = precision;
   b->esz = dbl(b) ? 8 : 4;
   b->budget = budget_bytes > 0 ? budget_bytes : (1LL << 62);

@@ -218,7 +218,6 @@ extern "C" void hydro_amd_grid_destroy(hydro_amd_grid* g) {
   if (g->dlog) (void) hipFree(g->dlog);
   if (g->hctl) (void) hipHostFree(g->hctl);
   if (g->st) (void) hipStreamDestroy(g->st);
-  stage_handles(-1);
   delete g;
 }
 
@@ -273,7 +272,6 @@ static int write_ctl(hydro_amd_grid* g, bool fresh = false) {
 extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   if (validate(p)) return nullptr;
   hydro_amd_grid* g = new hydro_amd_grid();
-  stage_handles(+1);
   g->p = *p;
   g->prec = p->precision;
   g->esz = dbl(g) ? sizeof(double) : sizeof(float);

@@ -145,7 +145,5 @@ int stage_h2d(void* dst, int dst_esz, long dst_pitch, const void* src, int src_e
               long rows, hipStream_t st);
 // Host memory to host memory, converting (4 <-> 8 bytes an element).
 void host_copy(void* dst, int dst_esz, const void* src, int src_esz, size_t n);
-// Live grids and batches, +1 / -1: staging memory is held for them.
-void stage_handles(int d);
 
 }  // namespace hydro

@@ -9,16 +9,16 @@
 // fresh pages (5 GB/s where they are 4 KB ones), eight 30, so a large state is
 // cut into slabs of rows that up to kLanes threads carry, each through two
 // buffers of its own, the DMA of one beside the host copy of the other.
-// 8192x8192 FP64 download: 153 ms with one thread, 46 with eight; 1021x767
+// 8192x8192 FP64 download: 153 ms with one thread, 54 with eight; 1021x767
 // upload 28.4 ms through hipMemcpy2D, 0.8 so.
 #include <hip/hip_runtime.h>
 
+#include <pthread.h>
 #include <string.h>
 
 #include <algorithm>
 #include <atomic>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 #include "hydro_kernels.hpp"
@@ -28,10 +28,12 @@ extern "C" int hydro_amd_set_error(const char* fmt, ...);  // hydro_capi.cpp
 namespace hydro {
 namespace {
 // Per buffer.  The link idles about 10 us between two DMA calls: 8192x8192
-// FP64 in 72 ms with slabs of 1 MB, 54 with 2, 46 with 4 (twelve threads).
-constexpr size_t kSlabBytes = 4u << 20;
-constexpr int kLanes = 8;      // threads, two buffers each
-constexpr int kLanesKept = 4;  // whose buffers stay when no grid or batch is left
+// FP64 in 72 ms with slabs of 1 MB, 54 with 2, 46 with 4; with 2 MB the memory
+// that the process keeps pinned is 32 MB.  (To give memory back with the last
+// grid or batch made programs that make one after the other pay 0.2-0.4 ms
+// for each.)
+constexpr size_t kSlabBytes = 2u << 20;
+constexpr int kLanes = 8;  // threads, two buffers each
 // Host bytes that are worth a thread (starting one takes about 17 us; 0.4 to
 // 1.5 MB measured alike from 700x500 up).
 constexpr size_t kThreadBytes = 3u << 19;
@@ -43,8 +45,7 @@ struct Lane {
 struct Stage {
   std::mutex mu;  // one staged copy at a time per process
   Lane lane[kLanes];
-  int ready = 0;    // lanes that have their buffers
-  int handles = 0;  // live grids and batches
+  int ready = 0;  // lanes that have their buffers
 };
 Stage g_stage;
 
@@ -87,22 +88,38 @@ void convert(void* dst, int desz, const void* src, int sesz, size_t n) {
 }
 
 // Runs work(k) for k = 0..n-1, k = 0 on the calling thread and the others on
-// threads of their own, where they can be had.
+// threads of their own, where they can be had.  Their stacks are small, so that
+// the C library keeps them for the next call: eight of the usual 8 MB are
+// more than it keeps, and were they unmapped each time, the next device
+// allocations of the process took 0.3-0.7 ms longer.
+template <typename F>
+struct Share {
+  const F* work;
+  int k;
+  static void* run(void* p) {
+    const Share* s = (const Share*) p;
+    (*s->work)(s->k);
+    return nullptr;
+  }
+};
 template <typename F>
 void on_threads(int n, const F& work) {
-  std::thread th[kLanes];
+  pthread_t th[kLanes];
+  Share<F> share[kLanes];
   int started = 0;
-  for (int k = 1; k < n; k++) {
-    try {
-      th[k] = std::thread([&work, k] { work(k); });
+  pthread_attr_t attr;
+  if (n > 1 && pthread_attr_init(&attr) == 0) {
+    (void) pthread_attr_setstacksize(&attr, 1u << 20);
+    for (int k = 1; k < n; k++) {
+      share[k] = Share<F>{&work, k};
+      if (pthread_create(&th[k], &attr, Share<F>::run, &share[k]) != 0) break;
       started = k;
-    } catch (const std::system_error&) {
-      break;
     }
+    (void) pthread_attr_destroy(&attr);
   }
   work(0);
   for (int k = started + 1; k < n; k++) work(k);
-  for (int k = 1; k <= started; k++) th[k].join();
+  for (int k = 1; k <= started; k++) (void) pthread_join(th[k], nullptr);
 }
 
 int thread_count(size_t bytes) {
@@ -225,15 +242,6 @@ void host_copy(void* dst, int dst_esz, const void* src, int src_esz, size_t n) {
     const size_t a = std::min(n, per * k), m = std::min(n, a + per) - a;
     convert((char*) dst + a * dst_esz, dst_esz, (const char*) src + a * src_esz, src_esz, m);
   });
-}
-
-// A grid or batch is made (+1) or destroyed (-1): with the last one most of the
-// staging memory goes back.
-void stage_handles(int d) {
-  std::lock_guard<std::mutex> lk(g_stage.mu);
-  g_stage.handles += d;
-  if (g_stage.handles > 0) return;
-  while (g_stage.ready > kLanesKept) lane_free(g_stage.lane[--g_stage.ready]);
 }
 
 }  // namespace hydro
