@@ -162,7 +162,7 @@ __global__ __launch_bounds__(64) void k_batch_ctl_begin(const InstDev<S>* inst, 
     bool act = (t < tend) && (nstep < nstepmax) && !c->fault;
     bool bad = false;
     if (act && (nstep % 2) == 0) {
-      double dt = wave_reduce_dt(d.cour, kInstSlots, d.cf, d.dx, d.smallc);
+      double dt = wave_reduce_dt<kInstSlots>(d.cour, d.cf, d.dx, d.smallc);
       if (nstep == 0) dt = dt / 2.0;
       bad = !(dt > 0.0) || !__builtin_isfinite(dt);
       if (threadIdx.x == 0 && !bad) c->dt = dt;

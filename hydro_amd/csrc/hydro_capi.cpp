@@ -73,7 +73,6 @@ struct hydro_amd_grid {
   uint64_t* cour = nullptr;
   RunCtl* ctl = nullptr;    // [2]: even and odd steps (hydro_kernels.hpp)
   RunCtl* hctl = nullptr;   // [2], pinned host copy: every RunCtl / dt transfer goes through it
-  double* dscal = nullptr;  // device scalar for dt
   double* dlog = nullptr;
   int dlog_cap = 0;
   hipStream_t st = nullptr;
@@ -214,7 +213,6 @@ extern "C" void hydro_amd_grid_destroy(hydro_amd_grid* g) {
     if (g->mem[k]) (void) hipFree(g->mem[k]);
   if (g->cour) (void) hipFree(g->cour);
   if (g->ctl) (void) hipFree(g->ctl);
-  if (g->dscal) (void) hipFree(g->dscal);
   if (g->dlog) (void) hipFree(g->dlog);
   if (g->hctl) (void) hipHostFree(g->hctl);
   if (g->st) (void) hipStreamDestroy(g->st);
@@ -290,8 +288,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
       alloc_buffer(g, 0) || alloc_buffer(g, 1) ||
       hipMalloc(&g->cour, 2 * kCourSlots * sizeof(uint64_t)) != hipSuccess ||
       hipMalloc(&g->ctl, 2 * sizeof(RunCtl)) != hipSuccess ||
-      hipHostMalloc(&g->hctl, 2 * sizeof(RunCtl), hipHostMallocDefault) != hipSuccess ||
-      hipMalloc(&g->dscal, sizeof(double)) != hipSuccess) {
+      hipHostMalloc(&g->hctl, 2 * sizeof(RunCtl), hipHostMallocDefault) != hipSuccess) {
     if (g_err.empty()) fail("device allocation failed");
     hydro_amd_grid_destroy(g);
     return nullptr;
@@ -307,7 +304,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
 
 extern "C" long long hydro_amd_grid_bytes(const hydro_amd_grid* g) {
   return g ? (long long) (2 * (4 * g->plane + kOrigin + 64) * g->esz +
-                          2 * kCourSlots * sizeof(uint64_t) + 2 * sizeof(RunCtl) + 8 +
+                          2 * kCourSlots * sizeof(uint64_t) + 2 * sizeof(RunCtl) +
                           g->dlog_cap * 8)
            : 0;
 }
@@ -498,11 +495,11 @@ static void ensure_cour(hydro_amd_grid* g) {
 extern "C" int hydro_amd_grid_compute_deltat(hydro_amd_grid* g, double* dt) {
   if (!g || !dt) return fail("null argument");
   ensure_cour(g);
-  launch_dt_finalize(g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, g->dscal, g->st);
+  // (straight into pinned memory: a copy would be a launch more)
+  launch_dt_finalize(g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, &g->hctl->dt, g->st);
   HIPCHK(hipGetLastError());
   g->cour_dirty = false;
   g->cour_ver = 0;
-  HIPCHK(hipMemcpyAsync(&g->hctl->dt, g->dscal, sizeof(double), hipMemcpyDeviceToHost, g->st));
   HIPCHK(hipStreamSynchronize(g->st));
   *dt = g->hctl->dt;
   return 0;

@@ -129,23 +129,34 @@ __global__ __launch_bounds__(256) void k_sweep_y(GridGeom g, Phys<S> ph, double 
 
 // ---- standalone CFL maximum -------------------------------------------------
 
+// CFL maxima over a thread's cells: a wave takes 64 columns of a row, the
+// workgroup's waves consecutive rows, from row blockIdx.y * 4 + wave in strides
+// of 4 * gridDim.y (by rows and columns: with one running cell index a 64-bit
+// division per cell cost as much as the cell's arithmetic).
 template <typename S>
-__global__ __launch_bounds__(256) void k_courant(GridGeom g, Phys<S> ph, GridView<S> in,
-                                                 uint64_t* cour, const RunCtl* ctl) {
-  if (ctl && !ctl->active) return;
-  double cx = 0.0, cy = 0.0;
-  const long n = (long) g.nx * g.ny;
-  for (long t = (long) blockIdx.x * blockDim.x + threadIdx.x; t < n;
-       t += (long) gridDim.x * blockDim.x) {
-    const long jj = t / g.nx;
-    const long ii = t - jj * g.nx;
-    const long o = (jj + 2) * g.pitch + ii + 2;
+__device__ __forceinline__ void courant_cells(const GridGeom& g, const Phys<S>& ph,
+                                              const GridView<S>& in, double& cx, double& cy) {
+  const int i = (int) blockIdx.x * 64 + (threadIdx.x & 63);
+  if (i >= g.nx) return;
+  const int step = 4 * gridDim.y;
+#pragma unroll 2
+  for (int j = (int) blockIdx.y * 4 + wave_id(); j < g.ny; j += step) {
+    const long o = (j + 2L) * g.pitch + i + 2;
     S ax, ay;
     courant_cell<S>(in.p[0][o], in.p[1][o], in.p[2][o], in.p[3][o], ph, ax, ay);
     cx = maxm(cx, (double) ax);
     cy = maxm(cy, (double) ay);
   }
-  commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
+}
+
+template <typename S>
+__global__ __launch_bounds__(256) void k_courant(GridGeom g, Phys<S> ph, GridView<S> in,
+                                                 uint64_t* cour, const RunCtl* ctl) {
+  if (ctl && !ctl->active) return;
+  double cx = 0.0, cy = 0.0;
+  courant_cells<S>(g, ph, in, cx, cy);
+  commit_courant(cx, cy, cour, kCourSlots,
+                 (blockIdx.y * gridDim.x + blockIdx.x) % kCourSlots);
 }
 
 // ---- ghost cells -------------------------------------------------------------
@@ -169,7 +180,7 @@ __global__ __launch_bounds__(256) void k_boundary(int idim, GridGeom g, int bl, 
 
 __global__ __launch_bounds__(64) void k_dt_finalize(uint64_t* cour, double cf, double dx,
                                                     double smallc, double* dt_out) {
-  const double dt = wave_reduce_dt(cour, kCourSlots, cf, dx, smallc);
+  const double dt = wave_reduce_dt<kCourSlots>(cour, cf, dx, smallc);
   if (threadIdx.x == 0) *dt_out = dt;
 }
 
@@ -181,7 +192,7 @@ __global__ __launch_bounds__(64) void k_ctl_begin(RunCtl* ctl, uint64_t* cour, d
   if (threadIdx.x != 0) c.log = nullptr;  // one thread logs
   close_step(c);
   if ((c.t < c.tend) && (c.nstep < c.nstepmax)) {  // wave-uniform
-    c.dt = wave_reduce_dt(cour, kCourSlots, cf, dx, smallc);
+    c.dt = wave_reduce_dt<kCourSlots>(cour, cf, dx, smallc);
     if (c.nstep == 0) c.dt = c.dt / 2.0;
     c.active = 1;
   }
@@ -394,16 +405,20 @@ void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView
 }
 #endif
 
+// Workgroups of a CFL pass: 64 columns x 4 rows each, the rows strided over at
+// most about 2048 of them (8 waves a SIMD).
+static dim3 courant_grid(const GridGeom& g) {
+  const unsigned ncb = cdiv(g.nx, 64);
+  const unsigned rows = cdiv(g.ny, 4), most = ncb < 2048 ? 2048 / ncb : 1;
+  return dim3(ncb, rows < most ? rows : most);
+}
+
 template <typename S>
 void launch_courant(const GridGeom& g, const PhysArgs& pa, GridView<S> in, uint64_t* cour,
                     const RunCtl* ctl, hipStream_t st) {
   const Phys<S> ph = make_phys<S>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type, pa.niter,
                                   pa.iorder, pa.scheme);
-  const long n = (long) g.nx * g.ny;
-  long nb = cdiv(n, 256 * 8);
-  if (nb > 4096) nb = 4096;
-  if (nb < 1) nb = 1;
-  hipLaunchKernelGGL(k_courant<S>, dim3((unsigned) nb), dim3(256), 0, st, g, ph, in, cour, ctl);
+  hipLaunchKernelGGL(k_courant<S>, courant_grid(g), dim3(256), 0, st, g, ph, in, cour, ctl);
 }
 
 #ifdef HYDRO_BASE_UNIT

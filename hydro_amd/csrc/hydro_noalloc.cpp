@@ -4,7 +4,7 @@
 // The kernels are those of hydro_amd_grid_compute_deltat (k_courant, then
 // k_dt_finalize; hydro_kernels.hip).  Their scratch, the CFL max-slots, is a
 // file-scope device array here instead of a grid's hipMalloc'ed buffer, so a
-// call allocates nothing: it queues three kernels on the caller's stream and
+// call allocates nothing: it queues two kernels on the caller's stream and
 // returns, which also makes it capturable into a HIP graph.
 //
 // The array exists once per GPU (each device holds its own copy until the
@@ -13,8 +13,9 @@
 // that device current, and that address is what the launches take.  All calls
 // on one GPU share the array: calls that overlap on one GPU (different
 // streams, or different host threads) race on it; calls queued in order on
-// one stream do not.  Each call clears the slots first, with a fill kernel
-// rather than a memset node.
+// one stream do not.  The slots are zero when the process starts, and
+// k_dt_finalize, which is the last kernel of every call, leaves them so (a
+// launch that cleared them first was a third of a small grid's call).
 #include <hip/hip_runtime.h>
 
 #include <mutex>
@@ -91,7 +92,6 @@ extern "C" int hydro_amd_compute_deltat_noalloc(const hydro_amd_params* p, const
   ph.iorder = p->iorder;
   ph.scheme = p->scheme;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  launch_clear_slots(slots, st);
   launch_courant<double>(g, ph, v, slots, nullptr, st);
   launch_dt_finalize(slots, p->courant_factor, p->dx, p->smallc, d_dt, st);
   const hipError_t e = hipGetLastError();

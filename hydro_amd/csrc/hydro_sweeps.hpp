@@ -108,18 +108,33 @@ __device__ __forceinline__ void commit_courant(double cx, double cy, uint64_t* c
   __syncthreads();
 }
 
-// Max over nslot slot pairs (clearing them), then compute_deltat.c:197:
+// Max over NSLOT slot pairs (clearing them), then compute_deltat.c:197:
 // dt = cfl*dx / MAX(cx, MAX(cy, smallc)).  Called by one whole wave; every
-// lane returns the same dt.
-__device__ __forceinline__ double wave_reduce_dt(uint64_t* cour, int nslot, double cf, double dx,
+// lane returns the same dt.  (All loads go out before the first is used: with
+// a load, a clearing store and a maximum per trip the 1024 pairs of a grid
+// took sixteen round trips to memory.)
+template <int NSLOT>
+__device__ __forceinline__ double wave_reduce_dt(uint64_t* cour, double cf, double dx,
                                                  double smallc) {
-  double cx = 0.0, cy = 0.0;
+  constexpr int K = NSLOT / 64;
+  static_assert(NSLOT % 64 == 0, "whole slots a lane");
   const int lane = threadIdx.x & 63;
-  for (int s = lane; s < nslot; s += 64) {
-    cx = maxm(cx, __longlong_as_double((long long) cour[s]));
-    cy = maxm(cy, __longlong_as_double((long long) cour[nslot + s]));
-    cour[s] = 0;
-    cour[nslot + s] = 0;
+  uint64_t x[K], y[K];
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    x[k] = cour[lane + 64 * k];
+    y[k] = cour[NSLOT + lane + 64 * k];
+  }
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    cour[lane + 64 * k] = 0;
+    cour[NSLOT + lane + 64 * k] = 0;
+  }
+  double cx = 0.0, cy = 0.0;
+#pragma unroll
+  for (int k = 0; k < K; k++) {
+    cx = maxm(cx, __longlong_as_double((long long) x[k]));
+    cy = maxm(cy, __longlong_as_double((long long) y[k]));
   }
   cx = wave_max(cx);
   cy = wave_max(cy);

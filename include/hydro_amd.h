@@ -238,7 +238,7 @@ double hydro_amd_stream_probe(long long cells, int reps);
  * [4][ny+4][nx+4] (d_uold); dt is written to the device double d_dt.  The
  * kernels are queued on `stream` (a hipStream_t; NULL = the null stream) and
  * the call returns without waiting.  Scratch: a 16 KiB file-scope device
- * array per GPU (the CFL max-slots), cleared at the start of every call; no
+ * array per GPU (the CFL max-slots), zero again after every call; no
  * hipMalloc or hipFree, any grid size up to (nx+4)*(ny+4) = 2^40.  Calls that
  * overlap on one GPU (other streams, other threads) race on that array. */
 int hydro_amd_compute_deltat_noalloc(const hydro_amd_params *p, const double *d_uold,
