@@ -79,7 +79,7 @@ struct hydro_amd_grid {
   long state_ver = 1;
   long cour_ver = 0;     // state version whose CFL maxima the slots hold (0: none)
   bool cour_dirty = false;
-  SweepTune tune = {0, 1, 4, 8};  // set by precision at creation
+  SweepTune tune = {0, 1, 0, 0};  // set by precision at creation
   // host mirror of the run control, valid between calls
   double t = 0, dt = 0;
   int nstep = 0;
@@ -273,9 +273,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   g->p = *p;
   g->prec = p->precision;
   g->esz = dbl(g) ? sizeof(double) : sizeof(float);
-  // the 4-wave LDS x form in both precisions (FP64: within 2 % of the DPP
-  // form at 8192^2 and faster on small grids; mixed: its fastest form)
-  g->tune = dbl(g) ? SweepTune{0, 1, 4, 8} : SweepTune{0, 4, 4, 16};
+  g->tune = SweepTune{0, dbl(g) ? 1 : 4, 0, 0};
   g->geom.nx = p->nx;
   g->geom.ny = p->ny;
   g->geom.pitch = ((long) p->nx + 4 + 31) / 32 * 32;

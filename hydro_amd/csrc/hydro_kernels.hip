@@ -293,6 +293,28 @@ static int y_rows(long ncolblk, long ny, int most) {
   return (int) cdiv(ny, nseg);
 }
 
+// The x sweep's form and the row pieces that a workgroup walks, when the caller
+// has not said.  The one-wave form (64-cell pieces) is the faster one in FP64
+// at every size (8192x8192: 1.45 against 1.48 ms a sweep, 2048x1536: 200
+// against 212 us a step) and in the other forms on small and middle grids
+// (2048x1536: fast 119 against 123 us a step, mixed 85 against 88; 1021x767:
+// 68 / 71, 57 / 59); the four-wave form, with fewer halo cells, where there are
+// enough of its pieces to fill the GPU many times over (8192x1024, 33800
+// pieces: 285 / 288; 8192x8192 1.83 / 1.88 ms).  The number of pieces goes by
+// the square root, as y_rows; the best measured, one wave: 1 at 1021x767, 3 at
+// 2048x1536, 4 at 4099x3001, 8-16 at 8192x8192, 16-32 at 16384x12000; four
+// waves: 6 at 8192x1024, 6-8 at 4099x3001 and 8192x8192, 16-32 at 16384x12000.
+template <typename S, int FD>
+static int x_waves(const GridGeom& g) {
+  if (sizeof(S) == 8 && FD != kFast) return 1;
+  return (long) cdiv(g.nx, 64 * 4 - 4) * g.ny >= 24000 ? 4 : 1;
+}
+static int x_pieces(long n, int by, int most) {
+  int k = 1;
+  while (k < most && (long) by * by * (k + 1) * (k + 1) <= n) k++;
+  return k;
+}
+
 // The sweep launch for one arithmetic form FD (shapes as in launch_sweep).
 template <typename S, int FD>
 static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, double dx,
@@ -308,12 +330,15 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
       if (c) F(false, true); else F(false, false);  \
     }                                       \
   } while (0)
-  if (idim == 1 && (tune.xwaves == 2 || tune.xwaves == 4)) {
-    const int W = tune.xwaves;
+  int xwaves = tune.xwaves;
+  if (xwaves <= 0) xwaves = x_waves<S, FD>(g);
+  if (idim == 1 && (xwaves == 2 || xwaves == 4)) {
+    const int W = xwaves;
     const int nseg = (int) cdiv(g.nx, 64 * W - 4);
     const long pieces = (long) nseg * g.ny;
-    int xiter = tune.xiter > 0 ? tune.xiter : 8;
-    while (xiter > 1 && cdiv(pieces, xiter) < 1024) xiter >>= 1;
+    int xiter = tune.xiter;
+    if (xiter <= 0) xiter = x_pieces(pieces, 32, 16);
+    else while (xiter > 1 && cdiv(pieces, xiter) < 1024) xiter >>= 1;
     const dim3 grid(cdiv(pieces, xiter)), blk(64 * W);
 #define HXB(A, B, WW) \
   hipLaunchKernelGGL((k_sweep_xb<S, A, B, WW, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, \
@@ -325,10 +350,11 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
   } else if (idim == 1) {
     const int nseg = (int) cdiv(g.nx, kXSeg);
     const long waves = (long) nseg * g.ny;
-    const int xw = tune.xwaves > 0 ? tune.xwaves : 4;
-    int xiter = tune.xiter > 0 ? tune.xiter : 8;
-    // keep at least ~4 workgroups per CU before walking several segments
-    while (xiter > 1 && cdiv(waves, (long) xw * xiter) < 1024) xiter >>= 1;
+    const int xw = xwaves;
+    int xiter = tune.xiter;
+    if (xiter <= 0) xiter = x_pieces(waves, 100, 32);
+    // (given: keep at least ~4 workgroups per CU before walking several segments)
+    else while (xiter > 1 && cdiv(waves, (long) xw * xiter) < 1024) xiter >>= 1;
     const dim3 grid(cdiv(waves, (long) xw * xiter)), blk(64 * xw);
 #define HX(A, B) \
   hipLaunchKernelGGL((k_sweep_x<S, A, B, FD>), grid, blk, 0, st, g, ph, dx, dt_val, ctl, nxt, \

@@ -66,8 +66,8 @@ constexpr int kGhostMin = 3;
 struct SweepTune {
   int yseg;     // rows per y-sweep thread (column march length); 0: by the grid's size
   int ywaves;   // waves per y-sweep workgroup (1..4)
-  int xwaves;   // waves per x-sweep workgroup (1..4)
-  int xiter;    // row segments each x-sweep wave walks
+  int xwaves;   // waves per x-sweep workgroup (1..4); 0: by the grid's size
+  int xiter;    // row segments each x-sweep wave walks; 0: by the grid's size
 };
 
 // ---- launchers (hydro_kernels.hip) -----------------------------------------

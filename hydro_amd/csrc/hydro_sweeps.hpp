@@ -191,45 +191,44 @@ __device__ __forceinline__ int ghost_source(int idim, int n, int lo, int hi, int
   return low ? n + gi : gi - n;
 }
 
-// The conserved values at padded column i (at most nx+3 is read) of the row
-// at `base`, ghosts formed; o: where the cell was read (its own place for an
-// interior cell).  edge: the row piece touches ghost columns (wave-uniform).
-template <typename S>
-__device__ __forceinline__ void load_x(const GridGeom& g, const GridView<S>& in,
-                                       const GridView<S>& out, const GhostFill& gf, long base,
-                                       int i, bool edge, long& o, S& U0, S& U1, S& U2, S& U3) {
+// Where the cell of padded column i (nx+3 at most) of a row is read: its own
+// column, or a ghost's source.  edge: the row piece touches ghost columns
+// (wave-uniform).
+__device__ __forceinline__ int x_source(const GridGeom& g, const GhostFill& gf, int i, bool edge) {
   const int ic = i < g.nx + 4 ? i : g.nx + 3;
-  if (!edge) {
-    o = base + ic;
-    U0 = in.p[0][o];
-    U1 = in.p[1][o];
-    U2 = in.p[2][o];
-    U3 = in.p[3][o];
-    return;
-  }
-  bool neg = false;
-  const bool ghost = ic < 2 || ic >= g.nx + 2;
-  const int is = ghost ? ghost_source(1, g.nx, gf.lo, gf.hi, ic, neg) : ic;
-  o = base + is;
-  U0 = in.p[0][o];
-  U1 = in.p[1][o];
-  U2 = in.p[2][o];
-  U3 = in.p[3][o];
+  bool neg;
+  return edge && (ic < 2 || ic >= g.nx + 2) ? ghost_source(1, g.nx, gf.lo, gf.hi, ic, neg) : ic;
+}
+// Makes the cell just read at its source the ghost it stands for: reflected,
+// and stored.  Kept apart from the load, so that it waits for the values only
+// where they are needed anyway (in the LDS form a piece later: the sign change
+// at the load cost the whole sweep 2-3 %).  o: where it was read.
+template <typename S>
+__device__ __forceinline__ void x_ghost(const GridGeom& g, const GridView<S>& in,
+                                        const GridView<S>& out, const GhostFill& gf, long o,
+                                        int i, S U0, S& U1, S U2, S U3) {
+  const int ic = i < g.nx + 4 ? i : g.nx + 3;
+  if (ic >= 2 && ic < g.nx + 2) return;
+  bool neg;
+  const int is = ghost_source(1, g.nx, gf.lo, gf.hi, ic, neg);
   if (neg) U1 = -U1;
   if (is != i && i == ic && gf.to != 0) {
     const GridView<S>& d = gf.to == 1 ? in : out;
-    d.p[0][base + i] = U0;
-    d.p[1][base + i] = U1;
-    d.p[2][base + i] = U2;
-    d.p[3][base + i] = U3;
+    const long og = o - is + i;
+    d.p[0][og] = U0;
+    d.p[1][og] = U1;
+    d.p[2][og] = U2;
+    d.p[3][og] = U3;
   }
 }
 
 // FD, the arithmetic form (hydro_numerics.hpp): kGated -- the range-gated
 // FP64 divisions may be used (FP64 launches with enough waves to keep the
 // SIMDs busy); kIeee -- the IEEE code alone; kFast -- the FP64 fast form.
-template <typename S, bool ST1, bool COUR, int FD>
-__device__ __forceinline__ void x_segment(const GridGeom& g, const Phys<S>& ph,
+// EDGE: the segment touches ghost columns (x_segment picks; the other form has
+// none of the ghosts' code in it).
+template <typename S, bool ST1, bool COUR, int FD, bool EDGE>
+__device__ __forceinline__ void x_segment_at(const GridGeom& g, const Phys<S>& ph,
                                           const TraceK<S>& tk, double dtdx,
                                           const GridView<S>& in, const GridView<S>& out,
                                           const GhostFill& gf, long jrow, int seg, double& cx,
@@ -237,10 +236,11 @@ __device__ __forceinline__ void x_segment(const GridGeom& g, const Phys<S>& ph,
   const int lane = threadIdx.x & 63;
   const long j = jrow + 2;
   const int i = kXSeg * seg + lane;  // padded column of this lane
-  const bool edge = seg == 0 || kXSeg * seg + 63 >= g.nx + 2;
-  long o;
-  S U0, U1, U2, U3;
-  load_x<S>(g, in, out, gf, j * g.pitch, i, edge, o, U0, U1, U2, U3);
+  // (o is its own cell where it is updated)
+  const long o = j * g.pitch + (EDGE ? x_source(g, gf, i, true) : i);
+  const S U0 = in.p[0][o], U2 = in.p[2][o], U3 = in.p[3][o];
+  S U1 = in.p[1][o];
+  if (EDGE) x_ghost<S>(g, in, out, gf, o, i, U0, U1, U2, U3);
   Prim<S> pc;
   bool fc = false;
   if constexpr (FD == kFast) {
@@ -284,6 +284,18 @@ __device__ __forceinline__ void x_segment(const GridGeom& g, const Phys<S>& ph,
   }
 }
 
+template <typename S, bool ST1, bool COUR, int FD>
+__device__ __forceinline__ void x_segment(const GridGeom& g, const Phys<S>& ph,
+                                          const TraceK<S>& tk, double dtdx,
+                                          const GridView<S>& in, const GridView<S>& out,
+                                          const GhostFill& gf, long jrow, int seg, double& cx,
+                                          double& cy) {
+  if (seg == 0 || kXSeg * seg + 63 >= g.nx + 2)  // wave-uniform
+    x_segment_at<S, ST1, COUR, FD, true>(g, ph, tk, dtdx, in, out, gf, jrow, seg, cx, cy);
+  else
+    x_segment_at<S, ST1, COUR, FD, false>(g, ph, tk, dtdx, in, out, gf, jrow, seg, cx, cy);
+}
+
 // ---- x sweep, workgroup form: W waves share one row piece through LDS ------
 
 // LDS of one workgroup: three exchange buffers (primitives, right-face states,
@@ -321,7 +333,7 @@ __device__ __forceinline__ Q4<S> lds_get(const S (&b)[4][64 * W + 2], int slot) 
 template <typename S>
 struct XCell {
   long o;
-  int i;
+  int i0;  // the piece's first column (workgroup-uniform)
   S U0, U1, U2, U3;
   Prim<S> pc;
   bool fc;
@@ -353,16 +365,21 @@ __device__ __forceinline__ void x_blocks(const GridGeom& g, const Phys<S>& ph,
   const int t = threadIdx.x;
   SegWalk w(first, nseg);
   if (npieces <= 0 || w.row >= g.ny) return;  // workgroup-uniform
+  // whether a piece touches ghost columns
+  auto edge = [&](int i0) { return i0 == 0 || i0 + N > g.nx + 2; };
   // a piece's cell: its loads, then its primitives (published)
   auto fetch = [&](const SegWalk& ww) {
     XCell<S> c;
-    c.i = (N - 4) * ww.seg + t;
-    const bool edge = ww.seg == 0 || (N - 4) * ww.seg + N > g.nx + 2;
-    load_x<S>(g, in, out, gf, ((long) ww.row + 2) * g.pitch, c.i, edge, c.o, c.U0, c.U1, c.U2,
-              c.U3);
+    c.i0 = (N - 4) * ww.seg;
+    c.o = ((long) ww.row + 2) * g.pitch + x_source(g, gf, c.i0 + t, edge(c.i0));
+    c.U0 = in.p[0][c.o];
+    c.U1 = in.p[1][c.o];
+    c.U2 = in.p[2][c.o];
+    c.U3 = in.p[3][c.o];
     return c;
   };
   auto prims = [&](XCell<S>& c) {
+    if (edge(c.i0)) x_ghost<S>(g, in, out, gf, c.o, c.i0 + t, c.U0, c.U1, c.U2, c.U3);
     c.fc = false;
     // kGated: FastDiv for the primitives when the wave's cells are in range,
     // for the traces when every wave's are (the slopes read neighbours of
@@ -384,7 +401,7 @@ __device__ __forceinline__ void x_blocks(const GridGeom& g, const Phys<S>& ph,
   // update a piece from its own right-face flux and the left neighbour's
   auto update = [&](const XCell<S>& c, const Q4<double>& fr) {
     const Q4<double> fl = lds_get<W>(sh.f, t);
-    const bool wr = t >= 2 && t <= N - 3 && c.i <= g.nx + 1;
+    const bool wr = t >= 2 && t <= N - 3 && c.i0 + t <= g.nx + 1;
     const double n0 = update1<S>(c.U0, fl.r, fr.r, dtdx);
     const double n1 = update1<S>(c.U1, fl.u, fr.u, dtdx);
     const double n2 = update1<S>(c.U2, fl.v, fr.v, dtdx);
@@ -500,29 +517,28 @@ __device__ __forceinline__ Cell<S> stash_get_cell(const S (&b)[4][64], int lane)
   return Cell<S>{b[0][lane], b[1][lane], b[2][lane], b[3][lane]};
 }
 
-// Column i of padded row j (wave-uniform), a ghost row formed from its source.
 template <typename S>
-__device__ __forceinline__ Cell<S> load_y(const GridGeom& g, const GridView<S>& in,
-                                          const GridView<S>& out, const GhostFill& gf, bool colok,
-                                          int j, long i) {
-  const bool ghost = j < 2 || j >= g.ny + 2;
-  bool neg = false;
-  const int js = ghost ? ghost_source(2, g.ny, gf.lo, gf.hi, j, neg) : j;
-  const long o = (long) js * g.pitch + i;
+__device__ __forceinline__ Cell<S> load_y(const GridView<S>& in, long o) {
   // gather with the IU/IV swap of conservar.c:106-109
-  Cell<S> u{in.p[0][o], in.p[2][o], in.p[1][o], in.p[3][o]};
-  if (ghost) {  // wave-uniform
-    if (neg) u.u1 = -u.u1;
-    if (js != j && gf.to != 0 && colok) {
-      const GridView<S>& d = gf.to == 1 ? in : out;
-      const long od = (long) j * g.pitch + i;
-      d.p[0][od] = u.u0;
-      d.p[2][od] = u.u1;
-      d.p[1][od] = u.u2;
-      d.p[3][od] = u.u3;
-    }
+  return Cell<S>{in.p[0][o], in.p[2][o], in.p[1][o], in.p[3][o]};
+}
+
+// As x_ghost, for column i of padded row j (wave-uniform).
+template <typename S>
+__device__ __forceinline__ void y_ghost(const GridGeom& g, const GridView<S>& in,
+                                        const GridView<S>& out, const GhostFill& gf, bool colok,
+                                        int j, long i, Cell<S>& u) {
+  bool neg;
+  const int js = ghost_source(2, g.ny, gf.lo, gf.hi, j, neg);
+  if (neg) u.u1 = -u.u1;
+  if (js != j && gf.to != 0 && colok) {
+    const GridView<S>& d = gf.to == 1 ? in : out;
+    const long o = (long) j * g.pitch + i;
+    d.p[0][o] = u.u0;
+    d.p[2][o] = u.u1;
+    d.p[1][o] = u.u2;
+    d.p[3][o] = u.u3;
   }
-  return u;
 }
 
 template <typename S, bool ST1, bool COUR, int FD>
@@ -536,11 +552,26 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
   const bool o1 = ph.iorder == 1;
 
   // prologue: cells j0-2 .. j0+1
-  auto load = [&](int j) { return load_y<S>(g, in, out, gf, colok, j, i); };
-  Cell<S> ua = load(j0 - 2);
-  Cell<S> ub = load(j0 - 1);
+  // (a ghost row is read at its source and made a ghost where it is used)
+  const int top = g.ny + 2;
+  bool neg;
+  const int s0 = ghost_source(2, g.ny, gf.lo, gf.hi, 0, neg);
+  const int s1 = ghost_source(2, g.ny, gf.lo, gf.hi, 1, neg);
+  const int s2 = ghost_source(2, g.ny, gf.lo, gf.hi, top, neg);
+  const int s3 = ghost_source(2, g.ny, gf.lo, gf.hi, top + 1, neg);
+  auto load = [&](int j) {
+    const int js = j >= top ? (j == top ? s2 : s3) : j;
+    return load_y<S>(in, (long) js * P + i);
+  };
+  Cell<S> ua = load_y<S>(in, (long) (j0 == 2 ? s0 : j0 == 3 ? s1 : j0 - 2) * P + i);
+  Cell<S> ub = load_y<S>(in, (long) (j0 == 2 ? s1 : j0 - 1) * P + i);
   Cell<S> uc = load(j0);
   Cell<S> ud = load(j0 + 1);
+  if (j0 < 4) {
+    y_ghost<S>(g, in, out, gf, colok, j0 - 2, i, ua);
+    if (j0 == 2) y_ghost<S>(g, in, out, gf, colok, 1, i, ub);
+  }
+  if (j0 + 1 >= top) y_ghost<S>(g, in, out, gf, colok, j0 + 1, i, ud);
   // rows j0 and j0+1 await their updates
   stash_put_cell(ys->u[j0 % 3], lane, uc);
   stash_put_cell(ys->u[(j0 + 1) % 3], lane, ud);
@@ -592,7 +623,8 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
     // the values in registers)
     asm volatile("" ::: "memory");
     const long oc = (long) (j - 2) * P + i;
-    const Cell<S> uE = uN;
+    Cell<S> uE = uN;
+    if (j >= top) y_ghost<S>(g, in, out, gf, colok, j, i, uE);
     const int sj = j % 3;  // wave-uniform
     stash_put_cell(ys->u[sj], lane, uE);
     const int jn = j + 1 <= j1 + 1 ? j + 1 : j1 + 1;  // last row: a harmless reload

@@ -104,9 +104,10 @@ int hydro_amd_grid_set_limits(hydro_amd_grid *g, double tend, int nstepmax);
  * (1..4) and row pieces each x-sweep workgroup walks.  With 2 or 4 x waves
  * the workgroup shares one row piece of 64*xwaves cells through LDS; with 1
  * or 3 each wave takes its own 64-cell piece and exchanges neighbours by DPP
- * lane rotations.  A new grid starts with (1, 4, 8) for the last three in
- * FP64 and (4, 4, 16) in mixed precision, and rows by its size: the square
- * root of (nx / 64) * ny over 32, between 1 and 64 (32 in the fast form). */
+ * lane rotations.  A new grid's shape goes by its size: y rows by the square
+ * root of (nx / 64) * ny over 32, between 1 and 64 (32 in the fast form); in x
+ * the one-wave form, or the four-wave form on large grids of the fast and
+ * mixed forms, and row pieces by the square root of their number. */
 int hydro_amd_grid_set_tune(hydro_amd_grid *g, int yseg, int ywaves, int xwaves, int xiter);
 /* Autotuner: times the candidate launch shapes of both sweeps on this grid
  * (reps launches each, HIP events; the sweeps read the state and write only
