@@ -403,12 +403,15 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
   // keeps the SIMDs busy.  A sweep of a small grid has too few waves for
   // that: each wave's march is latency-bound, and the gates' wave-wide
   // tests, branches and larger code lengthen it, so such launches run the
-  // kIeee kernels (the results are the same bits either way).
+  // kIeee kernels (the results are the same bits either way).  y sweep of a
+  // flow that moves everywhere, gated / IEEE, as part of a step: 250x125 22.5 /
+  // 21.8 us, 1021x767 (4096 waves) 72 / 72, 1531x1200 138 / 144, 2048x1536 218 / 229.
   constexpr long kFastDivWaves = 4096;  // 4 waves per SIMD on 256 CUs
   if constexpr (sizeof(S) == 8) {
-    const bool fd = ph.fastdiv &&
-                    (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny
-                               : (long) cdiv(g.nx, 64) * cdiv(g.ny, 16)) >= kFastDivWaves;
+    const long ncb = cdiv(g.nx, 64);
+    const long rows = tune.yseg > 0 ? 16 : y_rows(ncb, g.ny, 64);
+    const bool fd = ph.fastdiv && (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny
+                                             : ncb * cdiv(g.ny, rows)) >= kFastDivWaves;
     if (fd)
       launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, nxt, cour, tune,
                                  st1, st);
