@@ -76,17 +76,18 @@ struct hydro_amd_grid {
   double* dlog = nullptr;
   int dlog_cap = 0;
   hipStream_t st = nullptr;
+  int cur = 0;           // the buffer that holds the state
   long state_ver = 1;
   long cour_ver = 0;     // state version whose CFL maxima the slots hold (0: none)
   bool cour_dirty = false;
-  SweepTune tune = {0, 1, 0, 0};  // set by precision at creation
+  SweepTune tune = {0, 1, 0, 0, -1};  // set by precision at creation
   // host mirror of the run control, valid between calls
   double t = 0, dt = 0;
   int nstep = 0;
   bool queued = false;  // steps were queued that the mirror does not show yet
-  // cached two-step graph
-  hipGraphExec_t gexec = nullptr;
-  bool gexec_cour = false;
+  bool flips = false;   // each of them moves the state to the other buffer
+  // cached two-step graphs, by the buffer that the even step reads
+  hipGraphExec_t gexec[2] = {nullptr, nullptr};
   // kernel timing: events around each sweep / boundary launch (graphs off)
   bool prof = false;
   std::vector<hipEvent_t> ev_pool;
@@ -198,10 +199,11 @@ extern "C" void hydro_amd_params_from_surface(const hydroparam_t* H, hydro_amd_p
 }
 
 static void drop_graph(hydro_amd_grid* g) {
-  if (g->gexec) {
-    (void) hipGraphExecDestroy(g->gexec);
-    g->gexec = nullptr;
-  }
+  for (auto& e : g->gexec)
+    if (e) {
+      (void) hipGraphExecDestroy(e);
+      e = nullptr;
+    }
 }
 
 extern "C" void hydro_amd_grid_destroy(hydro_amd_grid* g) {
@@ -273,7 +275,7 @@ extern "C" hydro_amd_grid* hydro_amd_grid_create(const hydro_amd_params* p) {
   g->p = *p;
   g->prec = p->precision;
   g->esz = dbl(g) ? sizeof(double) : sizeof(float);
-  g->tune = SweepTune{0, dbl(g) ? 1 : 4, 0, 0};
+  g->tune = SweepTune{0, dbl(g) ? 1 : 4, 0, 0, -1};
   g->geom.nx = p->nx;
   g->geom.ny = p->ny;
   g->geom.pitch = ((long) p->nx + 4 + 31) / 32 * 32;
@@ -309,12 +311,18 @@ extern "C" long long hydro_amd_grid_bytes(const hydro_amd_grid* g) {
 
 static void bump(hydro_amd_grid* g) { g->state_ver++; }
 
+static int run_finish(hydro_amd_grid* g, int* steps_done);
+
+// Takes up the outcome of queued steps: which buffer the state is in, t, nstep.
+static int settle(hydro_amd_grid* g) { return g->queued ? run_finish(g, nullptr) : 0; }
+
 static int do_init(hydro_amd_grid* g, int bx, int by0, int by1, double e) {
   if (dbl(g))
     launch_init<double>(g->geom, g->vd[0], g->vd[1], bx, by0, by1, e, g->st);
   else
     launch_init<float>(g->geom, g->vf[0], g->vf[1], bx, by0, by1, e, g->st);
   HIPCHK(hipGetLastError());
+  g->cur = 0;
   bump(g);
   g->t = 0;
   g->nstep = 0;
@@ -343,6 +351,7 @@ extern "C" int hydro_amd_grid_init_blast(hydro_amd_grid* g, int bx, int by, doub
 
 extern "C" int hydro_amd_grid_upload(hydro_amd_grid* g, const double* u) {
   if (!g || !u) return fail("null argument");
+  if (settle(g)) return -1;
   const long nxt = g->p.nx + 4, rows = 4L * (g->p.ny + 4);
   void* dst = (char*) g->mem[0] + kOrigin * g->esz;
   if (stage_h2d(dst, (int) g->esz, g->geom.pitch, u, 8, nxt, rows, g->st)) return -1;
@@ -350,14 +359,16 @@ extern "C" int hydro_amd_grid_upload(hydro_amd_grid* g, const double* u) {
   const long total = 4 * g->plane + kOrigin + 64;
   HIPCHK(hipMemcpyAsync(g->mem[1], g->mem[0], (size_t) total * g->esz,
                         hipMemcpyDeviceToDevice, g->st));
+  g->cur = 0;
   bump(g);
   return 0;
 }
 
 extern "C" int hydro_amd_grid_download(hydro_amd_grid* g, double* u) {
   if (!g || !u) return fail("null argument");
+  if (settle(g)) return -1;
   const long nxt = g->p.nx + 4, rows = 4L * (g->p.ny + 4);
-  const void* src = (const char*) g->mem[0] + kOrigin * g->esz;
+  const void* src = (const char*) g->mem[g->cur] + kOrigin * g->esz;
   return stage_d2h(u, 8, src, (int) g->esz, g->geom.pitch, nxt, rows, g->st) ? -1 : 0;
 }
 
@@ -376,14 +387,15 @@ extern "C" int hydro_amd_grid_image(hydro_amd_grid* g, int shrink_size, unsigned
   const long long need = 3LL * w * h;
   if (cap < need) return fail("image buffer of %lld bytes, %lld needed", cap, need);
   if (need == 0) return 0;
+  if (settle(g)) return -1;
   void* d = nullptr;  // [8-byte maximum key][pixels]
   HIPCHK(hipMallocAsync(&d, (size_t) (8 + need), g->st));
   unsigned long long* key = (unsigned long long*) d;
   unsigned char* px = (unsigned char*) d + 8;
   if (dbl(g))
-    launch_image<double>(g->geom, g->vd[0].p[0], s, w, h, key, px, g->st);
+    launch_image<double>(g->geom, g->vd[g->cur].p[0], s, w, h, key, px, g->st);
   else
-    launch_image<float>(g->geom, g->vf[0].p[0], s, w, h, key, px, g->st);
+    launch_image<float>(g->geom, g->vf[g->cur].p[0], s, w, h, key, px, g->st);
   const hipError_t e1 = hipMemcpyAsync(rgb, px, (size_t) need, hipMemcpyDeviceToHost, g->st);
   const hipError_t e2 = hipFreeAsync(d, g->st);
   const hipError_t e3 = hipStreamSynchronize(g->st);
@@ -409,11 +421,11 @@ static bool folds_ghosts(const hydro_amd_grid* g) {
 }
 
 // One sweep with its ghosts, reading buffer `src` and writing the other; the
-// ghost values are left in buffer 0, the state between steps.
-static void enq_sweep(hydro_amd_grid* g, int idim, int src, double dt, const RunCtl* ctl,
-                      RunCtl* nxt, bool cour) {
+// ghost values are left in buffer `state`, which holds the state between steps.
+static void enq_sweep(hydro_amd_grid* g, int idim, int src, int state, double dt,
+                      const RunCtl* ctl, RunCtl* nxt, bool cour) {
   uint64_t* c = cour ? g->cour : nullptr;
-  const int fill = folds_ghosts(g) ? (src == 0 ? 1 : 2) : -1;
+  const int fill = folds_ghosts(g) ? (src == state ? 1 : 2) : -1;
   if (fill < 0) enq_boundary(g, idim, src, ctl);
   timed(g, idim == 1 ? 0 : 1, [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
@@ -431,19 +443,55 @@ static void enq_sweep(hydro_amd_grid* g, int idim, int src, double dt, const Run
 static void enq_courant(hydro_amd_grid* g, const RunCtl* ctl) {
   timed(g, 3, [&] {
     if (dbl(g))  // (the FP64 fast form too: one launch per state, IEEE arithmetic)
-      launch_courant<double>(g->geom, g->ph, g->vd[0], g->cour, ctl, g->st);
+      launch_courant<double>(g->geom, g->ph, g->vd[g->cur], g->cour, ctl, g->st);
     else
-      launch_courant<float>(g->geom, g->ph, g->vf[0], g->cour, ctl, g->st);
+      launch_courant<float>(g->geom, g->ph, g->vf[g->cur], g->cour, ctl, g->st);
   });
 }
 
-// hydro_godunov.c:98-237: boundary + sweep for both directions, state back in
-// buffer 0.  `cour` folds the CFL maxima of the result into the second sweep.
-static void enq_godunov(hydro_amd_grid* g, int idim_start, double dt, const RunCtl* ctl,
-                        RunCtl* nxt, bool cour) {
+// Rows a workgroup of the whole-step kernel takes on this grid, or 0: the two
+// sweep kernels.  The whole step saves a launch and the y march's serial
+// solves and pays with halo cells, so it is for grids whose waves do not fill
+// the GPU; counted in its waves, the lines lie where the two were measured
+// alike.  A step, whole / two sweeps, blast (a flow that moves everywhere):
+// 250x125 FP64 20.8 / 23.5 us (17.8 / 21.8), fast 13.6 / 17.2, mixed 12.1 / 15.3;
+// 500x500 (9000 waves) FP64 35.8 / 41.1 (42.5 / 43.3), fast 24.8 / 27.1; 777x600
+// (15600) FP64 48.8 / 53.6 (58.6 / 57.4), fast 32.2 / 35.6; mixed with 16 rows
+// 500x500 18.3 / 21.5, 1021x767 (18400) 30.3 / 33.1, 1531x1200 (41600) 53.7 / 53.9.
+static int step_rows(const hydro_amd_grid* g) {
+  if (!folds_ghosts(g) || g->prof) return 0;  // (profiles are of the sweeps)
+  if (g->tune.step >= 0) return g->tune.step;
+  auto waves = [&](long rows) {
+    return ((g->p.nx + 59L) / 60) * ((g->p.ny + rows - 5) / (rows - 4)) * rows;
+  };
+  if (g->prec == HYDRO_AMD_FP64) return waves(8) <= 10000 ? 8 : 0;
+  if (g->prec == HYDRO_AMD_FP64_FAST) return waves(8) <= 16000 ? 8 : 0;
+  return waves(8) <= 5000 ? 8 : waves(16) <= 24000 ? 16 : 0;
+}
+
+// hydro_godunov.c:98-237: both directions, ghosts refilled before each, on the
+// state in buffer src; returns the buffer that the new state is in.  `cour`
+// folds the CFL maxima of the result into the second sweep.
+static int enq_godunov(hydro_amd_grid* g, int src, int idim_start, double dt, const RunCtl* ctl,
+                       RunCtl* nxt, bool cour) {
   const int d1 = idim_start == 1 ? 1 : 2, d2 = 3 - d1;
-  enq_sweep(g, d1, 0, dt, ctl, nxt, false);
-  enq_sweep(g, d2, 1, dt, ctl, nullptr, cour);
+  const int rows = d1 == 2 || !cour ? step_rows(g) : 0;  // (x first folds no maxima)
+  if (rows) {
+    uint64_t* c = cour ? g->cour : nullptr;
+    if (g->prec == HYDRO_AMD_FP64_FAST)
+      launch_step_fast(d1, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, nxt, c, rows,
+                       g->st);
+    else if (g->prec == HYDRO_AMD_FP64)
+      launch_step<double>(d1, g->geom, g->ph, g->vd[src], g->vd[1 - src], dt, ctl, nxt, c, rows,
+                          g->st);
+    else
+      launch_step<float>(d1, g->geom, g->ph, g->vf[src], g->vf[1 - src], dt, ctl, nxt, c, rows,
+                         g->st);
+    return 1 - src;
+  }
+  enq_sweep(g, d1, src, src, dt, ctl, nxt, false);
+  enq_sweep(g, d2, 1 - src, src, dt, ctl, nullptr, cour);
+  return src;
 }
 
 static void prepare_slots(hydro_amd_grid* g) {
@@ -454,8 +502,9 @@ static void prepare_slots(hydro_amd_grid* g) {
 
 static int godunov_impl(hydro_amd_grid* g, int idim, double dt, bool want_cour) {
   if (idim != 1 && idim != 2) return fail("idim must be 1 or 2 (got %d)", idim);
+  if (settle(g)) return -1;
   if (want_cour) prepare_slots(g);
-  enq_godunov(g, idim, dt, nullptr, nullptr, want_cour);
+  g->cur = enq_godunov(g, g->cur, idim, dt, nullptr, nullptr, want_cour);
   HIPCHK(hipGetLastError());
   bump(g);
   if (want_cour) {
@@ -477,7 +526,8 @@ extern "C" int hydro_amd_grid_godunov(hydro_amd_grid* g, int idim, double dt) {
 extern "C" int hydro_amd_grid_make_boundary(hydro_amd_grid* g, int idim) {
   if (!g) return fail("null grid");
   if (idim != 1 && idim != 2) return fail("idim must be 1 or 2 (got %d)", idim);
-  enq_boundary(g, idim, 0, nullptr);
+  if (settle(g)) return -1;
+  enq_boundary(g, idim, g->cur, nullptr);
   HIPCHK(hipGetLastError());
   return 0;
 }
@@ -492,6 +542,7 @@ static void ensure_cour(hydro_amd_grid* g) {
 
 extern "C" int hydro_amd_grid_compute_deltat(hydro_amd_grid* g, double* dt) {
   if (!g || !dt) return fail("null argument");
+  if (settle(g)) return -1;
   ensure_cour(g);
   // (straight into pinned memory: a copy would be a launch more)
   launch_dt_finalize(g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, &g->hctl->dt, g->st);
@@ -507,13 +558,13 @@ extern "C" int hydro_amd_grid_compute_deltat(hydro_amd_grid* g, double* dt) {
 
 // One step of main.c:244-298 with run control on the device; `n` is the step
 // number the host expects (its parity fixes the sweep order and the control).
-static void enq_step(hydro_amd_grid* g, int n) {
+// From the state in buffer src; returns the buffer of the new state.
+static int enq_step(hydro_amd_grid* g, int src, int n) {
   if (n % 2 == 0) {
     launch_ctl_begin(g->ctl, g->cour, g->p.courant_factor, g->p.dx, g->p.smallc, g->st);
-    enq_godunov(g, 1, 0.0, g->ctl, g->ctl + 1, false);
-  } else {
-    enq_godunov(g, 2, 0.0, g->ctl + 1, nullptr, true);
+    return enq_godunov(g, src, 1, 0.0, g->ctl, g->ctl + 1, false);
   }
+  return enq_godunov(g, src, 2, 0.0, g->ctl + 1, nullptr, true);
 }
 
 // The outcome of the queued steps (ctl[0]).
@@ -524,19 +575,19 @@ static int read_ctl(hydro_amd_grid* g, RunCtl* c) {
   return 0;
 }
 
-static int get_graph(hydro_amd_grid* g) {
-  // steps (even, odd) captured once; valid while the grid's buffers live
-  if (g->gexec) return 0;
+static int get_graph(hydro_amd_grid* g, int src) {
+  // steps (even, odd) captured once; valid while the grid's buffers live (two
+  // steps leave the state in the buffer that they found it in)
+  if (g->gexec[src]) return 0;
   hipGraph_t graph;
   HIPCHK(hipStreamBeginCapture(g->st, hipStreamCaptureModeThreadLocal));
-  enq_step(g, 0);
-  enq_step(g, 1);
+  enq_step(g, enq_step(g, src, 0), 1);
   hipError_t e = hipStreamEndCapture(g->st, &graph);
   if (e != hipSuccess) return fail("graph capture: %s", hipGetErrorString(e));
-  e = hipGraphInstantiate(&g->gexec, graph, nullptr, nullptr, 0);
+  e = hipGraphInstantiate(&g->gexec[src], graph, nullptr, nullptr, 0);
   (void) hipGraphDestroy(graph);
   if (e != hipSuccess) {
-    g->gexec = nullptr;
+    g->gexec[src] = nullptr;
     return fail("graph instantiate: %s", hipGetErrorString(e));
   }
   return 0;
@@ -549,6 +600,7 @@ static int run_finish(hydro_amd_grid* g, int* steps_done) {
   if (g->prof) prof_collect(g);
   const int done = c.nstep - g->nstep;
   if (done > 0) {
+    if (g->flips && done % 2 == 1) g->cur = 1 - g->cur;
     g->state_ver += done;
     // after an odd step the slots hold the maxima of the current state; after
     // an even one they were consumed by that step's dt
@@ -572,7 +624,7 @@ static int run_finish(hydro_amd_grid* g, int* steps_done) {
 static int run_enqueue(hydro_amd_grid* g, int max_steps, int log_cap,
                        hipEvent_t start = nullptr) {
   if (max_steps <= 0) return 0;
-  if (g->queued && run_finish(g, nullptr)) return -1;  // the step parity below is the mirror's
+  if (settle(g)) return -1;  // the step parity below is the mirror's
   // dt of an even step comes from the CFL maxima of the current state
   if (g->nstep % 2 == 0) ensure_cour(g);
   // control, log setup + limits
@@ -593,20 +645,21 @@ static int run_enqueue(hydro_amd_grid* g, int max_steps, int log_cap,
   // nothing rewrites the pinned copy before the next synchronising call
   HIPCHK(hipMemcpyAsync(g->ctl, g->hctl, 2 * sizeof(RunCtl), hipMemcpyHostToDevice, g->st));
   g->queued = true;
+  g->flips = step_rows(g) > 0;
   if (start) HIPCHK(hipEventRecord(start, g->st));
-  int n = g->nstep, left = max_steps;
+  int n = g->nstep, left = max_steps, src = g->cur;
   if (n % 2 == 1) {  // finish the odd step first so the graph starts even
-    enq_step(g, n);
+    src = enq_step(g, src, n);
     n++;
     left--;
   }
   if (left >= 2 && !g->prof) {
-    if (get_graph(g)) return -1;
-    for (; left >= 2; left -= 2, n += 2) HIPCHK(hipGraphLaunch(g->gexec, g->st));
+    if (get_graph(g, src)) return -1;
+    for (; left >= 2; left -= 2, n += 2) HIPCHK(hipGraphLaunch(g->gexec[src], g->st));
   }
-  for (; left >= 2; left--, n++) enq_step(g, n);
+  for (; left >= 2; left--, n++) src = enq_step(g, src, n);
   if (left == 1) {
-    enq_step(g, n);
+    src = enq_step(g, src, n);
     n++;
   }
   launch_ctl_end(g->ctl, n % 2 == 0, g->st);  // (n: the next step)
@@ -675,6 +728,7 @@ extern "C" int hydro_amd_grid_state(hydro_amd_grid* g, double* t, int* nstep, do
 extern "C" int hydro_amd_grid_set_state(hydro_amd_grid* g, double t, int nstep, double dt) {
   if (!g) return fail("null grid");
   if (nstep < 0) return fail("nstep < 0");
+  if (settle(g)) return -1;
   g->t = t;
   g->nstep = nstep;
   g->dt = dt;
@@ -683,6 +737,7 @@ extern "C" int hydro_amd_grid_set_state(hydro_amd_grid* g, double t, int nstep, 
 
 extern "C" int hydro_amd_grid_set_limits(hydro_amd_grid* g, double tend, int nstepmax) {
   if (!g) return fail("null grid");
+  if (settle(g)) return -1;
   g->p.tend = tend;
   g->p.nstepmax = nstepmax;
   return write_ctl(g);
@@ -713,9 +768,9 @@ extern "C" int hydro_amd_grid_profile(hydro_amd_grid* g, double* ms, long long* 
 
 // ---- autotuner ------------------------------------------------------------------------
 
-// Times one sweep launch shape: `reps` launches reading buffer 0 and writing
-// buffer 1's interior (buffer 0, the state, is untouched; buffer 1 is scratch
-// between steps), HIP events on the grid's stream.  Returns ms per launch.
+// Times one sweep launch shape: `reps` launches reading the state's buffer and
+// writing the other's interior (the state is untouched; the other buffer is
+// scratch between steps), HIP events on the grid's stream.  Returns ms per launch.
 // Average time of one sweep launch in direction idim with launch shape t
 // (reading the state, writing the scratch buffer); with cour non-null, the
 // variant that also folds the CFL maxima of its output into cour.
@@ -727,16 +782,16 @@ static double time_sweep(hydro_amd_grid* g, int idim, const SweepTune& t, int re
     (void) hipEventDestroy(a);
     return 1e30;
   }
-  const int fill = folds_ghosts(g) ? 0 : -1;
+  const int fill = folds_ghosts(g) ? 0 : -1, src = g->cur, dst = 1 - g->cur;
   auto launch = [&] {
     if (g->prec == HYDRO_AMD_FP64_FAST)
-      launch_sweep_fast(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, nullptr, cour, t,
+      launch_sweep_fast(idim, g->geom, g->ph, g->vd[src], g->vd[dst], 1e-12, nullptr, nullptr, cour, t,
                         fill, g->st);
     else if (g->prec == HYDRO_AMD_FP64)
-      launch_sweep<double>(idim, g->geom, g->ph, g->vd[0], g->vd[1], 1e-12, nullptr, nullptr, cour, t,
+      launch_sweep<double>(idim, g->geom, g->ph, g->vd[src], g->vd[dst], 1e-12, nullptr, nullptr, cour, t,
                            fill, g->st);
     else
-      launch_sweep<float>(idim, g->geom, g->ph, g->vf[0], g->vf[1], 1e-12, nullptr, nullptr, cour, t,
+      launch_sweep<float>(idim, g->geom, g->ph, g->vf[src], g->vf[dst], 1e-12, nullptr, nullptr, cour, t,
                           fill, g->st);
   };
   launch();  // warm
@@ -778,21 +833,22 @@ static SweepTune tune_by_steps(hydro_amd_grid* g, const std::vector<SweepTune>& 
     return fallback;
   }
   const double t0 = g->t, dt0 = g->dt;
-  const int n0 = g->nstep;
+  const int n0 = g->nstep, cur0 = g->cur;
   const bool slots_valid = g->cour_ver == g->state_ver;
   const bool dirty0 = g->cour_dirty;
-  bool ok = hipMemcpyAsync(save, g->mem[0], bytes, hipMemcpyDeviceToDevice, g->st) ==
+  bool ok = hipMemcpyAsync(save, g->mem[cur0], bytes, hipMemcpyDeviceToDevice, g->st) ==
                 hipSuccess &&
             hipMemcpyAsync(save + bytes, g->cour, slot_bytes, hipMemcpyDeviceToDevice, g->st) ==
                 hipSuccess;
   auto restore = [&] {
     ok = ok &&
-         hipMemcpyAsync(g->mem[0], save, bytes, hipMemcpyDeviceToDevice, g->st) == hipSuccess &&
+         hipMemcpyAsync(g->mem[cur0], save, bytes, hipMemcpyDeviceToDevice, g->st) == hipSuccess &&
          hipMemcpyAsync(g->cour, save + bytes, slot_bytes, hipMemcpyDeviceToDevice, g->st) ==
              hipSuccess;
     g->t = t0;
     g->nstep = n0;
     g->dt = dt0;
+    g->cur = cur0;
     bump(g);
     g->cour_ver = slots_valid ? g->state_ver : 0;
     g->cour_dirty = dirty0;
@@ -856,7 +912,10 @@ extern "C" int hydro_amd_grid_autotune(hydro_amd_grid* g, int reps, int* best) {
     }
   }
   HIPCHK(hipStreamSynchronize(g->st));
+  if (settle(g)) return -1;
   SweepTune cur = g->tune, bt = g->tune;
+  const int whole = step_rows(g);  // (tried against the sweeps where it is the default)
+  cur.step = bt.step = 0;
   // y sweep: rows per lane (the slab height each column march covers) x
   // waves per workgroup
   // Candidates are timed in two passes, in opposite orders, and scored by
@@ -919,6 +978,11 @@ extern "C" int hydro_amd_grid_autotune(hydro_amd_grid* g, int reps, int* best) {
       t.xiter = xs[xi].xiter;
       combos.push_back(t);
     }
+  if (whole) {
+    SweepTune t = combos[0];
+    t.step = whole;
+    combos.push_back(t);
+  }
   bt = tune_by_steps(g, combos, bt);
   HIPCHK(hipGetLastError());
   g->tune = bt;
@@ -944,6 +1008,7 @@ extern "C" int hydro_amd_grid_set_tune(hydro_amd_grid* g, int yseg, int ywaves, 
   g->tune.ywaves = ywaves;
   g->tune.xwaves = xwaves;
   g->tune.xiter = xiter;
+  g->tune.step = 0;
   drop_graph(g);
   return 0;
 }

@@ -127,6 +127,34 @@ __global__ __launch_bounds__(256) void k_sweep_y(GridGeom g, Phys<S> ph, double 
   if (COUR) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
 }
 
+// ---- whole step ----------------------------------------------------------------
+
+// Both sweeps of one tile per workgroup (tile_step), from one state buffer
+// into the other.
+template <typename S, bool ST1, bool XY, int W, int FD>
+__global__ __launch_bounds__(64 * W) void k_step(GridGeom g, Phys<S> ph, double dx,
+                                                 double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                                                 GridView<S> in, GridView<S> out, int bl, int br,
+                                                 int bd, int bu, uint64_t* cour, int nct) {
+  __shared__ TileLds<S, W> sh;
+  const int w = wave_id(), lane = threadIdx.x & 63;
+  // (the cells' loads are on their way before the control is read)
+  const TPlace<S> p = tile_load<S>(g, in, bl, br, bd, bu, 60 * (blockIdx.x % nct) + lane,
+                                   (W - 4) * (blockIdx.x / nct) + w);
+  double dt = dt_val;
+  if (ctl) {
+    open_odd_step(ctl, nxt);
+    if (!ctl->active) return;  // grid-uniform
+    dt = ctl->dt;
+  }
+  const double dtdx = dt / dx;
+  const TraceK<S> tk = make_tracek<S>((S) dtdx, ph.scheme);
+  double cx = 0.0, cy = 0.0;
+  // (odd steps, y first, fold the CFL maxima that the next step's dt needs)
+  tile_step<S, ST1, !XY, XY, W, FD>(g, ph, tk, dtdx, p, out, w, lane, sh, cx, cy);
+  if (!XY && cour) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
+}
+
 // ---- standalone CFL maximum -------------------------------------------------
 
 // CFL maxima over a thread's cells: a wave takes 64 columns of a row, the
@@ -139,7 +167,6 @@ __device__ __forceinline__ void courant_cells(const GridGeom& g, const Phys<S>& 
   const int i = (int) blockIdx.x * 64 + (threadIdx.x & 63);
   if (i >= g.nx) return;
   const int step = 4 * gridDim.y;
-#pragma unroll 2
   for (int j = (int) blockIdx.y * 4 + wave_id(); j < g.ny; j += step) {
     const long o = (j + 2L) * g.pitch + i + 2;
     S ax, ay;
@@ -383,6 +410,34 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
 #undef DISPATCH
 }
 
+// The whole-step launch for one arithmetic form (see launch_step).
+template <typename S, int FD>
+static void launch_step_fd(bool xy, const GridGeom& g, const Phys<S>& ph, const PhysArgs& pa,
+                           GridView<S> in, GridView<S> out, double dt_val, const RunCtl* ctl,
+                           RunCtl* nxt, uint64_t* cour, int waves, hipStream_t st) {
+  const bool st1 = pa.slope_type == 1.0;
+  const int nct = (int) cdiv(g.nx, 60);
+#define HS(A, B, W)                                                                              \
+  hipLaunchKernelGGL((k_step<S, A, B, W, FD>), dim3((unsigned) nct * cdiv(g.ny, W - 4)),         \
+                     dim3(64 * W), 0, st, g, ph, pa.dx, dt_val, ctl, nxt, in, out, pa.bl, pa.br, \
+                     pa.bd, pa.bu, cour, nct)
+#define HSW(A, B)                                             \
+  do {                                                        \
+    if constexpr (sizeof(S) == 4) {                           \
+      if (waves == 16) HS(A, B, 16); else HS(A, B, 8);        \
+    } else {                                                  \
+      HS(A, B, 8);                                            \
+    }                                                         \
+  } while (0)
+  if (st1) {
+    if (xy) HSW(true, true); else HSW(true, false);
+  } else {
+    if (xy) HSW(false, true); else HSW(false, false);
+  }
+#undef HSW
+#undef HS
+}
+
 // The ghosts of one sweep: formed by it (fill 0..2, see GhostFill::to), or in
 // memory already (fill < 0).
 static GhostFill ghost_fill(int idim, const PhysArgs& pa, int fill) {
@@ -410,8 +465,8 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
   if constexpr (sizeof(S) == 8) {
     const long ncb = cdiv(g.nx, 64);
     const long rows = tune.yseg > 0 ? 16 : y_rows(ncb, g.ny, 64);
-    const bool fd = ph.fastdiv && (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny
-                                             : ncb * cdiv(g.ny, rows)) >= kFastDivWaves;
+    const bool fd = ph.fastdiv && (idim == 1 ? (long) cdiv(g.nx, kXSeg) * g.ny >= kFastDivWaves
+                                             : ncb * cdiv(g.ny, rows) > kFastDivWaves);
     if (fd)
       launch_sweep_fd<S, kGated>(idim, g, ph, pa.dx, in, out, gf, dt_val, ctl, nxt, cour, tune,
                                  st1, st);
@@ -423,7 +478,25 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
                                  st1, st);
   }
 }
+
+template <typename S>
+void launch_step(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> in, GridView<S> out,
+                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int waves,
+                 hipStream_t st) {
+  const Phys<S> ph = make_phys<S>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type, pa.niter,
+                                  pa.iorder, pa.scheme);
+  // (FP64: the IEEE code, as in every launch that does not fill the SIMDs)
+  launch_step_fd<S, kIeee>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, waves, st);
+}
 #else
+void launch_step_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,
+                      GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                      uint64_t* cour, int waves, hipStream_t st) {
+  const Phys<double> ph = make_phys<double>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type,
+                                            pa.niter, pa.iorder, pa.scheme);
+  launch_step_fd<double, kFast>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, waves, st);
+}
+
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,
                        GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
                        uint64_t* cour, const SweepTune& tune, int fill, hipStream_t st) {
@@ -436,7 +509,7 @@ void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView
 
 // Workgroups of a CFL pass: 64 columns x 4 rows each, the rows strided over at
 // most about 2048 of them (8 waves a SIMD).
-static dim3 courant_grid(const GridGeom& g) {
+[[maybe_unused]] static dim3 courant_grid(const GridGeom& g) {
   const unsigned ncb = cdiv(g.nx, 64);
   const unsigned rows = cdiv(g.ny, 4), most = ncb < 2048 ? 2048 / ncb : 1;
   return dim3(ncb, rows < most ? rows : most);
@@ -489,12 +562,18 @@ template void launch_boundary<float>(int, const GridGeom&, const PhysArgs&, Grid
 template void launch_sweep<double>(int, const GridGeom&, const PhysArgs&, GridView<double>,
                                    GridView<double>, double, const RunCtl*, RunCtl*, uint64_t*,
                                    const SweepTune&, int, hipStream_t);
+template void launch_step<double>(int, const GridGeom&, const PhysArgs&, GridView<double>,
+                                  GridView<double>, double, const RunCtl*, RunCtl*, uint64_t*, int,
+                                  hipStream_t);
 template void launch_courant<double>(const GridGeom&, const PhysArgs&, GridView<double>,
                                      uint64_t*, const RunCtl*, hipStream_t);
 #elif defined(HYDRO_MIXED_UNIT)
 template void launch_sweep<float>(int, const GridGeom&, const PhysArgs&, GridView<float>,
                                   GridView<float>, double, const RunCtl*, RunCtl*, uint64_t*,
                                   const SweepTune&, int, hipStream_t);
+template void launch_step<float>(int, const GridGeom&, const PhysArgs&, GridView<float>,
+                                  GridView<float>, double, const RunCtl*, RunCtl*, uint64_t*, int,
+                                  hipStream_t);
 template void launch_courant<float>(const GridGeom&, const PhysArgs&, GridView<float>,
                                     uint64_t*, const RunCtl*, hipStream_t);
 #endif

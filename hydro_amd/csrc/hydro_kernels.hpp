@@ -68,6 +68,8 @@ struct SweepTune {
   int ywaves;   // waves per y-sweep workgroup (1..4)
   int xwaves;   // waves per x-sweep workgroup (1..4); 0: by the grid's size
   int xiter;    // row segments each x-sweep wave walks; 0: by the grid's size
+  int step;     // rows a workgroup of the whole-step kernel takes (8, 16); 0: the two
+                // sweep kernels; -1: by the grid's size
 };
 
 // ---- launchers (hydro_kernels.hip) -----------------------------------------
@@ -94,6 +96,19 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> i
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView<double> in,
                        GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
                        uint64_t* cour, const SweepTune& tune, int fill_ghosts, hipStream_t st);
+
+// Both sweeps of a step in one launch, x first (idim 1) or y first (idim 2,
+// which folds the CFL maxima when cour is non-null), from one state buffer
+// into the other with every ghost cell formed and stored; the rest as
+// launch_sweep.  waves: the rows a workgroup takes, 8 (mixed form: or 16).  For grids of at least
+// kGhostMin cells each way.
+template <typename S>
+void launch_step(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> in, GridView<S> out,
+                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int waves,
+                 hipStream_t st);
+void launch_step_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView<double> in,
+                      GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
+                      uint64_t* cour, int waves, hipStream_t st);
 
 template <typename S>
 void launch_courant(const GridGeom& g, const PhysArgs& ph, GridView<S> in, uint64_t* cour,

@@ -682,6 +682,195 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
   if (j <= j1 + 1) row(j);
 }
 
+// ---- whole step: both sweeps of a tile of the grid in one workgroup -----------
+
+// The W waves of a workgroup own W rows of 64 columns, one row a wave, and
+// take them through both sweeps; the middle (W - 4) x 60 cells come out
+// updated.  The x sweep of a row stays in its wave (lane rotations, as
+// x_segment), the y sweep exchanges between the waves through LDS, the state
+// between the two sweeps stays in registers.  A step is then one launch with
+// one Riemann solve of each direction in a row, where the two sweeps take two
+// launches of at least 4.3 us and the y march solves a segment's faces one
+// after the other.  The price is the halo: W / (W - 4) x 64 / 60 of the cells
+// are computed for each that is kept.  (One loop body for both directions, half
+// the code, was slower on every grid: 250x125 fast form 15.0 us a step against
+// 14.0, 500x500 30.3 against 26.5.)
+template <typename S, int W>
+struct TileLds {
+  // primitives, then fluxes (written after the barrier that follows the last
+  // read of the primitives); right-face states
+  S q[4][W][64], x[4][W][64];
+};
+
+template <typename S, int W>
+__device__ __forceinline__ void tile_put(S (&b)[4][W][64], int w, int lane, const Q4<S>& v) {
+  b[0][w][lane] = v.r;
+  b[1][w][lane] = v.u;
+  b[2][w][lane] = v.v;
+  b[3][w][lane] = v.p;
+}
+template <typename S, int W>
+__device__ __forceinline__ Q4<S> tile_get(const S (&b)[4][W][64], int w, int lane) {
+  return Q4<S>{b[0][w][lane], b[1][w][lane], b[2][w][lane], b[3][w][lane]};
+}
+
+// A cell of the tile: conserved values in grid slot order.
+template <typename S>
+struct TCell {
+  S r, mx, my, e;
+};
+
+// x sweep of one wave's row (the arithmetic of x_segment): lanes 2..61 return
+// their updated cell, the others something of no use.
+template <typename S, bool ST1, int FD>
+__device__ __forceinline__ TCell<S> tile_x(const Phys<S>& ph, const TraceK<S>& tk, double dtdx,
+                                           const TCell<S>& u) {
+  Prim<S> pc;
+  if constexpr (FD == kFast) pc = prim_fast(u.r, u.mx, u.my, u.e, ph);
+  else pc = prim_cell<S, false>(u.r, u.mx, u.my, u.e, ph);
+  Q4<S> dq = {(S) 0, (S) 0, (S) 0, (S) 0};
+  if (ph.iorder != 1) {
+    const Q4<S> qm = from_left4(pc.q), qp = from_right4(pc.q);
+    dq = slope_form<S, ST1, FD>(qm, pc.q, qp, ph);
+  }
+  Q4<S> qxm, qxp;
+  if constexpr (FD == kFast || sizeof(S) == 4)
+    trace_fast(pc.q, dq, pc.c, pc.cinv, pc.rinv, tk, qxm, qxp);
+  else trace_cell<S>(pc.q, dq, pc.c, tk, qxm, qxp);
+  const Q4<S> qr = from_right4(qxp);
+  const Q4<double> fr = to_d4(riemann_flux<S, FD>(qxm, qr, ph));
+  const Q4<double> fl = from_left4(fr);
+  return TCell<S>{(S) update1<S>(u.r, fl.r, fr.r, dtdx), (S) update1<S>(u.mx, fl.u, fr.u, dtdx),
+                  (S) update1<S>(u.my, fl.v, fr.v, dtdx), (S) update1<S>(u.e, fl.p, fr.p, dtdx)};
+}
+
+// y sweep across the workgroup's rows: waves 2..W-3 return their updated
+// cells, the others something of no use.  Every thread calls it (barriers).
+// A wave does only what a kept row needs of it.
+template <typename S, bool ST1, int W, int FD>
+__device__ __forceinline__ TCell<S> tile_y(const Phys<S>& ph, const TraceK<S>& tk, double dtdx,
+                                           const TCell<S>& u, int w, int lane,
+                                           TileLds<S, W>& sh) {
+  // slots with IU and IV swapped (conservar.c:106-109)
+  Prim<S> pc;
+  if constexpr (FD == kFast) pc = prim_fast(u.r, u.my, u.mx, u.e, ph);
+  else pc = prim_cell<S, false>(u.r, u.my, u.mx, u.e, ph);
+  tile_put<S, W>(sh.q, w, lane, pc.q);
+  __syncthreads();
+  Q4<S> qxm, qxp;
+  if (w >= 1 && w <= W - 2) {  // wave-uniform, as the tests on w below
+    Q4<S> dq = {(S) 0, (S) 0, (S) 0, (S) 0};
+    if (ph.iorder != 1)
+      dq = slope_form<S, ST1, FD>(tile_get<S, W>(sh.q, w - 1, lane), pc.q,
+                                  tile_get<S, W>(sh.q, w + 1, lane), ph);
+    if constexpr (FD == kFast || sizeof(S) == 4)
+      trace_fast(pc.q, dq, pc.c, pc.cinv, pc.rinv, tk, qxm, qxp);
+    else trace_cell<S>(pc.q, dq, pc.c, tk, qxm, qxp);
+    tile_put<S, W>(sh.x, w, lane, qxp);
+  }
+  __syncthreads();
+  Q4<S> fr;
+  if (w >= 1 && w <= W - 3) {
+    fr = riemann_flux<S, FD>(qxm, tile_get<S, W>(sh.x, w + 1, lane), ph);
+    tile_put<S, W>(sh.q, w, lane, fr);
+  }
+  __syncthreads();
+  TCell<S> n = u;
+  if (w >= 2 && w <= W - 3) {
+    const Q4<double> l = to_d4(tile_get<S, W>(sh.q, w - 1, lane)), r = to_d4(fr);
+    n.r = (S) update1<S>(u.r, l.r, r.r, dtdx);
+    n.my = (S) update1<S>(u.my, l.u, r.u, dtdx);
+    n.mx = (S) update1<S>(u.mx, l.v, r.v, dtdx);
+    n.e = (S) update1<S>(u.e, l.p, r.p, dtdx);
+  }
+  return n;
+}
+
+template <typename S>
+__device__ __forceinline__ void tile_store(const GridView<S>& out, long o, const TCell<S>& v) {
+  out.p[0][o] = v.r;
+  out.p[1][o] = v.mx;
+  out.p[2][o] = v.my;
+  out.p[3][o] = v.e;
+}
+
+// One thread's place in the grid and its cell as loaded: ghosts from their
+// source cells, before any change of sign.
+template <typename S>
+struct TPlace {
+  int i, j;         // padded column and row (may lie past the grid)
+  bool gx, gy;      // a ghost column / row of the grid, to be written
+  bool rawx, rawy;  // its source is itself a ghost: not swept in the other direction
+  bool negx, negy;  // reflected
+  TCell<S> u;
+};
+template <typename S>
+__device__ __forceinline__ TPlace<S> tile_load(const GridGeom& g, const GridView<S>& in, int bl,
+                                               int br, int bd, int bu, int i, int j) {
+  TPlace<S> p;
+  p.i = i;
+  p.j = j;
+  p.negx = p.negy = p.rawx = p.rawy = p.gx = p.gy = false;
+  const int ic = i < g.nx + 4 ? i : g.nx + 3, jc = j < g.ny + 4 ? j : g.ny + 3;
+  int is = ic, js = jc;
+  if (ic < 2 || ic >= g.nx + 2) {
+    is = ghost_source(1, g.nx, bl, br, ic, p.negx);
+    p.rawx = is < 2 || is >= g.nx + 2;
+    p.gx = is != i && i == ic;
+  }
+  if (jc < 2 || jc >= g.ny + 2) {
+    js = ghost_source(2, g.ny, bd, bu, jc, p.negy);
+    p.rawy = js < 2 || js >= g.ny + 2;
+    p.gy = js != j && j == jc;
+  }
+  const long o = (long) js * g.pitch + is;
+  p.u = TCell<S>{in.p[0][o], in.p[1][o], in.p[2][o], in.p[3][o]};
+  return p;
+}
+
+// The step of one tile from its loaded cells; XY: the x sweep first (even
+// steps).  Ghost cells: those of the first direction hold values of the state
+// before the step, those of the second values of the state between the sweeps
+// (make_boundary before each, hydro_godunov.c:98-110), so a ghost line of the
+// second direction is swept in the first like its source line, unless the
+// source is itself a ghost.
+template <typename S, bool ST1, bool COUR, bool XY, int W, int FD>
+__device__ __forceinline__ void tile_step(const GridGeom& g, const Phys<S>& ph,
+                                          const TraceK<S>& tk, double dtdx, TPlace<S> p,
+                                          const GridView<S>& out, int w, int lane,
+                                          TileLds<S, W>& sh, double& cx, double& cy) {
+  const bool midx = lane >= 2 && lane <= 61, midy = w >= 2 && w <= W - 3;
+  const bool inx = p.i >= 2 && p.i <= g.nx + 1, iny = p.j >= 2 && p.j <= g.ny + 1;
+  const long o = (long) p.j * g.pitch + p.i;
+  TCell<S> u = p.u, v;
+  if constexpr (XY) {
+    if (p.negx) u.mx = -u.mx;
+    if (p.gx && midy && iny) tile_store(out, o, u);
+    v = tile_x<S, ST1, FD>(ph, tk, dtdx, u);
+    if (p.rawy) v = u;
+    if (p.negy) v.my = -v.my;
+    if (p.gy && midx && inx) tile_store(out, o, v);
+    v = tile_y<S, ST1, W, FD>(ph, tk, dtdx, v, w, lane, sh);
+  } else {
+    if (p.negy) u.my = -u.my;
+    if (p.gy && midx && inx) tile_store(out, o, u);
+    v = tile_y<S, ST1, W, FD>(ph, tk, dtdx, u, w, lane, sh);
+    if (p.rawx) v = u;
+    if (p.negx) v.mx = -v.mx;
+    if (p.gx && midy && iny) tile_store(out, o, v);
+    if (midy) v = tile_x<S, ST1, FD>(ph, tk, dtdx, v);  // wave-uniform
+  }
+  if (midx && midy && inx && iny) {
+    tile_store(out, o, v);
+    if (COUR) {
+      S ax, ay;
+      courant_cell<S, FD>(v.r, v.mx, v.my, v.e, ph, ax, ay);
+      cx = maxm(cx, (double) ax);
+      cy = maxm(cy, (double) ay);
+    }
+  }
+}
+
 // ---- ghost cells -------------------------------------------------------------
 
 // make_boundary.c:237-289 (x) and 381-433 (y) for one interior line k and one
