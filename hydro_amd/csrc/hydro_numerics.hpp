@@ -598,6 +598,43 @@ __device__ __forceinline__ void trace_tail(const Q4<R>& q, const Q4<R>& dq, R cc
   }
 }
 
+// trace_tail with its factors of one half taken out of the products: for cells
+// whose own and neighbour values passed cell_in, where no product comes near
+// under- or overflow (velocities, densities and pressures are zero or at least
+// 2^-81, so slopes are zero or at least 2^-134; spm, spp and sp0 are zero or at
+// least 2^-53), a power of two commutes with every rounding.  -half * spp * ap
+// is -(1/4) * (spp * (dprcc + du) * rOcc) and so on, azr and azv have -(1/2), and
+// the last sum of each state takes the factor in a multiply-add whose product
+// is exact: ten multiplications fewer, the same bits.
+template <typename R>
+__device__ __forceinline__ void trace_tail_scaled(const Q4<R>& q, const Q4<R>& dq, R cc, R csq,
+                                                  R rOcc, R OrOcc, R dprcc, R a0r,
+                                                  const TraceK<R>& k, Q4<R>& qxm, Q4<R>& qxp) {
+  const R one = (R) 1, q4 = (R) -0.25, q2 = (R) -0.5;
+  const R am = (dprcc - dq.u) * rOcc;  // 2 am
+  const R ap = (dprcc + dq.u) * rOcc;  // 2 ap
+  const R upcc = q.u + cc, umcc = q.u - cc;
+  R spmR = umcc * k.dtdx + one, sppR = upcc * k.dtdx + one, sp0R = q.u * k.dtdx + one;
+  R spmL = umcc * k.dtdx - one, sppL = upcc * k.dtdx - one, sp0L = q.u * k.dtdx - one;
+  if (!wave_all(upcc < k.zeror && umcc > k.zerol)) {  // as in trace_tail
+    spmR = (umcc >= k.zeror) ? k.project : spmR;
+    sppR = (upcc >= k.zeror) ? k.project : sppR;
+    sp0R = (q.u >= k.zeror) ? k.project : sp0R;
+    spmL = (umcc <= k.zerol) ? -k.project : spmL;
+    sppL = (upcc <= k.zerol) ? -k.project : sppL;
+    sp0L = (q.u <= k.zerol) ? -k.project : sp0L;
+  }
+  auto face = [&](R spm, R spp, R sp0, Q4<R>& x) {
+    const R p = spp * ap, m = spm * am, s = p + m;  // -4 apr, -4 amr
+    x.r = __builtin_fma(q4, __builtin_fma((R) 2, sp0 * a0r, s), q.r);
+    x.u = __builtin_fma(q4, (p - m) * OrOcc, q.u);
+    x.v = __builtin_fma(q2, sp0 * dq.v, q.v);
+    x.p = __builtin_fma(q4, s * csq, q.p);
+  };
+  face(spmR, sppR, sp0R, qxp);
+  face(spmL, sppL, sp0L, qxm);
+}
+
 // trace.c:85-147 for one cell in the FP64 form (quotients as the form
 // computes them, then trace_tail; the fast and mixed forms take trace_fast).
 // FAST: FastDiv, for cells whose own and neighbour values (the slope inputs)
@@ -616,7 +653,8 @@ __device__ __forceinline__ void trace_cell(const Q4<R>& q, const Q4<R>& dq, R cc
   else OrOcc = P::divn(cc, q.r);
   const R dprcc = P::div(dq.p, q.r * cc);
   const R a0r = dq.r - P::div(dq.p, csq);
-  trace_tail<R>(q, dq, cc, csq, rOcc, OrOcc, dprcc, a0r, k, qxm, qxp);
+  if constexpr (FAST) trace_tail_scaled<R>(q, dq, cc, csq, rOcc, OrOcc, dprcc, a0r, k, qxm, qxp);
+  else trace_tail<R>(q, dq, cc, csq, rOcc, OrOcc, dprcc, a0r, k, qxm, qxp);
 }
 
 // ---- FP64 Riemann solver (the FP64 form) ------------------------------------
@@ -636,16 +674,35 @@ __device__ __forceinline__ bool newton_step(double& pst, double pl, double pr, d
   P::sqrt2(cl * (1.0 + P::qn(g6 * (pst - pl), rpl)), cr * (1.0 + P::qn(g6 * (pst - pr), rpr)),
            wwl, wwr);
   const double swwl = wwl * wwl;
-  const double qlw = P::divn(2.0 * wwl * swwl, swwl + cl);
-  const double qrw = P::divn(2.0 * wwr * (wwr * wwr), (wwr * wwr) + cr);
-  const double usl = ul - P::divn(pst - pl, wwl);
-  const double usr = ur + P::divn(pst - pr, wwr);
-  const double t = (P::divn(qrw * qlw, qrw + qlw) * (usl - usr));
-  const double d = (t > (-pst)) ? t : (-pst);
-  pst += d;
-  const double rel = P::divn(d, pst + smallpp);
-  const double arel = (rel > 0) ? rel : -rel;
-  return !(arel > 1e-6);
+  if constexpr (std::is_same_v<P, FastDiv>) {
+    // The same values with fewer operations.  q_l / 2 and q_r / 2 stand for q_l
+    // and q_r (the factors 2.0 and the halved quotient are powers of two, every
+    // operand far from over- and underflow).  pst is no NaN here, so the
+    // clamp is a maximum (where it returns the other zero, pst += d and the
+    // test below do not see it).
+    const double hl = P::divn(wwl * swwl, swwl + cl);
+    const double hr = P::divn(wwr * (wwr * wwr), (wwr * wwr) + cr);
+    const double usl = ul - P::divn(pst - pl, wwl);
+    const double usr = ur + P::divn(pst - pr, wwr);
+    const double h = P::divn(hr * hl, hr + hl) * (usl - usr);
+    const double d = fmax(2.0 * h, -pst);
+    pst += d;
+    // |d / (pst + smallpp)| > 1e-6 from products, whose error is 2^-13 of the
+    // margin; a wave with a lane inside the margin divides.
+    const double s = pst + smallpp, a = fabs(d);
+    const bool over = a > s * (1e-6 * (1.0 + 0x1p-40));
+    if (wave_all(over || a < s * (1e-6 * (1.0 - 0x1p-40)))) return !over;
+    return !(P::divn(a, s) > 1e-6);
+  } else {
+    const double qlw = P::divn(2.0 * wwl * swwl, swwl + cl);
+    const double qrw = P::divn(2.0 * wwr * (wwr * wwr), (wwr * wwr) + cr);
+    const double usl = ul - P::divn(pst - pl, wwl);
+    const double usr = ur + P::divn(pst - pr, wwr);
+    const double t = (P::divn(qrw * qlw, qrw + qlw) * (usl - usr));
+    const double d = (t > (-pst)) ? t : (-pst);
+    pst += d;
+    return !(fabs(P::divn(d, pst + smallpp)) > 1e-6);
+  }
 }
 
 // Star state, sampling at x/t = 0 and flux (riemann.c:211-276, cmpflx.c:67-90)
@@ -691,7 +748,7 @@ __device__ __forceinline__ Q4<double> star_flux(double pst, const Q4<double>& ql
   co = fmax(ph.smallc, co);
   cstar = fmax(ph.smallc, cstar);
   double spout = co - sg * uo;
-  double spin = cstar - sg * ustar;
+  double spin = cstar - fabs(ustar);  // (sg * ustar, but for a zero's sign)
   const double ushock = P::qn(wo, rro) - sg * uo;
   if (ps >= po) {
     spin = ushock;
