@@ -6,8 +6,10 @@
 // the stream-ordered allocator (hipMallocAsync / hipFreeAsync on the batch's
 // stream), so admitting or retiring an instance never synchronises the
 // device.  The per-step work is two phase task tables (P and Q) built from
-// each instance's step parity; two steps (P,Q then Q,P) are captured once as a
-// HIP graph and replayed until the set of instances changes.
+// each instance's step parity, for each of two groups of the instances, which
+// run beside each other on streams of their own; a small load is one group, whose
+// two steps (P,Q then Q,P) are captured once as a HIP graph and replayed until the
+// set of instances changes.
 #include <hip/hip_runtime.h>
 
 #include <stdarg.h>
@@ -35,6 +37,8 @@ extern "C" int hydro_amd_set_error(const char* fmt, ...);  // hydro_capi.cpp
 namespace {
 constexpr long kOrigin = 30;  // same row origin as single grids (hydro_capi.cpp)
 constexpr int kMaxInst = 8192;
+constexpr int kGroups = 2;        // instances advanced side by side (split_load)
+constexpr long kSplitSegs = 4000;  // least x segments of a load in two groups
 
 struct Inst {
   bool live = false;
@@ -44,6 +48,16 @@ struct Inst {
   void* mem[2] = {nullptr, nullptr};
   long long bytes = 0;
   bool need_cour = false;  // CFL maxima of the initial state still to compute
+};
+
+// Instances that are advanced together, launch by launch, on one stream.
+struct Group {
+  // task lists, in this order: Px Py (phase P: x of even-step instances, y of
+  // odd ones), Qx Qy (phase Q: the other sweep of each), PB QB (ghost fills)
+  int n[6] = {0, 0, 0, 0, 0, 0};
+  int off[6] = {0, 0, 0, 0, 0, 0};
+  int n1[6] = {0, 0, 0, 0, 0, 0};  // leading tasks of slope_type == 1 instances
+  int first = 0, nids = 0;         // its part of the live ids
 };
 }  // namespace
 
@@ -56,15 +70,14 @@ struct hydro_amd_batch {
   RunCtl* ctl = nullptr;         // kMaxInst run controls
   uint64_t* cour = nullptr;      // kMaxInst * 2 * kInstSlots
   void* idev = nullptr;          // InstDev<S>[kMaxInst]
-  // task lists, in this order: Px Py (phase P: x of even-step instances, y of
-  // odd ones), Qx Qy (phase Q: the other sweep of each), PB QB (ghost fills)
-  BTask* tasks = nullptr;
+  BTask* tasks = nullptr;        // the groups' task lists
   int task_cap = 0;
   int* ids = nullptr;            // live ids (device)
   int* cids = nullptr;           // ids needing a CFL pass (device)
-  int n[6] = {0, 0, 0, 0, 0, 0}; // Px Py Qx Qy PB QB
-  int off[6] = {0, 0, 0, 0, 0, 0};
-  int n1[6] = {0, 0, 0, 0, 0, 0};  // leading tasks of slope_type == 1 instances
+  Group grp[kGroups];
+  int ngrp = 1;
+  hipStream_t st2 = nullptr;     // group 1's (group 0: st); made when first needed
+  hipEvent_t fork = nullptr, join = nullptr;
   BList* lists = nullptr;          // what the task tables are written from (device)
   int nids = 0;
   int maxid = -1;                // highest live id
@@ -92,6 +105,7 @@ static void drop_graphs(hydro_amd_batch* b) {
 extern "C" void hydro_amd_batch_destroy(hydro_amd_batch* b) {
   if (!b) return;
   if (b->st) (void) hipStreamSynchronize(b->st);
+  if (b->st2) (void) hipStreamSynchronize(b->st2);
   drop_graphs(b);
   for (auto& in : b->inst)
     for (auto& m : in.mem)
@@ -102,6 +116,9 @@ extern "C" void hydro_amd_batch_destroy(hydro_amd_batch* b) {
   if (b->hctl) (void) hipHostFree(b->hctl);
   if (b->hidev) (void) hipHostFree(b->hidev);
   if (b->st) (void) hipStreamDestroy(b->st);
+  if (b->st2) (void) hipStreamDestroy(b->st2);
+  for (auto e : {b->fork, b->join})
+    if (e) (void) hipEventDestroy(e);
   delete b;
 }
 
@@ -373,28 +390,33 @@ extern "C" int hydro_amd_batch_upload(hydro_amd_batch* b, int id, const double* 
 
 // ---- task tables -------------------------------------------------------------------
 
+static long x_segments(const hydro_amd_params& p) {
+  return (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+}
+
 // Task shape by the load.  As in a single grid's y sweep (y_rows,
 // hydro_kernels.hip), a task's fixed cost and the unevenness that long tasks
 // leave at a launch's end balance at a length proportional to the square root
-// of the work: sqrt(wave rows) / 32 rows, sqrt(segments) / 100 segments.  The
-// best of all shapes tried, x segments / y rows: 12 grids of 64-256 a side
-// 2 / 2; 30 of 150-500 2-4 / 8; 60 of 64-1024 4-8 / 12; 300 of 64-1024 8 / 32;
-// 24 of 128-4096 8-16 / 24-32.  A step took with the fixed shapes before (2
-// or 4 waves of 8 or 32 segments, 32 or 64 rows) and takes with these: 12 small
-// grids, mixed, 138 and 28 us; 30, fast, 156 and 113; 60, FP64, 701 and 650;
-// 24 of up to 4096, mixed, 1.21 and 1.16 ms.
+// of the work: sqrt(wave rows) / 28 rows, sqrt(segments) / 50 segments (with
+// one chain of launches, before split_load, half the segments).  The best of
+// all shapes tried, x segments / y rows: 4 grids of 64-100 a side 1 / 1; 12 of
+// 64-256 1 / 2-3; 2 of 900-1024 3-4 / 4; 30 of 150-500 4 / 6-8; 60 of 64-1024
+// 8-12 / 16-24; 300 of 64-1024 and 24 of 128-4096 8-32 / 32-64.  A step took
+// with fixed shapes (2 or 4 waves of 8 or 32 segments, 32 or 64 rows) in one
+// chain and takes with these: 12 small grids, mixed, 138 and 24 us; 30, fast,
+// 156 and 94; 60, FP64, 701 and 565; 24 of up to 4096, mixed, 1.21 and 1.12 ms.
 static void shape_by_load(hydro_amd_batch* b) {
   long segs = 0, wrows = 0;
   for (int id : b->live_ids) {
     const hydro_amd_params& p = b->inst[id].p;
-    segs += (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+    segs += x_segments(p);
     wrows += (long) ((p.nx + 63) / 64) * p.ny;
   }
   auto root = [](long n, double by, int most) {
     return std::max(1, std::min(most, (int) (std::sqrt((double) n) / by + 0.5)));
   };
-  b->xiter = b->tune.xiter > 0 ? b->tune.xiter : root(segs, 100, 32);
-  b->yseg = b->tune.yseg > 0 ? b->tune.yseg : root(wrows, 32, 32);
+  b->xiter = b->tune.xiter > 0 ? b->tune.xiter : root(segs, 50, 16);
+  b->yseg = b->tune.yseg > 0 ? b->tune.yseg : root(wrows, 28, 40);
 }
 
 // Rows per wave in an instance's y tasks: the instance's rows split evenly
@@ -441,7 +463,7 @@ static BList sweep_tasks(const hydro_amd_batch* b, int id, int kind) {
   const long W = b->tune.waves;
   BList l{id, kind, 0, 0, 0, 0};
   if (kind == 1) {
-    const long per = W * b->xiter, tot = (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+    const long per = W * b->xiter, tot = x_segments(p);
     l.per = (int) per;
     l.count = (int) ((tot + per - 1) / per);
   } else {
@@ -469,6 +491,46 @@ static int read_ctl(hydro_amd_batch* b) {
   return 0;
 }
 
+// Parts a load into two groups of about the same work, each with a
+// stream of its own: an instance waits only for its own sweeps, so where one
+// group's launch runs out of tasks the other's fills the GPU (alone, the y
+// sweeps of 60 grids of 64-1024 a side kept 3.05 of 4 waves a SIMD busy and
+// issued 75 % of the time; the x sweeps 4.35 of 5, 89 %), and longer tasks pay.  A
+// step, one group and two, each at its best shape: 12 grids of 64-256, mixed, 30
+// and 24 us; 30 of 150-500, fast, 115 and 94; 60 of 64-1024, FP64 640 and 558,
+// fast 400 and 373, mixed 238 and 218; 24 of 128-4096, mixed, 1146 and 1117.
+// Three groups: the same within 1 %.  Below kSplitSegs the ten launches of a
+// step of two groups are what the step costs (17-19 us on the host): 4 grids of
+// 64-100 a side, 625 segments, mixed, 13.2 us as one group's graph and 18.6; 12
+// of 64-256, 5500 segments, 20.9 and 18.9, FP64 38.0 and 29.4.
+static int split_load(hydro_amd_batch* b) {
+  auto work = [&](int id) { return (long) b->inst[id].p.nx * b->inst[id].p.ny; };
+  for (auto& gr : b->grp) gr = Group();
+  b->grp[0].nids = (int) b->live_ids.size();
+  long segs = 0;
+  for (int id : b->live_ids) segs += x_segments(b->inst[id].p);
+  b->ngrp = b->grp[0].nids > 1 && segs >= kSplitSegs ? 2 : 1;
+  if (b->ngrp == 1) return 0;
+  if (!b->st2) BCHK(hipStreamCreateWithFlags(&b->st2, hipStreamNonBlocking));
+  if (!b->fork) BCHK(hipEventCreateWithFlags(&b->fork, hipEventDisableTiming));
+  if (!b->join) BCHK(hipEventCreateWithFlags(&b->join, hipEventDisableTiming));
+  // the largest first, each to the group with the least so far
+  std::stable_sort(b->live_ids.begin(), b->live_ids.end(),
+                   [&](int x, int y) { return work(x) > work(y); });
+  std::vector<int> part[kGroups];
+  long sum[kGroups] = {0, 0};
+  for (int id : b->live_ids) {
+    const int q = sum[1] < sum[0] ? 1 : 0;
+    part[q].push_back(id);
+    sum[q] += work(id);
+  }
+  b->live_ids = part[0];
+  b->live_ids.insert(b->live_ids.end(), part[1].begin(), part[1].end());
+  b->grp[0].nids = b->grp[1].first = (int) part[0].size();
+  b->grp[1].nids = (int) part[1].size();
+  return 0;
+}
+
 // Rebuilds the device instance array and the phase tables from the current
 // live set and their step parities (the stream must be idle).
 static int rebuild(hydro_amd_batch* b) {
@@ -482,32 +544,37 @@ static int rebuild(hydro_amd_batch* b) {
     }
   if (read_ctl(b)) return -1;
   shape_by_load(b);
-  // each sweep list: tasks of slope_type == 1 instances first (their own
-  // kernel variant), then the others
-  std::vector<BList> L[6][2];
-  for (int id : b->live_ids) {
-    const bool even = (b->hctl[id].nstep % 2) == 0;
-    const int gen = b->inst[id].p.slope_type == 1.0 ? 0 : 1;
-    L[even ? 0 : 2][gen].push_back(sweep_tasks(b, id, 1));
-    L[even ? 3 : 1][gen].push_back(sweep_tasks(b, id, 2));
-    if (!folds_ghosts(b->inst[id])) {
-      L[4][0].push_back(ghost_tasks(b, id, even ? 1 : 2));
-      L[5][0].push_back(ghost_tasks(b, id, even ? 2 : 1));
-    }
-  }
+  if (split_load(b)) return -1;
   std::vector<BList> all;
   long need = 0;
-  for (int k = 0; k < 6; k++) {
-    b->off[k] = (int) need;
-    for (auto& part : L[k]) {
-      for (BList& l : part) {
-        l.first = (int) need;
-        need += l.count;
-        all.push_back(l);
+  for (int q = 0; q < b->ngrp; q++) {
+    Group& gr = b->grp[q];
+    // each sweep list: tasks of slope_type == 1 instances first (their own
+    // kernel variant), then the others
+    std::vector<BList> L[6][2];
+    for (int m = gr.first; m < gr.first + gr.nids; m++) {
+      const int id = b->live_ids[m];
+      const bool even = (b->hctl[id].nstep % 2) == 0;
+      const int gen = b->inst[id].p.slope_type == 1.0 ? 0 : 1;
+      L[even ? 0 : 2][gen].push_back(sweep_tasks(b, id, 1));
+      L[even ? 3 : 1][gen].push_back(sweep_tasks(b, id, 2));
+      if (!folds_ghosts(b->inst[id])) {
+        L[4][0].push_back(ghost_tasks(b, id, even ? 1 : 2));
+        L[5][0].push_back(ghost_tasks(b, id, even ? 2 : 1));
       }
-      if (&part == &L[k][0]) b->n1[k] = (int) (need - b->off[k]);
     }
-    b->n[k] = (int) (need - b->off[k]);
+    for (int k = 0; k < 6; k++) {
+      gr.off[k] = (int) need;
+      for (auto& part : L[k]) {
+        for (BList& l : part) {
+          l.first = (int) need;
+          need += l.count;
+          all.push_back(l);
+        }
+        if (&part == &L[k][0]) gr.n1[k] = (int) (need - gr.off[k]);
+      }
+      gr.n[k] = (int) (need - gr.off[k]);
+    }
   }
   if (need > (1L << 30)) return hydro_amd_set_error("batch too large: %ld tasks", need);
   b->nids = (int) b->live_ids.size();
@@ -543,52 +610,75 @@ static int rebuild(hydro_amd_batch* b) {
   return 0;
 }
 
-// The sweeps of task list k (kind 1: x, 2: y) in the batch's arithmetic form,
-// reading buffer `phase`.
+static hipStream_t stream_of(const hydro_amd_batch* b, int q) { return q == 0 ? b->st : b->st2; }
+
+// The sweeps of group q's task list k (kind 1: x, 2: y) in the batch's
+// arithmetic form, reading buffer `phase`.
 template <typename S>
-static void sweep_list(hydro_amd_batch* b, int kind, const InstDev<S>* I, int k, int phase,
-                       bool ghosts) {
+static void sweep_list(hydro_amd_batch* b, int q, int kind, int k, int phase, bool ghosts) {
+  const InstDev<S>* I = (const InstDev<S>*) b->idev;
+  const Group& gr = b->grp[q];
   if constexpr (sizeof(S) == 8) {
     if (b->prec == HYDRO_AMD_FP64_FAST) {
-      launch_batch_sweep_fast(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
-                              b->tune.waves, b->xiter, b->st);
+      launch_batch_sweep_fast(kind, I, b->tasks + gr.off[k], gr.n[k], gr.n1[k], phase, ghosts,
+                              b->tune.waves, b->xiter, stream_of(b, q));
       return;
     }
   }
-  launch_batch_sweep<S>(kind, I, b->tasks + b->off[k], b->n[k], b->n1[k], phase, ghosts,
-                        b->tune.waves, b->xiter, b->st);
+  launch_batch_sweep<S>(kind, I, b->tasks + gr.off[k], gr.n[k], gr.n1[k], phase, ghosts,
+                        b->tune.waves, b->xiter, stream_of(b, q));
 }
 
-// One phase: the ghost fills of its narrow instances, then its x tasks and its
-// y tasks.
+// One phase of a group: the ghost fills of its narrow instances, then its x
+// tasks and its y tasks.
 template <typename S>
-static void enq_phase(hydro_amd_batch* b, int which, int phase) {
-  const InstDev<S>* I = (const InstDev<S>*) b->idev;
+static void enq_phase(hydro_amd_batch* b, int q, int which, int phase) {
   const int x = which == 0 ? 0 : 2, y = x + 1, bd = which == 0 ? 4 : 5;
-  launch_batch_boundary<S>(I, b->tasks + b->off[bd], b->n[bd], phase, b->st);
-  sweep_list<S>(b, 1, I, x, phase, true);
-  sweep_list<S>(b, 2, I, y, phase, true);
+  launch_batch_boundary<S>((const InstDev<S>*) b->idev, b->tasks + b->grp[q].off[bd],
+                           b->grp[q].n[bd], phase, stream_of(b, q));
+  sweep_list<S>(b, q, 1, x, phase, true);
+  sweep_list<S>(b, q, 2, y, phase, true);
 }
 
 template <typename S>
-static void enq_step_t(hydro_amd_batch* b, bool flip) {
-  const InstDev<S>* I = (const InstDev<S>*) b->idev;
-  launch_batch_ctl<S>(I, b->ids, b->nids, true, b->st);
-  enq_phase<S>(b, flip ? 1 : 0, 0);
-  enq_phase<S>(b, flip ? 0 : 1, 1);
+static void enq_ctl(hydro_amd_batch* b, int q, bool begin) {
+  launch_batch_ctl<S>((const InstDev<S>*) b->idev, b->ids + b->grp[q].first, b->grp[q].nids,
+                      begin, stream_of(b, q));
+}
+
+template <typename S>
+static void enq_step_t(hydro_amd_batch* b, int q, bool flip) {
+  enq_ctl<S>(b, q, true);
+  enq_phase<S>(b, q, flip ? 1 : 0, 0);
+  enq_phase<S>(b, q, flip ? 0 : 1, 1);
 }
 
 // Closes the last step of a run (each step closes the one before it).
-static void enq_close(hydro_amd_batch* b) {
-  if (dbl(b))
-    launch_batch_ctl<double>((const InstDev<double>*) b->idev, b->ids, b->nids, false, b->st);
-  else
-    launch_batch_ctl<float>((const InstDev<float>*) b->idev, b->ids, b->nids, false, b->st);
+static void enq_close(hydro_amd_batch* b, int q) {
+  if (dbl(b)) enq_ctl<double>(b, q, false);
+  else enq_ctl<float>(b, q, false);
 }
 
-static void enq_step(hydro_amd_batch* b, bool flip) {
-  if (dbl(b)) enq_step_t<double>(b, flip);
-  else enq_step_t<float>(b, flip);
+static void enq_step(hydro_amd_batch* b, int q, bool flip) {
+  if (dbl(b)) enq_step_t<double>(b, q, flip);
+  else enq_step_t<float>(b, q, flip);
+}
+
+// The second group's stream starts after what is queued on the batch's stream.
+static int fork_groups(hydro_amd_batch* b) {
+  if (b->ngrp == 1) return 0;
+  BCHK(hipEventRecord(b->fork, b->st));
+  BCHK(hipStreamWaitEvent(b->st2, b->fork, 0));
+  return 0;
+}
+
+// What the batch's stream is given next starts after both groups' work.
+static int join_groups(hydro_amd_batch* b) {
+  if (b->ngrp == 1) return 0;
+  if (hipEventRecord(b->join, b->st2) != hipSuccess ||
+      hipStreamWaitEvent(b->st, b->join, 0) != hipSuccess)
+    BCHK(hipStreamSynchronize(b->st2));
+  return 0;
 }
 
 static int pending_courant(hydro_amd_batch* b) {
@@ -616,8 +706,8 @@ static int get_graph(hydro_amd_batch* b, int f) {
   if (b->gexec[f]) return 0;
   hipGraph_t graph;
   BCHK(hipStreamBeginCapture(b->st, hipStreamCaptureModeThreadLocal));
-  enq_step(b, f != 0);
-  enq_step(b, f == 0);
+  enq_step(b, 0, f != 0);
+  enq_step(b, 0, f == 0);
   hipError_t e = hipStreamEndCapture(b->st, &graph);
   if (e != hipSuccess) return hydro_amd_set_error("graph capture: %s", hipGetErrorString(e));
   e = hipGraphInstantiate(&b->gexec[f], graph, nullptr, nullptr, 0);
@@ -638,6 +728,20 @@ extern "C" int hydro_amd_batch_run_async(hydro_amd_batch* b, int steps) {
   }
   if (b->nids == 0 || steps == 0) return 0;
   if (pending_courant(b)) return -1;
+  if (b->ngrp > 1) {
+    // launch by launch: each group's run is one chain on its stream, met again
+    // only at the run's end (two steps of both groups as one graph: 12 grids of
+    // 64-256, mixed, 43 us a step against 26; 60 of 64-1024, fast, 411 / 402)
+    if (fork_groups(b)) return -1;
+    for (int k = 0; k < steps; k++) {
+      for (int q = 0; q < b->ngrp; q++) enq_step(b, q, b->flip);
+      b->flip = !b->flip;
+    }
+    for (int q = 0; q < b->ngrp; q++) enq_close(b, q);
+    if (join_groups(b)) return -1;
+    BCHK(hipGetLastError());
+    return 0;
+  }
   int left = steps;
   if (left >= 2) {
     const int f = b->flip ? 1 : 0;
@@ -645,10 +749,10 @@ extern "C" int hydro_amd_batch_run_async(hydro_amd_batch* b, int steps) {
     for (; left >= 2; left -= 2) BCHK(hipGraphLaunch(b->gexec[f], b->st));
   }
   if (left == 1) {
-    enq_step(b, b->flip);
+    enq_step(b, 0, b->flip);
     b->flip = !b->flip;
   }
-  enq_close(b);
+  enq_close(b, 0);
   BCHK(hipGetLastError());
   return 0;
 }
@@ -733,17 +837,20 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
   shape_by_load(b);
   const int rx = b->xiter, ry = b->yseg;
   for (int w : {1, 2, 4})
-    for (int xi : {std::max(1, rx / 2), rx, 2 * rx, 4 * rx})
+    for (int xi : {std::max(1, rx / 2), rx, 2 * rx})
       for (int ys : {std::max(1, ry / 2), ry, 2 * ry}) {
         if (hydro_amd_batch_set_tune(b, w, xi, ys) || rebuild(b)) break;
         for (int r = -1; r < reps; r++) {  // r = -1 warms up
           if (r == 0) (void) hipEventRecord(e0, b->st);
           // every x and y list at phase 0: reads buffer 0, writes buffer 1 only
+          if (fork_groups(b)) break;
           for (int k = 0; k < 4; k++) {
             const int kind = (k % 2 == 0) ? 1 : 2;
-            if (dbl(b)) sweep_list<double>(b, kind, (const InstDev<double>*) b->idev, k, 0, false);
-            else sweep_list<float>(b, kind, (const InstDev<float>*) b->idev, k, 0, false);
+            for (int q = 0; q < b->ngrp; q++)
+              if (dbl(b)) sweep_list<double>(b, q, kind, k, 0, false);
+              else sweep_list<float>(b, q, kind, k, 0, false);
           }
+          if (join_groups(b)) break;
         }
         (void) hipEventRecord(e1, b->st);
         float ms = 1e30f;
