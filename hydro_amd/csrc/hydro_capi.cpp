@@ -9,6 +9,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <cmath>
 #include <map>
 #include <mutex>
 #include <string>
@@ -449,24 +450,53 @@ static void enq_courant(hydro_amd_grid* g, const RunCtl* ctl) {
   });
 }
 
-// Rows a workgroup of the whole-step kernel takes on this grid, or 0: the two
-// sweep kernels.  The whole step saves a launch and the y march's serial
-// solves and pays with halo cells, so it is for grids whose waves do not fill
-// the GPU; counted in its waves, the lines lie where the two were measured
-// alike.  A step, whole / two sweeps, blast (a flow that moves everywhere):
-// 250x125 FP64 20.8 / 23.5 us (17.8 / 21.8), fast 13.6 / 17.2, mixed 12.1 / 15.3;
-// 500x500 (9000 waves) FP64 35.8 / 41.1 (42.5 / 43.3), fast 24.8 / 27.1; 777x600
-// (15600) FP64 48.8 / 53.6 (58.6 / 57.4), fast 32.2 / 35.6; mixed with 16 rows
-// 500x500 18.3 / 21.5, 1021x767 (18400) 30.3 / 33.1, 1531x1200 (41600) 53.7 / 53.9.
+// Rows a wave of the march kernel takes: the segments fill the GPU's `slots`
+// resident waves once or a whole number of times, sqrt(wave rows) / 240 (a
+// segment's fixed cost against the unevenness of its end, as y_rows).  The best
+// of 1-12 times, fast form: 2048x1536 (54000 wave rows) 1, 3200x2400 1-2, 4099x3001
+// 2-3, 6000x5000 3, 8192x8192 4-5, 16384x12000 (3.3e6) 7-10; mixed the same.
+static int march_rows(long ncol, long ny, long slots) {
+  const long times = std::max(1L, (long) (std::sqrt((double) (ncol * ny)) / 240 + 0.5));
+  const long nseg = std::max(1L, times * slots / ncol);
+  return (int) ((ny + nseg - 1) / nseg);
+}
+
+// How a whole step is launched on this grid (SweepTune::step).
+// Tiles save a launch and the y march's serial solves and pay with halo cells,
+// so they are for grids whose waves do not fill the GPU; counted in their waves,
+// the lines lie where they and the next were measured alike.  A step, tiles / two
+// sweeps, blast (a flow that moves everywhere): 250x125 FP64 20.8 / 23.5 us (17.8
+// / 21.8), fast 13.6 / 17.2, mixed 12.1 / 15.3; 500x500 (9000 waves) FP64 35.8 /
+// 41.1 (42.5 / 43.3), fast 24.8 / 27.1; 777x600 (15600) FP64 48.8 / 53.6 (58.6 /
+// 57.4), fast 32.2 / 35.6; mixed with 16 rows 500x500 18.3 / 21.5, 1021x767
+// (18400) 30.3 / 33.1, 1531x1200 (41600) 53.7 / 53.9.
+// The march passes over memory once a step instead of twice, which is what bounds
+// the large grids' sweeps in the fast form and half bounds them in the mixed
+// form (the FP64 form's arithmetic bounds it: no march).  March / two sweeps, fast:
+// 1021x767 (13800 wave rows) 40.7 / 40.1 (47.2 / 45.4), 1100x900 (17100) 45.7 /
+// 48.5 (53.0 / 54.6), 1400x1150 56.4 / 66.6 (67.9 / 76.8), 4099x3001 290 / 349,
+// 8192x1024 210 / 248, 8192x8192 1392 / 1794, 16384x12000 4010 / 5120; mixed:
+// 3400x2400 (137000) 144 / 144 (183 / 183), 3600x2600 (156000) 161 / 171 (206 /
+// 210), 4099x3001 204 / 219, 8192x8192 933 / 993, 16384x12000 2650 / 2810.  Its
+// waves update 60 columns, the sweeps' 63 and 64: in the mixed form, where that
+// counts, not where the grid's width makes it much worse (500x15000 145 / 142,
+// 192 / 176).
 static int step_rows(const hydro_amd_grid* g) {
   if (!folds_ghosts(g) || g->prof) return 0;  // (profiles are of the sweeps)
   if (g->tune.step >= 0) return g->tune.step;
-  auto waves = [&](long rows) {
-    return ((g->p.nx + 59L) / 60) * ((g->p.ny + rows - 5) / (rows - 4)) * rows;
-  };
+  const long nx = g->p.nx, ny = g->p.ny, ncol = (nx + 59) / 60;
+  auto waves = [&](long rows) { return ncol * ((ny + rows - 5) / (rows - 4)) * rows; };
   if (g->prec == HYDRO_AMD_FP64) return waves(8) <= 10000 ? 8 : 0;
-  if (g->prec == HYDRO_AMD_FP64_FAST) return waves(8) <= 16000 ? 8 : 0;
-  return waves(8) <= 5000 ? 8 : waves(16) <= 24000 ? 16 : 0;
+  if (g->prec == HYDRO_AMD_FP64_FAST) {
+    if (waves(8) <= 16000) return 8;
+    return ncol * ny >= 16000 ? kMarch + march_rows(ncol, ny, 4 * kSimds) : 0;
+  }
+  if (waves(8) <= 5000) return 8;
+  if (waves(16) <= 24000) return 16;
+  const long lanes = (nx + 251) / 252 * 256 + (nx + 63) / 64 * 64;  // of the sweeps
+  return ncol * ny >= 150000 && 100 * 2 * 64 * ncol <= 108 * lanes
+             ? kMarch + march_rows(ncol, ny, 5 * kSimds)
+             : 0;
 }
 
 // hydro_godunov.c:98-237: both directions, ghosts refilled before each, on the

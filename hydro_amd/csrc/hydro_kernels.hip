@@ -155,6 +155,46 @@ __global__ __launch_bounds__(64 * W) void k_step(GridGeom g, Phys<S> ph, double 
   if (!XY && cour) commit_courant(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
 }
 
+#if defined(HYDRO_FAST_UNIT) || defined(HYDRO_MIXED_UNIT)
+// Both sweeps of a large grid's step, one wave a workgroup (step_march): built for
+// the waves that the march's LDS slots leave room for, 4 a SIMD, in FP32 5.
+template <typename S, bool ST1, bool XY, int FD>
+__global__ __launch_bounds__(64) __attribute__((
+    amdgpu_waves_per_eu(sizeof(S) == 4 ? 5 : 4))) void k_step_march(GridGeom g, Phys<S> ph,
+                                                                    double dx, double dt_val,
+                                                                    const RunCtl* ctl, RunCtl* nxt,
+                                                                    GridView<S> in,
+                                                                    GridView<S> out, int bl,
+                                                                    int br, int bd, int bu,
+                                                                    uint64_t* cour, int nct,
+                                                                    int len) {
+  double dt = dt_val;
+  if (ctl) {
+    open_odd_step(ctl, nxt);
+    if (!ctl->active) return;  // grid-uniform
+    dt = ctl->dt;
+  }
+  const double dtdx = dt / dx;
+  const TraceK<S> tk = make_tracek<S>((S) dtdx, ph.scheme);
+  __shared__ YStash<S> ys;
+  const int j0 = 2 + (blockIdx.x / nct) * len, j1 = min(j0 + len, g.ny + 2);
+  double cx = 0.0, cy = 0.0;
+  step_march<S, ST1, !XY, XY, FD>(g, ph, tk, dtdx, in, out, bl, br, bd, bu, blockIdx.x % nct, j0,
+                                  j1, &ys, cx, cy);
+  if (!XY && cour) {
+    // (commit_courant for one wave: its LDS would leave room for 15 waves a CU
+    // instead of 16)
+    cx = wave_max(cx);
+    cy = wave_max(cy);
+    if (threadIdx.x == 0) {
+      unsigned long long* c = (unsigned long long*) cour + blockIdx.x % kCourSlots;
+      atomicMax(c, (unsigned long long) __double_as_longlong(cx));
+      atomicMax(c + kCourSlots, (unsigned long long) __double_as_longlong(cy));
+    }
+  }
+}
+#endif
+
 // ---- standalone CFL maximum -------------------------------------------------
 
 // CFL maxima over a thread's cells: a wave takes 64 columns of a row, the
@@ -414,9 +454,25 @@ static void launch_sweep_fd(int idim, const GridGeom& g, const Phys<S>& ph, doub
 template <typename S, int FD>
 static void launch_step_fd(bool xy, const GridGeom& g, const Phys<S>& ph, const PhysArgs& pa,
                            GridView<S> in, GridView<S> out, double dt_val, const RunCtl* ctl,
-                           RunCtl* nxt, uint64_t* cour, int waves, hipStream_t st) {
+                           RunCtl* nxt, uint64_t* cour, int rows, hipStream_t st) {
   const bool st1 = pa.slope_type == 1.0;
   const int nct = (int) cdiv(g.nx, 60);
+#if defined(HYDRO_FAST_UNIT) || defined(HYDRO_MIXED_UNIT)
+  if (rows > kMarch) {
+    const int nseg = (int) cdiv(g.ny, rows - kMarch), len = (int) cdiv(g.ny, nseg);
+#define HM(A, B)                                                                               \
+  hipLaunchKernelGGL((k_step_march<S, A, B, FD>), dim3((unsigned) nct * cdiv(g.ny, len)),      \
+                     dim3(64), 0, st, g, ph, pa.dx, dt_val, ctl, nxt, in, out, pa.bl, pa.br,   \
+                     pa.bd, pa.bu, cour, nct, len)
+    if (st1) {
+      if (xy) HM(true, true); else HM(true, false);
+    } else {
+      if (xy) HM(false, true); else HM(false, false);
+    }
+#undef HM
+    return;
+  }
+#endif
 #define HS(A, B, W)                                                                              \
   hipLaunchKernelGGL((k_step<S, A, B, W, FD>), dim3((unsigned) nct * cdiv(g.ny, W - 4)),         \
                      dim3(64 * W), 0, st, g, ph, pa.dx, dt_val, ctl, nxt, in, out, pa.bl, pa.br, \
@@ -424,7 +480,7 @@ static void launch_step_fd(bool xy, const GridGeom& g, const Phys<S>& ph, const 
 #define HSW(A, B)                                             \
   do {                                                        \
     if constexpr (sizeof(S) == 4) {                           \
-      if (waves == 16) HS(A, B, 16); else HS(A, B, 8);        \
+      if (rows == 16) HS(A, B, 16); else HS(A, B, 8);         \
     } else {                                                  \
       HS(A, B, 8);                                            \
     }                                                         \
@@ -481,20 +537,20 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
 
 template <typename S>
 void launch_step(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> in, GridView<S> out,
-                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int waves,
+                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int rows,
                  hipStream_t st) {
   const Phys<S> ph = make_phys<S>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type, pa.niter,
                                   pa.iorder, pa.scheme);
   // (FP64: the IEEE code, as in every launch that does not fill the SIMDs)
-  launch_step_fd<S, kIeee>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, waves, st);
+  launch_step_fd<S, kIeee>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, rows, st);
 }
 #else
 void launch_step_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,
                       GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
-                      uint64_t* cour, int waves, hipStream_t st) {
+                      uint64_t* cour, int rows, hipStream_t st) {
   const Phys<double> ph = make_phys<double>(pa.gamma, pa.smallr, pa.smallc, pa.slope_type,
                                             pa.niter, pa.iorder, pa.scheme);
-  launch_step_fd<double, kFast>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, waves, st);
+  launch_step_fd<double, kFast>(idim == 1, g, ph, pa, in, out, dt_val, ctl, nxt, cour, rows, st);
 }
 
 void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& pa, GridView<double> in,

@@ -68,9 +68,12 @@ struct SweepTune {
   int ywaves;   // waves per y-sweep workgroup (1..4)
   int xwaves;   // waves per x-sweep workgroup (1..4); 0: by the grid's size
   int xiter;    // row segments each x-sweep wave walks; 0: by the grid's size
-  int step;     // rows a workgroup of the whole-step kernel takes (8, 16); 0: the two
-                // sweep kernels; -1: by the grid's size
+  int step;     // whole steps in one launch: a tile's rows (8, 16), or (fast and mixed
+                // forms) kMarch + the rows of a march; 0: the two sweep kernels; -1: by
+                // the grid's size
 };
+constexpr int kMarch = 32;
+constexpr int kSimds = 1024;  // of the GPU: 256 CUs of 4
 
 // ---- launchers (hydro_kernels.hip) -----------------------------------------
 // Ghost cells: launch_sweep fills those of its direction itself (fill_ghosts
@@ -100,15 +103,16 @@ void launch_sweep_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView
 // Both sweeps of a step in one launch, x first (idim 1) or y first (idim 2,
 // which folds the CFL maxima when cour is non-null), from one state buffer
 // into the other with every ghost cell formed and stored; the rest as
-// launch_sweep.  waves: the rows a workgroup takes, 8 (mixed form: or 16).  For grids of at least
+// launch_sweep.  rows: SweepTune::step, positive (tiles of 8 rows, in the mixed
+// form or 16; marches in the fast and mixed forms).  For grids of at least
 // kGhostMin cells each way.
 template <typename S>
 void launch_step(int idim, const GridGeom& g, const PhysArgs& ph, GridView<S> in, GridView<S> out,
-                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int waves,
+                 double dt_val, const RunCtl* ctl, RunCtl* nxt, uint64_t* cour, int rows,
                  hipStream_t st);
 void launch_step_fast(int idim, const GridGeom& g, const PhysArgs& ph, GridView<double> in,
                       GridView<double> out, double dt_val, const RunCtl* ctl, RunCtl* nxt,
-                      uint64_t* cour, int waves, hipStream_t st);
+                      uint64_t* cour, int rows, hipStream_t st);
 
 template <typename S>
 void launch_courant(const GridGeom& g, const PhysArgs& ph, GridView<S> in, uint64_t* cour,

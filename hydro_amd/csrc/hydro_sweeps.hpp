@@ -871,6 +871,147 @@ __device__ __forceinline__ void tile_step(const GridGeom& g, const Phys<S>& ph,
   }
 }
 
+// ---- whole step of a large grid: one wave marches along the rows --------------
+
+// One wave takes 64 columns (the middle 60 come out updated) and rows [j0, j1)
+// through both sweeps: the y sweep is y_march's, its window and LDS slots the
+// same, and a row's x sweep (tile_x) comes before the row enters the window
+// (XY) or after it has left (y first).  Ghost cells as in tile_step.  The grid
+// passes through memory once a step: 64 bytes a cell in FP64 instead of the two
+// sweeps' 128, whose two passes alone took 1.76 of a step's 1.79 ms at 8192x8192
+// in the fast form; the march takes 1.39 ms.  The price is 64 / 60 in the y sweep
+// and, with x first, four more rows of x sweeps a segment.
+template <typename S, bool ST1, bool COUR, bool XY, int FD>
+__device__ __forceinline__ void step_march(const GridGeom& g, const Phys<S>& ph,
+                                           const TraceK<S>& tk, double dtdx,
+                                           const GridView<S>& in, const GridView<S>& out, int bl,
+                                           int br, int bd, int bu, int cb, int j0, int j1,
+                                           YStash<S>* ys, double& cx, double& cy) {
+  static_assert(FD == kFast || sizeof(S) == 4, "not for the FP64 form");
+  const long P = g.pitch;
+  const int lane = threadIdx.x & 63, i = 60 * cb + lane, top = g.ny + 2;
+  const bool o1 = ph.iorder == 1;
+  const bool wr = lane >= 2 && lane <= 61 && i <= g.nx + 1;
+  // the wave's columns: ghosts, and columns past the grid, read their source
+  const bool edge = cb == 0 || 60 * cb + 64 > g.nx + 2;  // wave-uniform
+  int is = i;
+  bool negx = false, rawx = false, gx = false;
+  if (edge) {
+    const int ic = i < g.nx + 4 ? i : g.nx + 3;
+    is = ic;
+    if (ic < 2 || ic >= g.nx + 2) {
+      is = ghost_source(1, g.nx, bl, br, ic, negx);
+      rawx = is < 2 || is >= g.nx + 2;
+      gx = is != i && i == ic;
+    }
+  }
+  bool neg;
+  const int s0 = ghost_source(2, g.ny, bd, bu, 0, neg);
+  const int s1 = ghost_source(2, g.ny, bd, bu, 1, neg);
+  const int s2 = ghost_source(2, g.ny, bd, bu, top, neg);
+  const int s3 = ghost_source(2, g.ny, bd, bu, top + 1, neg);
+  auto load = [&](int j) {
+    // (values, not references: a selected address would keep them in memory)
+    int js = j < 2 ? (j == 0 ? +s0 : +s1) : j;
+    if (j >= top) js = j == top ? +s2 : +s3;
+    const long o = (long) js * P + is;
+    return TCell<S>{in.p[0][o], in.p[1][o], in.p[2][o], in.p[3][o]};
+  };
+  auto store = [&](int j, const TCell<S>& v) {
+    const long o = (long) j * P + i;
+    st_stream(&out.p[0][o], v.r);
+    st_stream(&out.p[1][o], v.mx);
+    st_stream(&out.p[2][o], v.my);
+    st_stream(&out.p[3][o], v.e);
+  };
+  const Q4<S> z = {(S) 0, (S) 0, (S) 0, (S) 0};
+  // window: C = row j-2 (being updated), D = row j-1, as in y_march
+  Q4<S> qC = z, qD = z;
+  S cD = 0, rD = 0, iD = 0;
+  TCell<S> uN = load(j0 - 2);
+  // take row j, prefetch row j+1, update row j-2, shift the window
+  auto row = [&](int j) __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");  // (as in y_march)
+    TCell<S> u = uN;
+    uN = load(j <= j1 ? j + 1 : j1 + 1);  // last row: a harmless reload
+    const bool ghost = j < 2 || j >= top;  // wave-uniform
+    if constexpr (XY) {
+      if (edge) {
+        if (negx) u.mx = -u.mx;
+        if (gx && j >= j0 && j < j1) store(j, u);
+      }
+      const TCell<S> v = tile_x<S, ST1, FD>(ph, tk, dtdx, u);
+      if (!ghost) u = v;
+      else {
+        bool n;
+        const int js = ghost_source(2, g.ny, bd, bu, j, n);
+        if (js >= 2 && js < top) u = v;
+        if (n) u.my = -u.my;
+        if (js != j && wr) store(j, u);
+      }
+    } else if (ghost) {
+      bool n;
+      const int js = ghost_source(2, g.ny, bd, bu, j, n);
+      if (n) u.my = -u.my;
+      if (js != j && wr) store(j, u);
+    }
+    const int sj = j % 3;  // wave-uniform
+    stash_put_cell(ys->u[sj], lane, Cell<S>{u.r, u.my, u.mx, u.e});
+    Prim<S> pE;
+    if constexpr (FD == kFast) pE = prim_fast(u.r, u.my, u.mx, u.e, ph);
+    else pE = prim_cell<S, false>(u.r, u.my, u.mx, u.e, ph);
+    if (j >= j0) {
+      Q4<S> qxmD, qxpD;
+      const Q4<S> dqD = o1 ? z : slope_form<S, ST1, FD>(qC, qD, pE.q, ph);
+      trace_fast(qD, dqD, cD, iD, rD, tk, qxmD, qxpD);
+      const Q4<S> qxmC = stash_get(ys->xm, lane);
+      stash_put(ys->xm, lane, qxmD);
+      if (j > j0) {
+        const Q4<double> fcur = to_d4(riemann_flux<S, FD>(qxmC, qxpD, ph));  // face (j-2 | j-1)
+        const Q4<double> fprev = stash_get(ys->f, lane);
+        stash_put(ys->f, lane, fcur);
+        if (j > j0 + 1) {
+          asm volatile("" ::: "memory");
+          const Cell<S> uC = stash_get_cell(ys->u[sj == 2 ? 0 : sj + 1], lane);  // row j-2
+          TCell<S> n;
+          n.r = (S) update1<S>(uC.u0, fprev.r, fcur.r, dtdx);
+          n.my = (S) update1<S>(uC.u1, fprev.u, fcur.u, dtdx);
+          n.mx = (S) update1<S>(uC.u2, fprev.v, fcur.v, dtdx);
+          n.e = (S) update1<S>(uC.u3, fprev.p, fcur.p, dtdx);
+          if constexpr (!XY) {
+            if (edge) {
+              if (rawx) n = TCell<S>{uC.u0, uC.u2, uC.u1, uC.u3};
+              if (negx) n.mx = -n.mx;
+              if (gx) store(j - 2, n);
+            }
+            n = tile_x<S, ST1, FD>(ph, tk, dtdx, n);
+          }
+          if (wr) {
+            store(j - 2, n);
+            if (COUR) {
+              S ax, ay;
+              courant_cell<S, FD>(n.r, n.mx, n.my, n.e, ph, ax, ay);
+              cx = maxm(cx, (double) ax);
+              cy = maxm(cy, (double) ay);
+            }
+          }
+        }
+      }
+    }
+    qC = qD;
+    qD = pE.q;
+    cD = pE.c;
+    rD = pE.rinv;
+    iD = pE.cinv;
+  };
+  int j = j0 - 2;
+  for (; j + 1 <= j1 + 1; j += 2) {
+    row(j);
+    row(j + 1);
+  }
+  if (j <= j1 + 1) row(j);
+}
+
 // ---- ghost cells -------------------------------------------------------------
 
 // make_boundary.c:237-289 (x) and 381-433 (y) for one interior line k and one
