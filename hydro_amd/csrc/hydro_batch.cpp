@@ -48,6 +48,9 @@ struct Inst {
   void* mem[2] = {nullptr, nullptr};
   long long bytes = 0;
   bool need_cour = false;  // CFL maxima of the initial state still to compute
+  // the state is in mem[base] after step n0; where steps are whole (march > 0,
+  // their rows a wave), it changes buffers with each
+  int base = 0, n0 = 0, march = 0;
 };
 
 // Instances that are advanced together, launch by launch, on one stream.
@@ -85,7 +88,8 @@ struct hydro_amd_batch {
   bool flip = false;             // next step runs Q before P
   hipGraphExec_t gexec[2] = {nullptr, nullptr};
   BatchTune tune = {1, 0, 0};
-  int xiter = 1, yseg = 1;       // the shape in use (rebuild)
+  int xiter = 1, yseg = 1, march = 0;  // the shape in use (rebuild)
+  bool fresh = false;            // no step has been queued since hctl was read
   std::vector<int> live_ids;
   RunCtl* hctl = nullptr;        // pinned host copy of the run controls
   void* hidev = nullptr;         // pinned host copy of the instance array
@@ -185,10 +189,24 @@ extern "C" long long hydro_amd_batch_bytes_used(const hydro_amd_batch* b) {
 template <typename S>
 static GridView<S> view_of(const hydro_amd_batch* b, const Inst& in, int k) {
   GridView<S> v;
-  S* base = (S*) in.mem[k] + kOrigin;
+  S* base = (S*) in.mem[in.base ^ k] + kOrigin;  // k = 0: the state's after step n0
   for (int q = 0; q < 4; q++) v.p[q] = base + q * in.plane;
   (void) b;
   return v;
+}
+
+// A new initial state is (being) put into both buffers and the run control reset.
+static void reset_run(hydro_amd_batch* b, int id) {
+  Inst& in = b->inst[id];
+  in.base = in.n0 = in.march = 0;
+  in.need_cour = true;
+  RunCtl& c = b->hctl[id];
+  c = RunCtl();
+  c.tend = in.p.tend;
+  c.nstepmax = in.p.nstepmax;
+  launch_zero_u64(b->cour + (size_t) id * 2 * kInstSlots, 2 * kInstSlots, b->st);
+  launch_batch_set_ctl(b->ctl + id, 0.0, 0.0, in.p.tend, 0, in.p.nstepmax, 0, b->st);
+  b->dirty = true;  // parity back to even
 }
 
 extern "C" int hydro_amd_batch_add(hydro_amd_batch* b, const hydro_amd_params* p) {
@@ -226,12 +244,9 @@ extern "C" int hydro_amd_batch_add(hydro_amd_batch* b, const hydro_amd_params* p
     BCHK(hipMemsetAsync(in.mem[k], 0, sz, b->st));
   }
   in.live = true;
-  in.need_cour = true;
   b->used += in.bytes;
-  launch_zero_u64(b->cour + (size_t) id * 2 * kInstSlots, 2 * kInstSlots, b->st);
-  launch_batch_set_ctl(b->ctl + id, 0.0, 0.0, p->tend, 0, p->nstepmax, 0, b->st);
+  reset_run(b, id);
   BCHK(hipGetLastError());
-  b->dirty = true;
   return id;
 }
 
@@ -259,17 +274,14 @@ extern "C" int hydro_amd_batch_remove(hydro_amd_batch* b, int id) {
 static int init_inst(hydro_amd_batch* b, int id, int bx, int by0, int by1, double e) {
   Inst* in = live(b, id);
   if (!in) return -1;
+  reset_run(b, id);
   if (dbl(b))
     launch_init<double>(in->g, view_of<double>(b, *in, 0), view_of<double>(b, *in, 1), bx, by0,
                         by1, e, b->st);
   else
     launch_init<float>(in->g, view_of<float>(b, *in, 0), view_of<float>(b, *in, 1), bx, by0, by1,
                        e, b->st);
-  launch_zero_u64(b->cour + (size_t) id * 2 * kInstSlots, 2 * kInstSlots, b->st);
-  launch_batch_set_ctl(b->ctl + id, 0.0, 0.0, in->p.tend, 0, in->p.nstepmax, 0, b->st);
   BCHK(hipGetLastError());
-  in->need_cour = true;
-  b->dirty = true;  // parity back to even
   return 0;
 }
 
@@ -294,11 +306,35 @@ extern "C" int hydro_amd_batch_init_blast(hydro_amd_batch* b, int id, int bx, in
   return init_inst(b, id, bx + 2, by + 2, by + 3, e);
 }
 
+// Reads the run controls of ids [0, maxid] into the pinned host copy.
+static int read_ctl(hydro_amd_batch* b) {
+  if (b->maxid < 0) return 0;
+  BCHK(hipMemcpyAsync(b->hctl, b->ctl, sizeof(RunCtl) * (b->maxid + 1), hipMemcpyDeviceToHost,
+                      b->st));
+  BCHK(hipStreamSynchronize(b->st));
+  b->fresh = true;
+  return 0;
+}
+
+// The buffer that an instance's state is in, -1 on error.  Waits for the
+// batch's stream if steps of the instance may have been queued since its run
+// control was read.
+static int state_buf(hydro_amd_batch* b, int id) {
+  const Inst& in = b->inst[id];
+  if (!in.march) return in.base;
+  const RunCtl& c = b->hctl[id];
+  const bool ended = c.fault || !(c.t < c.tend) || c.nstep >= c.nstepmax;
+  if (!b->fresh && !ended && read_ctl(b)) return -1;
+  return in.base ^ ((c.nstep - in.n0) & 1);
+}
+
 extern "C" int hydro_amd_batch_download(hydro_amd_batch* b, int id, double* u) {
   Inst* in = live(b, id);
   if (!in || !u) return in ? hydro_amd_set_error("null argument") : -1;
   const long nxt = in->p.nx + 4, rows = 4L * (in->p.ny + 4);
-  const void* src = (const char*) in->mem[0] + kOrigin * b->esz;
+  const int k = state_buf(b, id);
+  if (k < 0) return -1;
+  const void* src = (const char*) in->mem[k] + kOrigin * b->esz;
   return stage_d2h(u, 8, src, (int) b->esz, in->g.pitch, nxt, rows, b->st) ? -1 : 0;
 }
 
@@ -308,7 +344,9 @@ int hydro_amd_batch_raw_view(hydro_amd_batch* b, int id, const void** src, long*
                              long* width, long* rows, int* esz) {
   Inst* in = live(b, id);
   if (!in) return -1;
-  *src = (const char*) in->mem[0] + kOrigin * b->esz;
+  const int k = state_buf(b, id);
+  if (k < 0) return -1;
+  *src = (const char*) in->mem[k] + kOrigin * b->esz;
   *pitch = in->g.pitch;
   *width = in->p.nx + 4;
   *rows = 4L * (in->p.ny + 4);
@@ -326,7 +364,9 @@ int hydro_amd_batch_download_raw(hydro_amd_batch* b, int id, void* dst, int* ele
   if (!in || !dst) return in ? hydro_amd_set_error("null argument") : -1;
   const long nxt = in->p.nx + 4, rows = 4L * (in->p.ny + 4);
   const size_t w = b->esz;
-  const void* src = (const char*) in->mem[0] + kOrigin * w;
+  const int k = state_buf(b, id);
+  if (k < 0) return -1;
+  const void* src = (const char*) in->mem[k] + kOrigin * w;
   if (stage_d2h(dst, (int) w, src, (int) w, in->g.pitch, nxt, rows, st ? st : b->st)) return -1;
   if (elem_size) *elem_size = (int) w;
   return 0;
@@ -381,10 +421,7 @@ extern "C" int hydro_amd_batch_upload(hydro_amd_batch* b, int id, const double* 
   if (stage_h2d(dst, (int) b->esz, in->g.pitch, u, 8, nxt, rows, b->st)) return -1;
   BCHK(hipMemcpyAsync(in->mem[1], in->mem[0], (size_t) in->bytes / 2, hipMemcpyDeviceToDevice,
                       b->st));
-  launch_zero_u64(b->cour + (size_t) id * 2 * kInstSlots, 2 * kInstSlots, b->st);
-  launch_batch_set_ctl(b->ctl + id, 0.0, 0.0, in->p.tend, 0, in->p.nstepmax, 0, b->st);
-  in->need_cour = true;
-  b->dirty = true;
+  reset_run(b, id);
   return 0;
 }
 
@@ -392,6 +429,11 @@ extern "C" int hydro_amd_batch_upload(hydro_amd_batch* b, int id, const double* 
 
 static long x_segments(const hydro_amd_params& p) {
   return (long) ((p.nx + kXSeg - 1) / kXSeg) * p.ny;
+}
+
+// The sweeps form the ghosts of all but very narrow instances.
+static bool folds_ghosts(const Inst& in) {
+  return in.p.nx >= kGhostMin && in.p.ny >= kGhostMin;
 }
 
 // Task shape by the load.  As in a single grid's y sweep (y_rows,
@@ -405,18 +447,32 @@ static long x_segments(const hydro_amd_params& p) {
 // with fixed shapes (2 or 4 waves of 8 or 32 segments, 32 or 64 rows) in one
 // chain and takes with these: 12 small grids, mixed, 138 and 24 us; 30, fast,
 // 156 and 94; 60, FP64, 701 and 565; 24 of up to 4096, mixed, 1.21 and 1.12 ms.
+// Large loads of the fast and mixed forms take whole steps instead (step_march;
+// for the line's reasons see step_rows, hydro_capi.cpp), in segments that fill the
+// 4096 waves the GPU holds twice, of at most 64 rows.  A step, sweeps and whole, the
+// best segment in brackets, of loads of so many wave rows: 49000 (30 grids of
+// 150-500) fast 92 and 92 us (8), mixed 67 and 65 (8); 219000 (60 of 64-1024) 364
+// and 305 (24), 224 and 209 (20-32); 1.07e6 (300 of 64-1024) 1772 and 1413 (64),
+// 1068 and 956 (96); 1.21e6 (24 of 128-4096) 2017 and 1552 (96), 1136 and 1021 (64).
 static void shape_by_load(hydro_amd_batch* b) {
-  long segs = 0, wrows = 0;
+  long segs = 0, wrows = 0, mrows = 0;
+  bool fold = true;
   for (int id : b->live_ids) {
     const hydro_amd_params& p = b->inst[id].p;
     segs += x_segments(p);
     wrows += (long) ((p.nx + 63) / 64) * p.ny;
+    mrows += (long) ((p.nx + 59) / 60) * p.ny;
+    fold = fold && folds_ghosts(b->inst[id]);
   }
   auto root = [](long n, double by, int most) {
     return std::max(1, std::min(most, (int) (std::sqrt((double) n) / by + 0.5)));
   };
   b->xiter = b->tune.xiter > 0 ? b->tune.xiter : root(segs, 50, 16);
   b->yseg = b->tune.yseg > 0 ? b->tune.yseg : root(wrows, 28, 40);
+  const long line = b->prec == HYDRO_AMD_FP64_FAST ? 80000 : 150000;
+  b->march = b->prec != HYDRO_AMD_FP64 && fold && b->tune.xiter <= 0 && mrows >= line
+                 ? (int) std::min(64L, mrows / 8192)
+                 : 0;
 }
 
 // Rows per wave in an instance's y tasks: the instance's rows split evenly
@@ -426,11 +482,6 @@ static int inst_yseg(const hydro_amd_batch* b, int ny) {
   const long W = b->tune.waves, per = W * b->yseg;
   const long nrg = (ny + per - 1) / per;
   return (int) ((ny + W * nrg - 1) / (W * nrg));
-}
-
-// The sweeps form the ghosts of all but very narrow instances.
-static bool folds_ghosts(const Inst& in) {
-  return in.p.nx >= kGhostMin && in.p.ny >= kGhostMin;
 }
 
 template <typename S>
@@ -454,6 +505,8 @@ static InstDev<S> inst_dev(hydro_amd_batch* b, int id) {
   d.fold = folds_ghosts(in);
   d.nseg = (in.p.nx + kXSeg - 1) / kXSeg;
   d.yseg = inst_yseg(b, in.p.ny);
+  d.march = in.march;
+  d.n0 = in.n0;
   return d;
 }
 
@@ -474,21 +527,21 @@ static BList sweep_tasks(const hydro_amd_batch* b, int id, int kind) {
   return l;
 }
 
+// An instance's whole steps.
+static BList march_tasks(const hydro_amd_batch* b, int id) {
+  const Inst& in = b->inst[id];
+  BList l{id, 3, 0, 0, 0, 0};
+  l.ncb = (in.p.nx + 59) / 60;
+  l.count = (int) (l.ncb * ((in.p.ny + in.march - 1) / in.march));
+  return l;
+}
+
 // Ghost fills of one narrow instance in direction idim, kBoundaryChunk
 // (line, var) pairs per task so a large instance spreads over many workgroups.
 static BList ghost_tasks(const hydro_amd_batch* b, int id, int idim) {
   const hydro_amd_params& p = b->inst[id].p;
   const long tot = 4L * (idim == 1 ? p.ny : p.nx);
   return BList{id, idim, 0, (int) ((tot + kBoundaryChunk - 1) / kBoundaryChunk), kBoundaryChunk, 0};
-}
-
-// Reads the run controls of ids [0, maxid] into the pinned host copy.
-static int read_ctl(hydro_amd_batch* b) {
-  if (b->maxid < 0) return 0;
-  BCHK(hipMemcpyAsync(b->hctl, b->ctl, sizeof(RunCtl) * (b->maxid + 1), hipMemcpyDeviceToHost,
-                      b->st));
-  BCHK(hipStreamSynchronize(b->st));
-  return 0;
 }
 
 // Parts a load into two groups of about the same work, each with a
@@ -544,6 +597,14 @@ static int rebuild(hydro_amd_batch* b) {
     }
   if (read_ctl(b)) return -1;
   shape_by_load(b);
+  for (int id : b->live_ids) {
+    Inst& in = b->inst[id];
+    in.base = state_buf(b, id);
+    in.n0 = b->hctl[id].nstep;
+    // (even segments)
+    const int nseg = b->march ? (in.p.ny + b->march - 1) / b->march : 1;
+    in.march = b->march ? (in.p.ny + nseg - 1) / nseg : 0;
+  }
   if (split_load(b)) return -1;
   std::vector<BList> all;
   long need = 0;
@@ -556,6 +617,10 @@ static int rebuild(hydro_amd_batch* b) {
       const int id = b->live_ids[m];
       const bool even = (b->hctl[id].nstep % 2) == 0;
       const int gen = b->inst[id].p.slope_type == 1.0 ? 0 : 1;
+      if (b->march) {
+        L[0][gen].push_back(march_tasks(b, id));
+        continue;
+      }
       L[even ? 0 : 2][gen].push_back(sweep_tasks(b, id, 1));
       L[even ? 3 : 1][gen].push_back(sweep_tasks(b, id, 2));
       if (!folds_ghosts(b->inst[id])) {
@@ -649,6 +714,15 @@ static void enq_ctl(hydro_amd_batch* b, int q, bool begin) {
 template <typename S>
 static void enq_step_t(hydro_amd_batch* b, int q, bool flip) {
   enq_ctl<S>(b, q, true);
+  if (b->march) {
+    const Group& gr = b->grp[q];
+    const BTask* t = b->tasks + gr.off[0];
+    if constexpr (sizeof(S) == 8)
+      launch_batch_march_fast((const InstDev<S>*) b->idev, t, gr.n[0], gr.n1[0], stream_of(b, q));
+    else
+      launch_batch_march((const InstDev<S>*) b->idev, t, gr.n[0], gr.n1[0], stream_of(b, q));
+    return;
+  }
   enq_phase<S>(b, q, flip ? 1 : 0, 0);
   enq_phase<S>(b, q, flip ? 0 : 1, 1);
 }
@@ -728,6 +802,7 @@ extern "C" int hydro_amd_batch_run_async(hydro_amd_batch* b, int steps) {
   }
   if (b->nids == 0 || steps == 0) return 0;
   if (pending_courant(b)) return -1;
+  b->fresh = false;
   if (b->ngrp > 1) {
     // launch by launch: each group's run is one chain on its stream, met again
     // only at the run's end (two steps of both groups as one graph: 12 grids of
@@ -816,6 +891,14 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
   BCHK(hipStreamSynchronize(b->st));
   if (b->dirty && rebuild(b)) return -1;
   if (b->nids == 0) return hydro_amd_set_error("empty batch");
+  if (b->march) {  // faster than the sweeps at their best shape (shape_by_load)
+    if (best) {
+      best[0] = b->tune.waves;
+      best[1] = b->xiter;
+      best[2] = b->yseg;
+    }
+    return 0;
+  }
   const int nc = b->maxid + 1;
   std::vector<RunCtl> saved(nc);
   BCHK(hipMemcpy(saved.data(), b->ctl, sizeof(RunCtl) * nc, hipMemcpyDeviceToHost));

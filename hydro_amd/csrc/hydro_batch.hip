@@ -18,6 +18,8 @@
 //   x task: wpb * xiter consecutive 60-cell row segments (each wave walks xiter)
 //   y task: 64 columns x (wpb * yseg) rows (each wave marches yseg rows; the
 //           instance's yseg evens its rows out over its row groups)
+//   whole steps (large loads of the fast and mixed forms; one launch a step for
+//           every parity): 60 columns x the instance's march rows, one wave
 // so the CFL reduction of a task never mixes instances.  Run control (t, dt,
 // nstep, active) and CFL slots are per instance, on the device.
 //
@@ -103,6 +105,62 @@ __global__ __launch_bounds__(256) void k_batch_sweep_y(const InstDev<S>* __restr
   }
 }
 
+// The buffer an instance's state is in between steps.
+template <typename S>
+__device__ __forceinline__ int state_buf(const InstDev<S>& d) {
+  return d.march ? (d.ctl->nstep - d.n0) & 1 : 0;
+}
+
+#if defined(HYDRO_FAST_UNIT) || defined(HYDRO_MIXED_UNIT)
+// Whole steps (step_march): of even steps x first, of odd ones y first with the
+// CFL maxima of the new state.
+template <typename S, bool ST1, int FD>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(
+    sizeof(S) == 4 ? 5 : 4))) void k_batch_march(const InstDev<S>* __restrict__ inst,
+                                                 const BTask* __restrict__ tasks) {
+  const BTask tk = tasks[blockIdx.x];
+  const InstDev<S>& d = inst[tk.inst];
+  if (!d.ctl->active) return;  // workgroup-uniform
+  const double dtdx = d.ctl->dt / d.dx;
+  const TraceK<S> tr = make_tracek<S>((S) dtdx, d.ph.scheme);
+  const int cur = state_buf(d);
+  const GridView<S> in = d.buf[cur], out = d.buf[1 - cur];
+  __shared__ YStash<S> ys;
+  const int j0 = 2 + tk.b * d.march, j1 = min(j0 + d.march, d.g.ny + 2);
+  double cx = 0.0, cy = 0.0;
+  if (d.ctl->nstep % 2 == 0) {
+    step_march<S, ST1, false, true, FD>(d.g, d.ph, tr, dtdx, in, out, d.bl, d.br, d.bd, d.bu, tk.a,
+                                        j0, j1, &ys, cx, cy);
+  } else {
+    step_march<S, ST1, true, false, FD>(d.g, d.ph, tr, dtdx, in, out, d.bl, d.br, d.bd, d.bu, tk.a,
+                                        j0, j1, &ys, cx, cy);
+    commit_courant_wave(cx, cy, d.cour, kInstSlots, blockIdx.x % kInstSlots);
+  }
+}
+
+template <typename S, int FD>
+static void launch_march_fd(const InstDev<S>* inst, const BTask* tasks, int ntask, int nst1,
+                            hipStream_t st) {
+  if (nst1 > 0)
+    hipLaunchKernelGGL((k_batch_march<S, true, FD>), dim3(nst1), dim3(64), 0, st, inst, tasks);
+  if (ntask > nst1)
+    hipLaunchKernelGGL((k_batch_march<S, false, FD>), dim3(ntask - nst1), dim3(64), 0, st, inst,
+                       tasks + nst1);
+}
+#endif
+#ifdef HYDRO_FAST_UNIT
+void launch_batch_march_fast(const InstDev<double>* inst, const BTask* tasks, int ntask, int nst1,
+                             hipStream_t st) {
+  launch_march_fd<double, kFast>(inst, tasks, ntask, nst1, st);
+}
+#endif
+#ifdef HYDRO_MIXED_UNIT
+void launch_batch_march(const InstDev<float>* inst, const BTask* tasks, int ntask, int nst1,
+                        hipStream_t st) {
+  launch_march_fd<float, kIeee>(inst, tasks, ntask, nst1, st);
+}
+#endif
+
 // Ghost fills of the instances too narrow for the sweeps to form theirs
 // (kind = direction): of (line, var) pairs [a, a + kBoundaryChunk)
 // of one instance per task, from buffer `phase` into both buffers.
@@ -122,21 +180,21 @@ __global__ __launch_bounds__(256) void k_batch_boundary(const InstDev<S>* inst,
   }
 }
 
-// CFL maxima of buffer 0 for the listed instances (admission / step 0).
+// CFL maxima of the listed instances' states (admission / step 0).
 template <typename S>
 __global__ __launch_bounds__(256) void k_batch_courant(const InstDev<S>* inst, const int* ids,
                                                        int nids) {
   for (int t = blockIdx.x; t < nids * 64; t += gridDim.x) {
     const InstDev<S>& d = inst[ids[t / 64]];
     const int part = t % 64;
+    const GridView<S> u = d.buf[state_buf(d)];
     const long n = (long) d.g.nx * d.g.ny;
     double cx = 0.0, cy = 0.0;
     for (long c = (long) part * blockDim.x + threadIdx.x; c < n; c += 64L * blockDim.x) {
       const long jj = c / d.g.nx, ii = c - jj * d.g.nx;
       const long o = (jj + 2) * d.g.pitch + ii + 2;
       S ax, ay;
-      courant_cell<S>(d.buf[0].p[0][o], d.buf[0].p[1][o], d.buf[0].p[2][o], d.buf[0].p[3][o],
-                      d.ph, ax, ay);
+      courant_cell<S>(u.p[0][o], u.p[1][o], u.p[2][o], u.p[3][o], d.ph, ax, ay);
       cx = maxm(cx, (double) ax);
       cy = maxm(cy, (double) ay);
     }

@@ -15,17 +15,20 @@ struct InstDev {
   GridGeom g;
   Phys<S> ph;
   double dx, cf, smallc;  // dt = cf*dx / max(cx, cy, smallc)
-  GridView<S> buf[2];     // state in buf[0] between steps
+  GridView<S> buf[2];     // state in buf[0] between steps; with march, after step n0
+                          // (RunCtl::nstep) and every other one from there
   RunCtl* ctl;
   uint64_t* cour;         // 2 * kInstSlots
   int bl, br, bd, bu;     // boundary types
   int fold;               // the sweeps form the ghosts (else k_batch_boundary does)
   int nseg;               // 60-cell segments per row
   int yseg;               // rows each wave marches in this instance's y tasks
+  int march, n0;          // whole steps, and their rows a wave; 0: the two sweeps
 };
 
 // One workgroup's work: kind 1 = x (a = first segment), 2 = y (a = 64-column
-// block, b = row-segment group); for ghost fills kind is the direction.
+// block, b = row-segment group), 3 = whole steps (a = 60-column block, b = row
+// segment); for ghost fills kind is the direction.
 struct BTask {
   int inst, kind, a, b;
 };
@@ -51,6 +54,12 @@ struct BatchTune {
 template <typename S>
 void launch_batch_sweep(int kind, const InstDev<S>* inst, const BTask* tasks, int ntask,
                         int nst1, int phase, bool ghosts, int waves, int xiter, hipStream_t st);
+// Whole steps (fast and mixed forms), on a table of kind 3: of instances with
+// march > 0, from the buffer their state is in into the other.
+void launch_batch_march(const InstDev<float>* inst, const BTask* tasks, int ntask, int nst1,
+                        hipStream_t st);
+void launch_batch_march_fast(const InstDev<double>* inst, const BTask* tasks, int ntask, int nst1,
+                             hipStream_t st);
 template <typename S>
 void launch_batch_boundary(const InstDev<S>* inst, const BTask* tasks, int ntask, int phase,
                            hipStream_t st);

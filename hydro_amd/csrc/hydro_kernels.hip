@@ -181,17 +181,7 @@ __global__ __launch_bounds__(64) __attribute__((
   double cx = 0.0, cy = 0.0;
   step_march<S, ST1, !XY, XY, FD>(g, ph, tk, dtdx, in, out, bl, br, bd, bu, blockIdx.x % nct, j0,
                                   j1, &ys, cx, cy);
-  if (!XY && cour) {
-    // (commit_courant for one wave: its LDS would leave room for 15 waves a CU
-    // instead of 16)
-    cx = wave_max(cx);
-    cy = wave_max(cy);
-    if (threadIdx.x == 0) {
-      unsigned long long* c = (unsigned long long*) cour + blockIdx.x % kCourSlots;
-      atomicMax(c, (unsigned long long) __double_as_longlong(cx));
-      atomicMax(c + kCourSlots, (unsigned long long) __double_as_longlong(cy));
-    }
-  }
+  if (!XY && cour) commit_courant_wave(cx, cy, cour, kCourSlots, blockIdx.x % kCourSlots);
 }
 #endif
 

@@ -108,6 +108,19 @@ __device__ __forceinline__ void commit_courant(double cx, double cy, uint64_t* c
   __syncthreads();
 }
 
+// The same for a workgroup of one wave, without LDS (which would leave the march
+// kernels room for 15 waves a CU instead of 16).
+__device__ __forceinline__ void commit_courant_wave(double cx, double cy, uint64_t* cour,
+                                                    int nslot, int slot) {
+  cx = wave_max(cx);
+  cy = wave_max(cy);
+  if (threadIdx.x == 0) {
+    atomicMax((unsigned long long*) &cour[slot], (unsigned long long) __double_as_longlong(cx));
+    atomicMax((unsigned long long*) &cour[nslot + slot],
+              (unsigned long long) __double_as_longlong(cy));
+  }
+}
+
 // Max over NSLOT slot pairs (clearing them), then compute_deltat.c:197:
 // dt = cfl*dx / MAX(cx, MAX(cy, smallc)).  Called by one whole wave; every
 // lane returns the same dt.  (All loads go out before the first is used: with

@@ -57,3 +57,53 @@ def test_groups(load, form):
         assert bits_differ(b.download(i), alone(late, 7, 7)) == 0
         for j, p, k in other.ids:
             assert bits_differ(other.download(j), alone(p, k, 7)) == 0, (p, "7 steps")
+
+
+@pytest.mark.parametrize("form", [hydro_amd.FP64_FAST, hydro_amd.MIXED])
+def test_whole_steps(form):
+    """Loads large enough for whole steps, whose states change buffers with each
+    step: odd and even counts, runs that end on their own at either parity, a
+    load that falls below the line and one whose narrow grid rules them out."""
+    big = [(1900, 2300), (700, 3001), (61, 5000), (500, 7)]
+    big += [(2001, 1200)] if form == hydro_amd.MIXED else []
+    with hydro_amd.Batch(form) as b:
+        ids = []
+        for k, (nx, ny) in enumerate(big):
+            p = params(nx, ny, k, form)
+            p.nstepmax = (2**31 - 1, 2**31 - 1, 5, 6)[k % 4]
+            i = b.add(p)
+            b.init_blast(i, nx // 2, ny // 3, 1.0 + k)
+            ids.append((i, p, k))
+
+        def check(steps):
+            for i, p, k in ids:
+                want = alone(p, k, min(steps, p.nstepmax))
+                assert bits_differ(b.download(i), want) == 0, (p, steps)
+        b.run(3)
+        check(3)
+        b.autotune(1)
+        b.run_async(1)
+        check(4)  # (without a sync)
+        b.run_async(3)
+        u = b.download(ids[2][0])
+        b.sync()
+        assert np.array_equal(u, b.download(ids[2][0]))
+        check(7)
+        thin = params(2, 90, 5, form)  # rules whole steps out
+        t = b.add(thin)
+        b.init_blast(t, 1, 30, 6.0)
+        b.run(2)
+        check(9)
+        b.remove(t)
+        b.run(1)
+        check(10)
+        b.remove(ids.pop(0)[0])  # (fast: below the line from here)
+        b.run(3)
+        check(13)
+        b.set_tune(2, 4, 8)
+        b.run(1)
+        check(14)
+        i, p, k = ids[0]
+        b.init_blast(i, p.nx // 2, p.ny // 3, 1.0 + k)
+        b.run(1)
+        assert bits_differ(b.download(i), alone(p, k, 1)) == 0
