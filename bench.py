@@ -15,10 +15,13 @@ are measured beside it on the same grid.
 
 Prints ONE JSON line.  `value` is interior cell-updates per second (the
 reference's MC/s unit x 1e6) over the timed steps, run as the product runs
-them: replayed HIP graphs, no per-launch instrumentation.  Per-kernel
+them: replayed HIP graphs, no per-launch instrumentation, and where it is
+the faster way (large grids in the fast and mixed forms) each step in one
+launch.  `step_bytes` holds that step against the bytes it cannot do without
+(each cell read and written once).  Per-kernel
 durations come from a second, instrumented pass over the same grid (HIP
-events recorded on the grid's own stream around every launch).  `roofline` is
-for the dominant sweep kernel: algorithmic bytes (64 B per cell per sweep in
+events recorded on the grid's own stream around every launch), always of the
+two sweep kernels.  `roofline` is for the dominant one of those: algorithmic bytes (64 B per cell per sweep in
 FP64: read 4 doubles, write 4) over its average duration; its `traffic` is
 the HBM bytes the kernel really moves (two rocprofv3 --pmc passes,
 calibrated on a copy kernel), and its `copy_ceiling` the rate of a plain copy
@@ -67,7 +70,8 @@ def progress(what):
 
 def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_steps=20):
     """Times `steps` steps of one grid on the product path (graph replay), then
-    an instrumented pass of prof_steps steps for per-kernel durations."""
+    an instrumented pass of prof_steps steps for per-kernel durations (of the
+    two sweep kernels, also where the product takes whole steps)."""
     import hydro_amd
     p = hydro_amd.Params(nx=nx, ny=ny, dx=1.0 / nx, courant_factor=0.8, niter_riemann=10,
                          iorder=2, slope_type=1.0, tend=1e30, nstepmax=2**31 - 1,
@@ -107,12 +111,17 @@ def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_
         "t_end": tstate[0],
         "kernels": {k: {"avg_ms": (v[0] / v[1] if v[1] else None), "launches": v[1]}
                     for k, v in prof.items()},
-        "kernels_note": f"instrumented pass of {prof_steps} steps after the timed region",
+        "kernels_note": f"instrumented pass of {prof_steps} steps after the timed region, "
+                        "by the two sweep kernels",
+        "step_bytes": {"bytes_per_cell": bpc,
+                       "achieved_GBps": round(cells * steps * bpc / elapsed / 1e9, 1),
+                       "frac": round(cells * steps * bpc / elapsed / 1e9 / HBM_PEAK_GBS, 4)},
         "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                      "traffic": None, "kernel": kern,
                      "algorithmic_bytes_per_launch": per_launch_bytes,
                      "bytes_per_cell_sweep": bpc},
+        # (the bytes of two sweeps, whatever the step's launches)
         "step_roofline_frac": round(cells * steps * 2 * bpc / elapsed / 1e9 / HBM_PEAK_GBS, 4),
     }
 
@@ -120,6 +129,7 @@ def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_
 def form_summary(r, precision):
     return {"form": FORM_NAMES[precision], "value": r["value"], "ms_per_step": r["ms_per_step"],
             "roofline_frac": r["roofline"]["frac"], "step_roofline_frac": r["step_roofline_frac"],
+            "step_bytes": r["step_bytes"],
             "kernels": r["kernels"], "launch_shape": r["tune"]}
 
 
@@ -579,6 +589,7 @@ def main():
                    "launch_shape": r["tune"], "timed_path": "replayed HIP graphs"},
         "roofline": r["roofline"],
         "step_roofline_frac": r["step_roofline_frac"],
+        "step_bytes": r["step_bytes"],
         "kernels": r["kernels"],
         "kernels_note": r["kernels_note"],
     }

@@ -481,9 +481,8 @@ static int march_rows(long ncol, long ny, long slots) {
 // waves update 60 columns, the sweeps' 63 and 64: in the mixed form, where that
 // counts, not where the grid's width makes it much worse (500x15000 145 / 142,
 // 192 / 176).
-static int step_rows(const hydro_amd_grid* g) {
-  if (!folds_ghosts(g) || g->prof) return 0;  // (profiles are of the sweeps)
-  if (g->tune.step >= 0) return g->tune.step;
+static int default_step(const hydro_amd_grid* g) {
+  if (!folds_ghosts(g)) return 0;
   const long nx = g->p.nx, ny = g->p.ny, ncol = (nx + 59) / 60;
   auto waves = [&](long rows) { return ncol * ((ny + rows - 5) / (rows - 4)) * rows; };
   if (g->prec == HYDRO_AMD_FP64) return waves(8) <= 10000 ? 8 : 0;
@@ -497,6 +496,11 @@ static int step_rows(const hydro_amd_grid* g) {
   return ncol * ny >= 150000 && 100 * 2 * 64 * ncol <= 108 * lanes
              ? kMarch + march_rows(ncol, ny, 5 * kSimds)
              : 0;
+}
+
+static int step_rows(const hydro_amd_grid* g) {
+  if (g->prof) return 0;  // (profiles are of the sweeps)
+  return g->tune.step >= 0 ? g->tune.step : default_step(g);
 }
 
 // hydro_godunov.c:98-237: both directions, ghosts refilled before each, on the
@@ -944,7 +948,7 @@ extern "C" int hydro_amd_grid_autotune(hydro_amd_grid* g, int reps, int* best) {
   HIPCHK(hipStreamSynchronize(g->st));
   if (settle(g)) return -1;
   SweepTune cur = g->tune, bt = g->tune;
-  const int whole = step_rows(g);  // (tried against the sweeps where it is the default)
+  const int whole = default_step(g);  // tried against the sweeps, kept where they can't be timed
   cur.step = bt.step = 0;
   // y sweep: rows per lane (the slab height each column march covers) x
   // waves per workgroup
@@ -1013,6 +1017,7 @@ extern "C" int hydro_amd_grid_autotune(hydro_amd_grid* g, int reps, int* best) {
     t.step = whole;
     combos.push_back(t);
   }
+  bt.step = whole;
   bt = tune_by_steps(g, combos, bt);
   HIPCHK(hipGetLastError());
   g->tune = bt;

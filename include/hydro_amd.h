@@ -107,17 +107,21 @@ int hydro_amd_grid_set_limits(hydro_amd_grid *g, double tend, int nstepmax);
  * lane rotations.  A new grid's shape goes by its size: y rows by the square
  * root of (nx / 64) * ny over 32, between 1 and 64 (32 in the fast form); in x
  * the one-wave form, or the four-wave form on large grids of the fast and
- * mixed forms, and row pieces by the square root of their number. */
+ * mixed forms, and row pieces by the square root of their number.  A new grid
+ * takes whole steps (both sweeps in one launch) instead where they are faster:
+ * small grids, and in the fast and mixed forms large ones; from this call on it
+ * takes the two sweeps. */
 int hydro_amd_grid_set_tune(hydro_amd_grid *g, int yseg, int ywaves, int xwaves, int xiter);
 /* Autotuner: times the candidate launch shapes of both sweeps on this grid
  * (reps launches each, HIP events; the sweeps read the state and write only
- * the scratch buffer, so the state is unchanged), keeps the fastest and
- * caches it per (nx, ny, precision) for the process.  best[4] (may be NULL)
+ * the scratch buffer, so the state is unchanged), then the best against whole
+ * steps, keeps the fastest and caches it per (nx, ny, precision) for the process.  best[4] (may be NULL)
  * receives yseg, ywaves, xwaves, xiter. */
 int hydro_amd_grid_autotune(hydro_amd_grid *g, int reps, int *best);
 /* Kernel timing with HIP events recorded on the grid's own stream around
- * every x-sweep, y-sweep, ghost-fill and CFL launch (graph replay is off
- * while enabled).  set_profile resets the sums; profile returns summed
+ * every x-sweep, y-sweep, ghost-fill and CFL launch (graph replay and whole
+ * steps are off while enabled; ghosts are filled by launches of their own only
+ * on grids narrower than 3 cells).  set_profile resets the sums; profile returns summed
  * milliseconds and launch counts in the order x sweep, y sweep, boundary,
  * CFL (arrays of 4). */
 int hydro_amd_grid_set_profile(hydro_amd_grid *g, int on);
@@ -128,9 +132,10 @@ long long hydro_amd_grid_bytes(const hydro_amd_grid *g);
 /* ---- batches: many independent grids advanced per launch ----------------
  * Each instance is a separate run of the reference time loop (own size,
  * gamma, blast, dt, t, nstep, tend/nstepmax), bit-identical to running it
- * alone with hydro_amd_grid_run.  A phase's launches take their work from task
- * tables mixing the instances' x and y sweeps; two steps are
- * replayed as a HIP graph.  Instances are admitted against an HBM budget
+ * alone with hydro_amd_grid_run.  Launches take their work from task tables
+ * mixing the instances: their x and y sweeps, or, in large loads of the fast
+ * and mixed forms, whole steps.  All but small loads run as two groups of
+ * instances beside each other.  Instances are admitted against an HBM budget
  * (state buffers only) with the stream-ordered allocator, so admission and
  * retirement never synchronise the device.  All instances share one
  * precision. */
@@ -163,8 +168,10 @@ int hydro_amd_batch_query(hydro_amd_batch *b, int *ids, double *t, int *nstep, d
                           int *active, int cap);
 /* Task shape (waves per workgroup 1..4, segments per wave in x tasks, rows per
  * wave in y tasks; without a call 1 wave, and lengths by the live set: the
- * square roots of its segments over 100 and of its 64-column rows over 32)
- * and its autotuner (times the shapes on the live set; state unchanged).
+ * square roots of its segments over 50 and of its 64-column rows over 28;
+ * from a call on, the two sweeps rather than whole steps)
+ * and its autotuner (times the shapes on the live set; state unchanged; a load
+ * that takes whole steps keeps them).
  * best[3] receives waves, xiter, yseg. */
 int hydro_amd_batch_set_tune(hydro_amd_batch *b, int waves, int xiter, int yseg);
 int hydro_amd_batch_autotune(hydro_amd_batch *b, int reps, int *best);
