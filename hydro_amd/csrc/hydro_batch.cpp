@@ -462,7 +462,7 @@ static void shape_by_load(hydro_amd_batch* b) {
     segs += x_segments(p);
     wrows += (long) ((p.nx + 63) / 64) * p.ny;
     mrows += (long) ((p.nx + 59) / 60) * p.ny;
-    fold = fold && folds_ghosts(b->inst[id]);
+    fold = fold && folds_ghosts(b->inst[id]) && p.nx < kMarchWidest;
   }
   auto root = [](long n, double by, int most) {
     return std::max(1, std::min(most, (int) (std::sqrt((double) n) / by + 0.5)));

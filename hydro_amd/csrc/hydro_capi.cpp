@@ -488,12 +488,13 @@ static int default_step(const hydro_amd_grid* g) {
   if (g->prec == HYDRO_AMD_FP64) return waves(8) <= 10000 ? 8 : 0;
   if (g->prec == HYDRO_AMD_FP64_FAST) {
     if (waves(8) <= 16000) return 8;
-    return ncol * ny >= 16000 ? kMarch + march_rows(ncol, ny, 4 * kSimds) : 0;
+    return ncol * ny >= 16000 && nx < kMarchWidest ? kMarch + march_rows(ncol, ny, 4 * kSimds)
+                                                   : 0;
   }
   if (waves(8) <= 5000) return 8;
   if (waves(16) <= 24000) return 16;
   const long lanes = (nx + 251) / 252 * 256 + (nx + 63) / 64 * 64;  // of the sweeps
-  return ncol * ny >= 150000 && 100 * 2 * 64 * ncol <= 108 * lanes
+  return ncol * ny >= 150000 && nx < kMarchWidest && 100 * 2 * 64 * ncol <= 108 * lanes
              ? kMarch + march_rows(ncol, ny, 5 * kSimds)
              : 0;
 }

@@ -73,6 +73,8 @@ struct SweepTune {
                 // the grid's size
 };
 constexpr int kMarch = 32;
+// Widest grid of the march (its lanes' offsets in a row are 32 bits of bytes).
+constexpr int kMarchWidest = 1 << 28;
 constexpr int kSimds = 1024;  // of the GPU: 256 CUs of 4
 
 // ---- launchers (hydro_kernels.hip) -----------------------------------------

@@ -39,6 +39,27 @@ __device__ __forceinline__ void st_stream(S* p, S v) {
   __builtin_nontemporal_store(v, p);
 }
 
+// Element `off` bytes past a wave-uniform address: the address stays in scalar
+// registers and the access takes the lane's 32-bit offset (a 64-bit address a
+// lane and variable cost the y march 16 vector instructions a row of 290 in the
+// mixed form; a step of 4099x3001 without them: fast 287 and 280-285 us, mixed 202
+// and 197, FP64 567 and 563; 8192x8192 FP64 2.775 and 2.74-2.77 ms).
+template <typename S>
+__device__ __forceinline__ S ld_lane(const S* base, unsigned off) {
+  return *reinterpret_cast<const S*>(reinterpret_cast<const char*>(base) + off);
+}
+template <typename S>
+__device__ __forceinline__ S* at_lane(S* base, unsigned off) {
+  return reinterpret_cast<S*>(reinterpret_cast<char*>(base) + off);
+}
+
+// The same offset, in a form that the compiler cannot fold into addresses of its
+// own kept from one row to the next (eight registers a set of planes).
+__device__ __forceinline__ unsigned lane_off(unsigned off) {
+  asm volatile("" : "+v"(off));
+  return off;
+}
+
 // ---- lane exchange -----------------------------------------------------------
 
 // lane l receives the value of lane l-1 (DPP wave_ror:1, so lane 0 receives
@@ -250,10 +271,23 @@ __device__ __forceinline__ void x_segment_at(const GridGeom& g, const Phys<S>& p
   const long j = jrow + 2;
   const int i = kXSeg * seg + lane;  // padded column of this lane
   // (o is its own cell where it is updated)
-  const long o = j * g.pitch + (EDGE ? x_source(g, gf, i, true) : i);
-  const S U0 = in.p[0][o], U2 = in.p[2][o], U3 = in.p[3][o];
-  S U1 = in.p[1][o];
-  if (EDGE) x_ghost<S>(g, in, out, gf, o, i, U0, U1, U2, U3);
+  const long row = j * g.pitch + kXSeg * seg;  // wave-uniform
+  const unsigned vo = lane_off((unsigned) (lane * sizeof(S)));
+  long o = 0;
+  S U0, U1, U2, U3;
+  if constexpr (EDGE) {
+    o = j * g.pitch + x_source(g, gf, i, true);
+    U0 = in.p[0][o];
+    U1 = in.p[1][o];
+    U2 = in.p[2][o];
+    U3 = in.p[3][o];
+    x_ghost<S>(g, in, out, gf, o, i, U0, U1, U2, U3);
+  } else {
+    U0 = ld_lane(in.p[0] + row, vo);
+    U1 = ld_lane(in.p[1] + row, vo);
+    U2 = ld_lane(in.p[2] + row, vo);
+    U3 = ld_lane(in.p[3] + row, vo);
+  }
   Prim<S> pc;
   bool fc = false;
   if constexpr (FD == kFast) {
@@ -284,10 +318,10 @@ __device__ __forceinline__ void x_segment_at(const GridGeom& g, const Phys<S>& p
   const double n2 = update1<S>(U2, fl.v, fr.v, dtdx);
   const double n3 = update1<S>(U3, fl.p, fr.p, dtdx);
   if (wr) {
-    out.p[0][o] = (S) n0;
-    out.p[1][o] = (S) n1;
-    out.p[2][o] = (S) n2;
-    out.p[3][o] = (S) n3;
+    *at_lane(out.p[0] + row, vo) = (S) n0;
+    *at_lane(out.p[1] + row, vo) = (S) n1;
+    *at_lane(out.p[2] + row, vo) = (S) n2;
+    *at_lane(out.p[3] + row, vo) = (S) n3;
     if (COUR) {
       S ax, ay;
       courant_cell<S, FD>((S) n0, (S) n1, (S) n2, (S) n3, ph, ax, ay);
@@ -531,9 +565,11 @@ __device__ __forceinline__ Cell<S> stash_get_cell(const S (&b)[4][64], int lane)
 }
 
 template <typename S>
-__device__ __forceinline__ Cell<S> load_y(const GridView<S>& in, long o) {
+__device__ __forceinline__ Cell<S> load_y(const GridView<S>& in, long row, unsigned off) {
   // gather with the IU/IV swap of conservar.c:106-109
-  return Cell<S>{in.p[0][o], in.p[2][o], in.p[1][o], in.p[3][o]};
+  off = lane_off(off);
+  return Cell<S>{ld_lane(in.p[0] + row, off), ld_lane(in.p[2] + row, off),
+                 ld_lane(in.p[1] + row, off), ld_lane(in.p[3] + row, off)};
 }
 
 // As x_ghost, for column i of padded row j (wave-uniform).
@@ -563,6 +599,9 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
   const long P = g.pitch;
   const int lane = threadIdx.x & 63;
   const bool o1 = ph.iorder == 1;
+  // lane 0's column (wave-uniform), and this lane's offset from it
+  const long i0 = __builtin_amdgcn_readfirstlane((int) i);
+  const unsigned vo = (unsigned) ((i - i0) * (long) sizeof(S));
 
   // prologue: cells j0-2 .. j0+1
   // (a ghost row is read at its source and made a ghost where it is used)
@@ -574,10 +613,10 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
   const int s3 = ghost_source(2, g.ny, gf.lo, gf.hi, top + 1, neg);
   auto load = [&](int j) {
     const int js = j >= top ? (j == top ? s2 : s3) : j;
-    return load_y<S>(in, (long) js * P + i);
+    return load_y<S>(in, (long) js * P + i0, vo);
   };
-  Cell<S> ua = load_y<S>(in, (long) (j0 == 2 ? s0 : j0 == 3 ? s1 : j0 - 2) * P + i);
-  Cell<S> ub = load_y<S>(in, (long) (j0 == 2 ? s1 : j0 - 1) * P + i);
+  Cell<S> ua = load_y<S>(in, (long) (j0 == 2 ? s0 : j0 == 3 ? s1 : j0 - 2) * P + i0, vo);
+  Cell<S> ub = load_y<S>(in, (long) (j0 == 2 ? s1 : j0 - 1) * P + i0, vo);
   Cell<S> uc = load(j0);
   Cell<S> ud = load(j0 + 1);
   if (j0 < 4) {
@@ -635,7 +674,7 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
     // (the compiler must read the slots the previous row wrote, not forward
     // the values in registers)
     asm volatile("" ::: "memory");
-    const long oc = (long) (j - 2) * P + i;
+    const long oc = (long) (j - 2) * P + i0;
     Cell<S> uE = uN;
     if (j >= top) y_ghost<S>(g, in, out, gf, colok, j, i, uE);
     const int sj = j % 3;  // wave-uniform
@@ -666,10 +705,11 @@ __device__ __forceinline__ void y_march(const GridGeom& g, const Phys<S>& ph,
     const double n3 = update1<S>(uC.u3, fprev.p, fcur.p, dtdx);
     if (colok) {
       // scatter back with the swap undone (conservar.c:177-180)
-      st_stream(&out.p[0][oc], (S) n0);
-      st_stream(&out.p[2][oc], (S) n1);
-      st_stream(&out.p[1][oc], (S) n2);
-      st_stream(&out.p[3][oc], (S) n3);
+      const unsigned so = lane_off(vo);
+      st_stream(at_lane(out.p[0] + oc, so), (S) n0);
+      st_stream(at_lane(out.p[2] + oc, so), (S) n1);
+      st_stream(at_lane(out.p[1] + oc, so), (S) n2);
+      st_stream(at_lane(out.p[3] + oc, so), (S) n3);
       if (COUR) {
         S ax, ay;
         courant_cell<S, FD>((S) n0, (S) n2, (S) n1, (S) n3, ph, ax, ay);
@@ -918,6 +958,9 @@ __device__ __forceinline__ void step_march(const GridGeom& g, const Phys<S>& ph,
       gx = is != i && i == ic;
     }
   }
+  // (rows of less than 4 GB: kMarchWidest)
+  const unsigned vi = (unsigned) is * (unsigned) sizeof(S);
+  const unsigned vo = (unsigned) i * (unsigned) sizeof(S);
   bool neg;
   const int s0 = ghost_source(2, g.ny, bd, bu, 0, neg);
   const int s1 = ghost_source(2, g.ny, bd, bu, 1, neg);
@@ -927,15 +970,18 @@ __device__ __forceinline__ void step_march(const GridGeom& g, const Phys<S>& ph,
     // (values, not references: a selected address would keep them in memory)
     int js = j < 2 ? (j == 0 ? +s0 : +s1) : j;
     if (j >= top) js = j == top ? +s2 : +s3;
-    const long o = (long) js * P + is;
-    return TCell<S>{in.p[0][o], in.p[1][o], in.p[2][o], in.p[3][o]};
+    const long row = (long) js * P;
+    const unsigned lo = lane_off(vi);
+    return TCell<S>{ld_lane(in.p[0] + row, lo), ld_lane(in.p[1] + row, lo),
+                    ld_lane(in.p[2] + row, lo), ld_lane(in.p[3] + row, lo)};
   };
   auto store = [&](int j, const TCell<S>& v) {
-    const long o = (long) j * P + i;
-    st_stream(&out.p[0][o], v.r);
-    st_stream(&out.p[1][o], v.mx);
-    st_stream(&out.p[2][o], v.my);
-    st_stream(&out.p[3][o], v.e);
+    const long row = (long) j * P;
+    const unsigned so = lane_off(vo);
+    st_stream(at_lane(out.p[0] + row, so), v.r);
+    st_stream(at_lane(out.p[1] + row, so), v.mx);
+    st_stream(at_lane(out.p[2] + row, so), v.my);
+    st_stream(at_lane(out.p[3] + row, so), v.e);
   };
   const Q4<S> z = {(S) 0, (S) 0, (S) 0, (S) 0};
   // window: C = row j-2 (being updated), D = row j-1, as in y_march
