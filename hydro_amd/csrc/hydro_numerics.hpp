@@ -42,8 +42,6 @@ struct Phys {
   R slope_inv;    // 1 / slope_type (the FP64 fast form's slopes)
   double smallr_inv;  // 1 / smallr (the FP64 fast form's star state)
   double gamma_d, gamma6_d, smallp_d, smallpp_d;  // Newton constants (double)
-  double gammap_d;    // (gamma + 1) / 2 (the FP64 fast form's Newton iteration)
-  double enthp_d;     // gamma / (gamma - 1) (the FP64 fast form's flux)
   int niter;      // niter_riemann
   int iorder;     // 1: first order (dq = 0)
   int scheme;     // 1 muscl, 2 plmde, 3 collela
@@ -69,8 +67,6 @@ __host__ __device__ inline Phys<R> make_phys(double gamma, double smallr, double
   p.gamma6_d = (gamma + 1.0) / (2.0 * gamma);
   p.smallp_d = (smallc * smallc) / gamma;
   p.smallpp_d = smallr * p.smallp_d;
-  p.gammap_d = 0.5 * (gamma + 1.0);
-  p.enthp_d = gamma / (gamma - 1.0);
   p.niter = niter;
   p.iorder = iorder;
   p.scheme = scheme;
@@ -270,9 +266,9 @@ __device__ __forceinline__ void xsqrt2(float a, float b, float& sa, float& sb) {
   sb = __builtin_amdgcn_sqrtf(b);
 }
 
-// FP64 reciprocals and reciprocal square roots (x > 0) of the Newton iteration
-// in the mixed and fast forms: the hardware estimates v_rcp_f64 / v_rsq_f64
-// refined by one Newton-Raphson step each, relative error about 2^-47 -- far
+// FP64 reciprocals and square roots (x > 0) of the Newton iteration in the mixed
+// and fast forms: the hardware estimates v_rcp_f64 / v_rsq_f64 refined by one
+// Newton-Raphson (or Goldschmidt) step each, relative error about 2^-47 -- far
 // below the iteration's 1e-6 tolerance and the FP32 rounding of the mixed
 // form's result.
 __device__ __forceinline__ double rcp_nr(double b) {
@@ -283,6 +279,15 @@ __device__ __forceinline__ double rsq_nr(double x) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = __builtin_fma(-(x * y), y, 1.0);
   return __builtin_fma(0.5 * y, e, y);
+}
+// sqrt(x) and 1/sqrt(x) from one v_rsq_f64 estimate g: with s = x g and the
+// residual r = 1/2 - s g/2, one Goldschmidt step gives s + s r and g + g r.
+__device__ __forceinline__ void sqrt_rsq_nr(double x, double& s, double& is) {
+  const double g = __builtin_amdgcn_rsq(x);
+  const double s0 = x * g;
+  const double r = __builtin_fma(-(g * 0.5), s0, 0.5);
+  s = __builtin_fma(s0, r, s0);
+  is = __builtin_fma(g, r, g);
 }
 // constoprim.c:62-78 + equation_of_state.c:64-81 for one cell.  U is in sweep
 // slot order (slot 1 = normal momentum).  FAST (FP64, for cells that passed
@@ -353,52 +358,43 @@ __device__ __forceinline__ bool wave_cell_in(S U0, S U1, S U2, S U3, const Phys<
 //
 // Quotients and square roots from the hardware estimates v_rcp_f64 and
 // v_rsq_f64 (relative error about 2^-24, measured on MI355X) refined by
-// one step instead of the correctly rounded sequences: of third order (rcp2,
-// sqrt_rsq2, sqrt_1ulp), which leaves a result within about an ulp, and
-// divisions by one denominator share its reciprocal.  Inside the Newton
-// pressure iteration a Newton-Raphson step (rcp_nr, rsq_nr: about 2^-47) is
-// enough except in the last iteration the
+// Newton-Raphson or coupled Goldschmidt steps instead of the correctly
+// rounded sequences: two steps (rcp2, sqrt_rsq2, sqrt_1ulp) leave a result
+// within about an ulp, and divisions by one denominator share its
+// reciprocal.  Inside the Newton pressure iteration one step (rcp_nr,
+// sqrt_rsq_nr: about 2^-48) is enough except in the last iteration the
 // limit allows: an error in an iterate is damped by the next Newton step, so
 // p* carries only the error of its last correction, below 1e-6 of p* when
 // the face converged, and a face stopped by the limit takes that last step
-// with the third-order ones.
+// with the two-step estimates.
 
-// One step of third order does what two of second order would: with e = 1 - b y,
-// 1 / b = y (1 + e + e^2 + ..), with e = 1 - x y^2, 1 / sqrt(x) =
-// y (1 + e / 2 + 3 e^2 / 8 + ..); what is left out is below 2^-68.  Mean and
-// largest error over 4e6 arguments in 2^[-60, 60], in ulps: rcp2 0.250 and 0.50
-// (two steps: the same), sqrt_rsq2's root 0.271 and 0.75 (0.311 and 1.45), its
-// reciprocal root 0.278 and 1.00 (0.315 and 1.63).
-
-// 1/b.
+// 1/b within about an ulp: the estimate and two Newton-Raphson steps.
 __device__ __forceinline__ double rcp2(double b) {
-  const double y = __builtin_amdgcn_rcp(b);
-  const double e = __builtin_fma(-b, y, 1.0);
-  return __builtin_fma(y, __builtin_fma(e, e, e), y);
+  const double y0 = __builtin_amdgcn_rcp(b);
+  const double y1 = __builtin_fma(__builtin_fma(-b, y0, 1.0), y0, y0);
+  return __builtin_fma(__builtin_fma(-b, y1, 1.0), y1, y1);
 }
-// sqrt(x) and 1/sqrt(x) for x > 0.
+// sqrt(x) and 1/sqrt(x) for x > 0, both within about an ulp: two coupled
+// Goldschmidt steps from one v_rsq_f64 estimate g (s = x g, h = g / 2,
+// r = 1/2 - s h, then s += s r, h += h r).
 __device__ __forceinline__ void sqrt_rsq2(double x, double& s, double& is) {
-  const double y = __builtin_amdgcn_rsq(x), a = x * y;
-  const double e = __builtin_fma(-a, y, 1.0);
-  const double q = e * __builtin_fma(e, 0.375, 0.5);
-  s = __builtin_fma(a, q, a);
-  is = __builtin_fma(y, q, y);
+  const double g = __builtin_amdgcn_rsq(x);
+  const double s0 = x * g, h0 = 0.5 * g;
+  const double r0 = __builtin_fma(-h0, s0, 0.5);
+  const double s1 = __builtin_fma(s0, r0, s0), h1 = __builtin_fma(h0, r0, h0);
+  const double r1 = __builtin_fma(-h1, s1, 0.5);
+  s = __builtin_fma(s1, r1, s1);
+  is = 2.0 * __builtin_fma(h1, r1, h1);
 }
-// sqrt(x) for x >= 0, within half an ulp (to 3 digits): one coupled
-// Goldschmidt step, then a residual correction (sqrt(+0) gives NaN here;
-// callers clamp the result with fmax, which returns the other operand for a
-// NaN).
+// sqrt(x) for x >= 0 within about an ulp: one coupled step, then a residual
+// correction (sqrt(+0) gives NaN here; callers clamp the result with fmax,
+// which returns the other operand for a NaN).
 __device__ __forceinline__ double sqrt_1ulp(double x) {
   const double g = __builtin_amdgcn_rsq(x);
   const double s0 = x * g, h0 = 0.5 * g;
   const double r0 = __builtin_fma(-h0, s0, 0.5);
   const double s1 = __builtin_fma(s0, r0, s0), h1 = __builtin_fma(h0, r0, h0);
   return __builtin_fma(__builtin_fma(-s1, s1, x), h1, s1);
-}
-__device__ __forceinline__ double rsq2(double x) {
-  double s, is;
-  sqrt_rsq2(x, s, is);
-  return is;
 }
 
 // constoprim.c:62-78 + equation_of_state.c:64-81 for one cell, fast form:
@@ -412,8 +408,10 @@ __device__ __forceinline__ Prim<double> prim_fast(double U0, double U1, double U
   const double r = fmax(U0, ph.smallr);
   const double ir = rcp2(r);
   const double u = U1 * ir, v = U2 * ir;
-  // gm1 * rho * (E / rho - (u^2 + v^2) / 2) without the way by 1 / rho
-  const double p = fmax(ph.gm1 * (U3 - 0.5 * (U1 * u + U2 * v)), r * ph.smallp);
+  const double eken = 0.5 * (u * u + v * v);
+  const double e = U3 * ir - eken;
+  double p = ph.gm1 * r * e;
+  p = fmax(p, r * ph.smallp);
   sqrt_rsq2(ph.gamma * p * ir, o.c, o.cinv);  // gamma p / rho > 0
   o.q = Q4<double>{r, u, v, p};
   o.rinv = ir;
@@ -875,11 +873,10 @@ __device__ __forceinline__ void trace_fast(const Q4<R>& q, const Q4<R>& dq, R cc
 
 // riemann.c:128-276 + cmpflx.c:67-90 for one face, fast form.  The first
 // guess and the Newton iteration are the reference's recurrence with fewer
-// divisions (as in the mixed form, here in FP64 throughout): with cl =
-// gamma pl rl, w^2 = cl (1 + gamma6 (p* - pl) / pl) is cl + (p* - pl) rl
-// (gamma + 1) / 2; w is needed only as 1/w, from its estimate; with 1 / q =
-// (w^2 + c) / (2 w^3) = (1 + c / w^2) / (2 w), qr ql / (qr + ql) is the
-// reciprocal of 1 / ql + 1 / qr; and |d / (p* + smallpp)| > 1e-6 is tested as
+// divisions (as in the mixed form, here in FP64 throughout): 1/pl and 1/pr
+// are loop invariants, 1/w comes from the estimate that gives w, with
+// q = a / b (a = 2 w^3, b = w^2 + c) qr ql / (qr + ql) = al ar / (al br +
+// ar bl) is one division, and |d / (p* + smallpp)| > 1e-6 is tested as
 // |d| > 1e-6 (p* + smallpp).  In the star state, sqrt(gamma po / ro) is
 // sqrt(gamma po ro) / ro with sqrt(gamma po ro) from the first guess; with
 // rstar = ro / X, one reciprocal of ro X gives 1/ro, 1/X and 1/rstar (1/smallr
@@ -904,28 +901,31 @@ __device__ __forceinline__ Q4<double> riemann_fast(const Q4<double>& ql, const Q
   sqrt_rsq2(cr, wr0, iwr0);
   double pst = fmax(((wr0 * pl + wl0 * pr) + wl0 * wr0 * (ul - ur)) * rcp2(wl0 + wr0), 0.0);
 
-  // Newton iteration (riemann.c:160-201): 30 operations a pass, 42 with w, w^3
-  // and q formed (a step of 2048x1536 with this and the shorter roots 98 us,
-  // 106 before; of 8192x1024 245 / 255; of 8192x8192, where memory bounds it, 1.78 /
-  // 1.81 ms).  The last iteration the limit
+  // Newton iteration (riemann.c:160-201).  The last iteration the limit
   // allows takes the estimates refined to an ulp: when a face stops there
   // unconverged, that step's correction is not damped by a later one.
-  const double gl = ph.gammap_d * rl, gr_ = ph.gammap_d * rr;
+  const double g6 = ph.gamma6_d;
+  const double ipl = rcp2(pl), ipr = rcp2(pr);
+  const double gpl = g6 * ipl, gpr = g6 * ipr;
   for (int it = 0; it < ph.niter; it++) {
     const bool last = it + 1 == ph.niter;  // wave-uniform
-    double iwl, iwr;
-    const double tl = pst - pl, tr = pst - pr;
-    const double xl = cl + tl * gl, xr = cr + tr * gr_;
+    const double xl = cl * (1.0 + (pst - pl) * gpl), xr = cr * (1.0 + (pst - pr) * gpr);
+    double wwl, iwl, wwr, iwr;
     if (!last) {
-      iwl = rsq_nr(xl);
-      iwr = rsq_nr(xr);
+      sqrt_rsq_nr(xl, wwl, iwl);
+      sqrt_rsq_nr(xr, wwr, iwr);
     } else {
-      iwl = rsq2(xl);
-      iwr = rsq2(xr);
+      sqrt_rsq2(xl, wwl, iwl);
+      sqrt_rsq2(xr, wwr, iwr);
     }
-    const double qi = iwl * (1.0 + cl * (iwl * iwl)) + iwr * (1.0 + cr * (iwr * iwr));
-    const double qq = last ? rcp2(qi) : rcp_nr(qi);
-    const double t = 2.0 * (((ul - tl * iwl) - (ur + tr * iwr)) * qq);
+    const double swl = wwl * wwl, swr = wwr * wwr;
+    const double al = 2.0 * wwl * swl, bl = swl + cl;
+    const double ar = 2.0 * wwr * swr, br = swr + cr;
+    const double usl = ul - (pst - pl) * iwl;
+    const double usr = ur + (pst - pr) * iwr;
+    const double den = al * br + ar * bl;
+    const double rden = last ? rcp2(den) : rcp_nr(den);
+    const double t = ((al * ar) * rden) * (usl - usr);
     const double d = fmax(t, -pst);  // (t > -pst ? t : -pst for every pst that is not NaN)
     pst += d;
     if (!(fabs(d) > 1e-6 * (pst + ph.smallpp_d))) break;
@@ -933,8 +933,9 @@ __device__ __forceinline__ Q4<double> riemann_fast(const Q4<double>& ql, const Q
 
   // star state and sampling at x/t = 0 (riemann.c:211-276)
   const double ps = pst;
-  const double xl = cl + (ps - pl) * gl, xr = cr + (ps - pr) * gr_;
-  const double iwl = rsq2(xl), iwr = rsq2(xr);
+  double wl, iwl, wr, iwr;
+  sqrt_rsq2(cr * (one + (ps - pr) * gpr), wr, iwr);
+  sqrt_rsq2(cl * (one + (ps - pl) * gpl), wl, iwl);
   // ((ul + (pl-ps)/wl) + ur) - (pr-ps)/wr, the reference's left-to-right sum
   const double ustar = half * (((ul + (pl - ps) * iwl) + ur) - (pr - ps) * iwr);
   const bool left = ustar > 0.0;
@@ -942,8 +943,8 @@ __device__ __forceinline__ Q4<double> riemann_fast(const Q4<double>& ql, const Q
   const double ro = left ? rl : rr;
   const double uo = left ? ul : ur;
   const double po = left ? pl : pr;
+  const double wo = left ? wl : wr;
   const double iwo = left ? iwl : iwr;
-  const double wo = (left ? xl : xr) * iwo;
   const double wo0 = left ? wl0 : wr0;
   // rstar = ro / X: one reciprocal of ro X gives 1/ro, 1/X and 1/rstar
   const double X = one + ro * (po - ps) * (iwo * iwo);
@@ -986,13 +987,15 @@ __device__ __forceinline__ Q4<double> riemann_fast(const Q4<double>& ql, const Q
   f.r = m;
   f.u = m * gu + gp;
   f.v = m * gv;
-  f.p = gu * (half * gr * (gu * gu + gv * gv) + gp * ph.enthp_d);
+  const double ekin = half * gr * (gu * gu + gv * gv);
+  const double etot = gp * ph.entho + ekin;
+  f.p = gu * (etot + gp);
   return f;
 }
 
 // The mixed-precision form (R = float) of riemann_flux: FP32 inputs, first
 // guess and star state, the Newton iteration in FP64 with the refined
-// hardware estimates (rcp_nr, rsq_nr).
+// hardware estimates (div_nr, rcp_nr, sqrt_rsq_nr).
 template <typename R>
 __device__ __forceinline__ Q4<R> riemann_flux_mixed(const Q4<R>& ql, const Q4<R>& qr,
                                                     const Phys<R>& ph) {
@@ -1008,12 +1011,17 @@ __device__ __forceinline__ Q4<R> riemann_flux_mixed(const Q4<R>& ql, const Q4<R>
   R cr = ph.gamma * pr * rr;
 
   // First guess and Newton iteration for p* (riemann.c:145-201), in double.
-  // The iteration is the reference's recurrence rearranged as in riemann_fast
-  // (p* >= 0, smallpp > 0), but for w^2, as the star state takes gamma6 / pl
-  // too.  A step of 8192x8192 with it 1.00 ms, 1.03 before, of 4099x3001 208 and
-  // 214 us.  (gamma6 cl / pl kept through the loop took the small grids' kernel
-  // past 64 registers, a step of 1021x767 from 29.7 to 37 us; one reciprocal of
-  // pl pr for both was slower by 1 %: a longer chain.)
+  // The iteration is the reference's recurrence rearranged to fewer
+  // operations: 1/pl and 1/pr are loop invariants; w is used as 1/w alone; with
+  // 1 / q = (w^2 + c) / (2 w^3) = (1 + c / w^2) / (2 w), qr ql / (qr + ql) is the
+  // reciprocal of 1 / ql + 1 / qr; |d / (p* + smallpp)| > 1e-6 is tested as
+  // |d| > 1e-6 (p* + smallpp) (p* >= 0, smallpp > 0).  An iterate's rounding is
+  // far below the FP32 result's: the same states as with w, w^3 and q formed, bit
+  // for bit, over 16 flows of up to 6000x5000 cells.  A step of 8192x8192 with it
+  // 1.00 ms, 1.03 before, of 4099x3001 208 and 214 us.  (gamma6 cl / pl kept
+  // through the loop took the small grids' kernel past 64 registers, a step of
+  // 1021x767 from 29.7 to 37 us; one reciprocal of pl pr for both was slower by
+  // 1 %: a longer chain.)
   // The first guess (riemann.c:145-150) is the iteration's starting point
   // and is formed in FP32: a Newton step squares its relative error (1e-7 ->
   // 1e-14), so the FP64 iterate it reaches is as accurate as from an FP64
