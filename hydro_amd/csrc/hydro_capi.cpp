@@ -660,8 +660,10 @@ static int run_enqueue(hydro_amd_grid* g, int max_steps, int log_cap,
                        hipEvent_t start = nullptr) {
   if (max_steps <= 0) return 0;
   if (settle(g)) return -1;  // the step parity below is the mirror's
-  // dt of an even step comes from the CFL maxima of the current state
+  // dt of an even step comes from the CFL maxima of the current state; an odd
+  // step folds its maxima into slots that hold no other state's
   if (g->nstep % 2 == 0) ensure_cour(g);
+  else prepare_slots(g);
   // control, log setup + limits
   HIPCHK(hipStreamSynchronize(g->st));  // the pinned copy may still feed a queued copy
   RunCtl c{};
