@@ -318,6 +318,7 @@ static int run_finish(hydro_amd_grid* g, int* steps_done);
 static int settle(hydro_amd_grid* g) { return g->queued ? run_finish(g, nullptr) : 0; }
 
 static int do_init(hydro_amd_grid* g, int bx, int by0, int by1, double e) {
+  if (settle(g)) return -1;  // (queued steps may leave maxima in the CFL slots)
   if (dbl(g))
     launch_init<double>(g->geom, g->vd[0], g->vd[1], bx, by0, by1, e, g->st);
   else

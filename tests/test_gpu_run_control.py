@@ -49,3 +49,15 @@ def test_odd_step_after_another_run(nx, ny, before):
         g.upload(u)
         g.set_state(0.25, 3, 1e-4)
         check(g, p, u, (0.25, 3, 1e-4), 6)
+
+
+@pytest.mark.parametrize("nx,ny", SIZES)
+def test_new_state_over_queued_steps(nx, ny):
+    p = params(nx, ny)
+    weak = (nx // 3, ny // 3, 1e-3 / p.dx / p.dx)
+    with hydro_amd.Grid(p) as g:
+        g.init_blast(nx // 2, ny // 2, 1.0 / p.dx / p.dx)
+        g.run(1)
+        g.run_async(1)  # the odd step, whose maxima are in the slots when it is done
+        g.init_blast(*weak)
+        check(g, p, oracle.Port().init_blast(to_oracle(p), *weak), None, 5)
