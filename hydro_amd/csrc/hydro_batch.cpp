@@ -908,21 +908,24 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
     forced[id].fault = 0;
     if (!(forced[id].dt > 0)) forced[id].dt = 1e-12;
   }
-  BCHK(hipMemcpy(b->ctl, forced.data(), sizeof(RunCtl) * nc, hipMemcpyHostToDevice));
   const BatchTune keep = b->tune;
   BatchTune bt = keep;
   double bms = 1e30;
-  hipEvent_t e0, e1;
-  BCHK(hipEventCreate(&e0));
-  BCHK(hipEventCreate(&e1));
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  hipError_t err = hipEventCreate(&e0);
+  if (err == hipSuccess) err = hipEventCreate(&e1);
+  // (from here to their restoration nothing returns: a control left active would
+  // be closed as a step that ran)
+  if (err == hipSuccess)
+    err = hipMemcpy(b->ctl, forced.data(), sizeof(RunCtl) * nc, hipMemcpyHostToDevice);
   // around the shape that goes by the load
   b->tune = BatchTune{1, 0, 0};
   shape_by_load(b);
   const int rx = b->xiter, ry = b->yseg;
   for (int w : {1, 2, 4})
-    for (int xi : {std::max(1, rx / 2), rx, 2 * rx})
+    for (int xi : {std::max(1, rx / 2), rx, 2 * rx})  // (none once err is set)
       for (int ys : {std::max(1, ry / 2), ry, 2 * ry}) {
-        if (hydro_amd_batch_set_tune(b, w, xi, ys) || rebuild(b)) break;
+        if (err != hipSuccess || hydro_amd_batch_set_tune(b, w, xi, ys) || rebuild(b)) break;
         for (int r = -1; r < reps; r++) {  // r = -1 warms up
           if (r == 0) (void) hipEventRecord(e0, b->st);
           // every x and y list at phase 0: reads buffer 0, writes buffer 1 only
@@ -943,12 +946,15 @@ extern "C" int hydro_amd_batch_autotune(hydro_amd_batch* b, int reps, int* best)
           bt = b->tune;
         }
       }
-  (void) hipEventDestroy(e0);
-  (void) hipEventDestroy(e1);
-  BCHK(hipMemcpy(b->ctl, saved.data(), sizeof(RunCtl) * nc, hipMemcpyHostToDevice));
-  if (bms == 1e30) {  // nothing could be timed
+  for (hipEvent_t e : {e0, e1})
+    if (e) (void) hipEventDestroy(e);
+  const hipError_t back =
+      hipMemcpy(b->ctl, saved.data(), sizeof(RunCtl) * nc, hipMemcpyHostToDevice);
+  if (err == hipSuccess) err = back;
+  if (err != hipSuccess || bms == 1e30) {  // nothing could be timed
     b->tune = keep;
     b->dirty = true;
+    BCHK(err);
   } else if (hydro_amd_batch_set_tune(b, bt.waves, bt.xiter, bt.yseg)) {
     return -1;
   }
