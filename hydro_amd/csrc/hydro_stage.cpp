@@ -10,7 +10,8 @@
 // cut into slabs of rows that up to kLanes threads carry, each through two
 // buffers of its own, the DMA of one beside the host copy of the other.
 // 8192x8192 FP64 download: 153 ms with one thread, 54 with eight; 1021x767
-// upload 28.4 ms through hipMemcpy2D, 0.8 so.
+// upload 28.4 ms through hipMemcpy2D, 0.8 so.  Where no pinned memory can be had,
+// the rows go through hipMemcpy2D all the same.
 #include <hip/hip_runtime.h>
 
 #include <pthread.h>
@@ -18,7 +19,9 @@
 
 #include <algorithm>
 #include <atomic>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 
 #include "hydro_kernels.hpp"
@@ -56,7 +59,7 @@ void lane_free(Lane& l) {
   l = Lane();
 }
 
-// At least one lane, up to n; how many there are.
+// Up to n lanes; how many there are (0: no pinned memory).
 int lanes_for(int n) {
   for (; g_stage.ready < n; g_stage.ready++) {
     Lane& l = g_stage.lane[g_stage.ready];
@@ -140,10 +143,65 @@ struct Block {
   hipStream_t st;
 };
 
+// `nr` host rows from row r0 on into (up) or out of a buffer of such rows.
+void host_rows(const Block& b, bool up, void* buf, long r0, long nr) {
+  const size_t row_bytes = (size_t) b.width * b.desz;
+  char* h = b.host + (size_t) r0 * b.hpitch * b.hesz;
+  if (b.hpitch == b.width) {
+    const size_t m = (size_t) nr * b.width;
+    if (up) convert(buf, b.desz, h, b.hesz, m);
+    else convert(h, b.hesz, buf, b.desz, m);
+    return;
+  }
+  for (long r = 0; r < nr; r++) {
+    char* hr = h + (size_t) r * b.hpitch * b.hesz;
+    char* br = (char*) buf + (size_t) r * row_bytes;
+    if (up) convert(br, b.desz, hr, b.hesz, b.width);
+    else convert(hr, b.hesz, br, b.desz, b.width);
+  }
+}
+
+// Queues the copy of `nr` rows between the device and host memory at `buf`,
+// whose rows are `pitch` bytes apart.
+hipError_t copy_rows(const Block& b, bool up, void* buf, size_t pitch, long r0, long nr) {
+  const size_t w = (size_t) b.width * b.desz, dp = (size_t) b.dpitch * b.desz;
+  char* d = b.dev + (size_t) r0 * dp;
+  return up ? hipMemcpy2DAsync(d, dp, buf, pitch, w, nr, hipMemcpyHostToDevice, b.st)
+            : hipMemcpy2DAsync(buf, pitch, d, dp, w, nr, hipMemcpyDeviceToHost, b.st);
+}
+
+int copy_error(bool up) {
+  return hydro_amd_set_error("%s copy failed", up ? "host-to-device" : "device-to-host");
+}
+
+// Without pinned memory: straight between the caller's array and the device, or
+// slab by slab through pageable memory where the elements are converted.
+int copy_pageable(const Block& b, bool up) {
+  const size_t row_bytes = (size_t) b.width * b.desz;
+  if (b.hesz == b.desz) {
+    if (copy_rows(b, up, b.host, (size_t) b.hpitch * b.hesz, 0, b.rows) != hipSuccess ||
+        hipStreamSynchronize(b.st) != hipSuccess)
+      return copy_error(up);
+    return 0;
+  }
+  const long per = std::max(1L, std::min((long) (kSlabBytes / row_bytes), b.rows));
+  std::unique_ptr<char[]> buf(new (std::nothrow) char[(size_t) per * row_bytes]);
+  if (!buf) return hydro_amd_set_error("staging allocation failed");
+  for (long r0 = 0; r0 < b.rows; r0 += per) {
+    const long nr = std::min(per, b.rows - r0);
+    if (up) host_rows(b, up, buf.get(), r0, nr);
+    if (copy_rows(b, up, buf.get(), row_bytes, r0, nr) != hipSuccess ||
+        hipStreamSynchronize(b.st) != hipSuccess)
+      return copy_error(up);
+    if (!up) host_rows(b, up, buf.get(), r0, nr);
+  }
+  return 0;
+}
+
 int copy_block(const Block& b, bool up) {
   const size_t row_bytes = (size_t) b.width * b.desz;
   int n = lanes_for(thread_count((size_t) b.width * b.rows * b.hesz));
-  if (n < 1) return hydro_amd_set_error("pinned staging allocation failed");
+  if (n < 1) return copy_pageable(b, up);
   // slabs small enough that every thread has two or more
   const long per = std::max(1L, std::min((long) (kSlabBytes / row_bytes),
                                          (b.rows + 2L * n - 1) / (2L * n)));
@@ -152,21 +210,6 @@ int copy_block(const Block& b, bool up) {
   int dev = 0;
   (void) hipGetDevice(&dev);
   std::atomic<int> bad{0};
-  auto host_copy = [&](void* buf, long r0, long nr) {
-    char* h = b.host + (size_t) r0 * b.hpitch * b.hesz;
-    if (b.hpitch == b.width) {
-      const size_t m = (size_t) nr * b.width;
-      if (up) convert(buf, b.desz, h, b.hesz, m);
-      else convert(h, b.hesz, buf, b.desz, m);
-      return;
-    }
-    for (long r = 0; r < nr; r++) {
-      char* hr = h + (size_t) r * b.hpitch * b.hesz;
-      char* br = (char*) buf + (size_t) r * row_bytes;
-      if (up) convert(br, b.desz, hr, b.hesz, b.width);
-      else convert(hr, b.hesz, br, b.desz, b.width);
-    }
-  };
   auto work = [&](int k) {
     Lane& l = g_stage.lane[k];
     if (hipSetDevice(dev) != hipSuccess) {
@@ -175,13 +218,9 @@ int copy_block(const Block& b, bool up) {
     }
     auto dma = [&](int q, long c) {
       const long r0 = c * per, nr = std::min(per, b.rows - r0);
-      char* d = b.dev + (size_t) r0 * b.dpitch * b.desz;
-      const hipError_t e =
-          up ? hipMemcpy2DAsync(d, (size_t) b.dpitch * b.desz, l.buf[q], row_bytes, row_bytes, nr,
-                                hipMemcpyHostToDevice, b.st)
-             : hipMemcpy2DAsync(l.buf[q], row_bytes, d, (size_t) b.dpitch * b.desz, row_bytes, nr,
-                                hipMemcpyDeviceToHost, b.st);
-      if (e != hipSuccess || hipEventRecord(l.ev[q], b.st) != hipSuccess) bad = 1;
+      if (copy_rows(b, up, l.buf[q], row_bytes, r0, nr) != hipSuccess ||
+          hipEventRecord(l.ev[q], b.st) != hipSuccess)
+        bad = 1;
     };
     int q = 0;
     if (!up && k < nslab) dma(0, k);
@@ -189,19 +228,19 @@ int copy_block(const Block& b, bool up) {
       const long r0 = c * per, nr = std::min(per, b.rows - r0);
       if (up) {
         if (c >= k + 2L * n && hipEventSynchronize(l.ev[q]) != hipSuccess) bad = 1;
-        host_copy(l.buf[q], r0, nr);
+        host_rows(b, up, l.buf[q], r0, nr);
         if (!bad) dma(q, c);
       } else {
         if (c + n < nslab) dma(q ^ 1, c + n);  // its buffer was emptied a slab ago
         if (hipEventSynchronize(l.ev[q]) != hipSuccess) bad = 1;
-        if (!bad) host_copy(l.buf[q], r0, nr);
+        if (!bad) host_rows(b, up, l.buf[q], r0, nr);
       }
     }
   };
   on_threads(n, work);
   // (the buffers are free again once the stream is past the copies)
   if ((up || bad) && hipStreamSynchronize(b.st) != hipSuccess) bad = 1;
-  return bad ? hydro_amd_set_error("%s copy failed", up ? "host-to-device" : "device-to-host") : 0;
+  return bad ? copy_error(up) : 0;
 }
 
 int staged(char* host, int hesz, char* dev, int desz, long pitch, long width, long rows,
