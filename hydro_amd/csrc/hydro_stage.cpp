@@ -44,35 +44,49 @@ constexpr size_t kThreadBytes = 3u << 19;
 struct Lane {
   void* buf[2] = {nullptr, nullptr};
   hipEvent_t ev[2] = {nullptr, nullptr};
+  int dev = -1;  // the events' device: a stream records only its own device's
 };
 struct Stage {
   std::mutex mu;  // one staged copy at a time per process
   Lane lane[kLanes];
-  int ready = 0;  // lanes that have their buffers
 };
 Stage g_stage;
 
-void lane_free(Lane& l) {
-  if (l.buf[0]) (void) hipHostFree(l.buf[0]);  // one allocation
-  for (hipEvent_t e : l.ev)
+void drop_events(Lane& l) {
+  for (hipEvent_t& e : l.ev) {
     if (e) (void) hipEventDestroy(e);
-  l = Lane();
+    e = nullptr;
+  }
+  l.dev = -1;
 }
 
-// Up to n lanes; how many there are (0: no pinned memory).
-int lanes_for(int n) {
-  for (; g_stage.ready < n; g_stage.ready++) {
-    Lane& l = g_stage.lane[g_stage.ready];
-    if (hipHostMalloc(&l.buf[0], 2 * kSlabBytes, hipHostMallocDefault) != hipSuccess ||
-        hipEventCreateWithFlags(&l.ev[0], hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&l.ev[1], hipEventDisableTiming) != hipSuccess) {
-      (void) hipGetLastError();
-      lane_free(l);
-      break;
+// The lane's buffers, and events of the current device `dev`.
+bool lane_ready(Lane& l, int dev) {
+  if (!l.buf[0]) {
+    if (hipHostMalloc(&l.buf[0], 2 * kSlabBytes, hipHostMallocPortable) != hipSuccess) {
+      l.buf[0] = nullptr;
+      return false;
     }
-    l.buf[1] = (char*) l.buf[0] + kSlabBytes;
+    l.buf[1] = (char*) l.buf[0] + kSlabBytes;  // one allocation
   }
-  return std::min(n, g_stage.ready);
+  if (l.dev == dev) return true;
+  drop_events(l);
+  if (hipEventCreateWithFlags(&l.ev[0], hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&l.ev[1], hipEventDisableTiming) != hipSuccess) {
+    drop_events(l);
+    return false;
+  }
+  l.dev = dev;
+  return true;
+}
+
+// Up to n lanes for copies on device `dev`, the current one; how many there are
+// (0: no pinned memory).
+int lanes_for(int n, int dev) {
+  int k = 0;
+  while (k < n && lane_ready(g_stage.lane[k], dev)) k++;
+  if (k < n) (void) hipGetLastError();
+  return k;
 }
 
 // n elements of sesz bytes to desz bytes (4 or 8 each).
@@ -198,17 +212,16 @@ int copy_pageable(const Block& b, bool up) {
   return 0;
 }
 
-int copy_block(const Block& b, bool up) {
+// dev: the stream's device, the current one.
+int copy_block(const Block& b, int dev, bool up) {
   const size_t row_bytes = (size_t) b.width * b.desz;
-  int n = lanes_for(thread_count((size_t) b.width * b.rows * b.hesz));
+  int n = lanes_for(thread_count((size_t) b.width * b.rows * b.hesz), dev);
   if (n < 1) return copy_pageable(b, up);
   // slabs small enough that every thread has two or more
   const long per = std::max(1L, std::min((long) (kSlabBytes / row_bytes),
                                          (b.rows + 2L * n - 1) / (2L * n)));
   const long nslab = (b.rows + per - 1) / per;
   n = (int) std::min<long>(n, nslab);
-  int dev = 0;
-  (void) hipGetDevice(&dev);
   std::atomic<int> bad{0};
   auto work = [&](int k) {
     Lane& l = g_stage.lane[k];
@@ -245,14 +258,22 @@ int copy_block(const Block& b, bool up) {
 
 int staged(char* host, int hesz, char* dev, int desz, long pitch, long width, long rows,
            hipStream_t st, bool up) {
-  std::lock_guard<std::mutex> lk(g_stage.mu);
-  const long most = (long) (kSlabBytes / desz);  // columns at a time
-  for (long c = 0; c < width; c += most) {
-    const Block b{host + (size_t) c * hesz, hesz, width, dev + (size_t) c * desz, desz, pitch,
-                  std::min(most, width - c), rows, st};
-    if (copy_block(b, up)) return -1;
+  int current = 0, device = 0;  // (a stream may be another device's than the current one)
+  if (hipGetDevice(&current) != hipSuccess || hipStreamGetDevice(st, &device) != hipSuccess ||
+      (device != current && hipSetDevice(device) != hipSuccess))
+    return copy_error(up);
+  int rc = 0;
+  {
+    std::lock_guard<std::mutex> lk(g_stage.mu);
+    const long most = (long) (kSlabBytes / desz);  // columns at a time
+    for (long c = 0; c < width && rc == 0; c += most) {
+      const Block b{host + (size_t) c * hesz, hesz, width, dev + (size_t) c * desz, desz, pitch,
+                    std::min(most, width - c), rows, st};
+      rc = copy_block(b, device, up);
+    }
   }
-  return 0;
+  if (device != current) (void) hipSetDevice(current);
+  return rc;
 }
 }  // namespace
 

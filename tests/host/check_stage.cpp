@@ -44,8 +44,31 @@ static int no_pinned_memory() {
   return 0;
 }
 
+// Streams of two devices in turn, whichever device is current.
+static int devices() {
+  hipStream_t st[2];
+  for (int d : {0, 1}) {
+    (void) hipSetDevice(d);
+    if (hipStreamCreateWithFlags(&st[d], 0) != hipSuccess) return 1;
+  }
+  for (int k = 0; k < 8; k++) {
+    const int of = k & 1, current = (k >> 1) & 1;
+    (void) hipSetDevice(current);
+    for (auto& s : kShapes)
+      if (!round_trip(st[of], s[0], s[1], 8)) {
+        printf("device %d's stream with device %d current\n", of, current);
+        return 2;
+      }
+    int now = -1;
+    (void) hipGetDevice(&now);
+    if (now != current) return 3;
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "no_pinned_memory") return no_pinned_memory();
+  if (which == "devices") return devices();
   return 99;
 }

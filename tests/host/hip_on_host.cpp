@@ -107,6 +107,11 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* st, unsigned) {
   *st = (hipStream_t) s;
   return hipSuccess;
 }
+hipError_t hipStreamGetDevice(hipStream_t st, hipDevice_t* d) {
+  ASK;
+  *d = of(st)->device;
+  return hipSuccess;
+}
 hipError_t hipStreamDestroy(hipStream_t st) {
   delete of(st);
   return hipSuccess;

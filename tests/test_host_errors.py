@@ -32,6 +32,6 @@ def test_batch_autotune_puts_the_controls_back(tmp_path):
     run_check(tmp_path, "check_batch_autotune.cpp", "hydro_batch.cpp")
 
 
-@pytest.mark.parametrize("check", ["no_pinned_memory"])
+@pytest.mark.parametrize("check", ["no_pinned_memory", "devices"])
 def test_staged_copies(tmp_path, check):
     run_check(tmp_path, "check_stage.cpp", "hydro_stage.cpp", check)
