@@ -263,7 +263,11 @@ int staged(char* host, int hesz, char* dev, int desz, long pitch, long width, lo
       (device != current && hipSetDevice(device) != hipSuccess))
     return copy_error(up);
   int rc = 0;
-  {
+  // Earlier work on the stream is waited for before the lanes are taken, which
+  // other threads' copies then do not wait for.
+  if (hipStreamSynchronize(st) != hipSuccess) {
+    rc = copy_error(up);
+  } else {
     std::lock_guard<std::mutex> lk(g_stage.mu);
     const long most = (long) (kSlabBytes / desz);  // columns at a time
     for (long c = 0; c < width && rc == 0; c += most) {

@@ -5,6 +5,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <chrono>
+#include <future>
 #include <string>
 #include <vector>
 
@@ -66,9 +68,45 @@ static int devices() {
   return 0;
 }
 
+// A copy whose stream has work queued before it holds up no other thread's copy.
+static int busy_stream(bool up) {
+  hipStream_t busy, idle;
+  if (hipStreamCreateWithFlags(&busy, 0) != hipSuccess ||
+      hipStreamCreateWithFlags(&idle, 0) != hipSuccess)
+    return 1;
+  std::vector<double> host(64 * 64), dev(64 * 64);
+  std::promise<void> reached;
+  bool told = false;
+  // (the copy has come as far as its stream's queued work)
+  onhost::refuse = [&](const char* name) {
+    if (!told && (!strcmp(name, "hipStreamSynchronize") || !strcmp(name, "hipEventSynchronize"))) {
+      told = true;
+      reached.set_value();
+    }
+    return false;
+  };
+  onhost::hold(busy, true);
+  auto first = std::async(std::launch::async, [&] {
+    return up ? stage_h2d(dev.data(), 8, 64, host.data(), 8, 64, 64, busy)
+              : stage_d2h(host.data(), 8, dev.data(), 8, 64, 64, 64, busy);
+  });
+  reached.get_future().wait();
+  auto second = std::async(std::launch::async, [&] { return round_trip(idle, 100, 80, 8); });
+  const bool free = second.wait_for(std::chrono::seconds(10)) == std::future_status::ready;
+  const bool waiting = first.wait_for(std::chrono::seconds(0)) != std::future_status::ready;
+  onhost::hold(busy, false);
+  if (!free || !waiting || !second.get() || first.get()) {
+    printf("up %d: other thread free %d, the copy waits %d\n", up, free, waiting);
+    return 2;
+  }
+  return 0;
+}
+
 int main(int argc, char** argv) {
   const std::string which = argc > 1 ? argv[1] : "";
   if (which == "no_pinned_memory") return no_pinned_memory();
   if (which == "devices") return devices();
+  if (which == "busy_upload") return busy_stream(true);
+  if (which == "busy_download") return busy_stream(false);
   return 99;
 }

@@ -1,5 +1,5 @@
-"""The library's host code against HIP calls that fail, on the CPU: its sources
-are compiled for the host alone and linked with a stand-in for the HIP runtime
+"""The library's host code against HIP calls that fail or wait, on the CPU: its
+sources are compiled for the host alone and linked with a stand-in for the HIP runtime
 (tests/host/hip_on_host.cpp)."""
 import os
 import shutil
@@ -32,6 +32,6 @@ def test_batch_autotune_puts_the_controls_back(tmp_path):
     run_check(tmp_path, "check_batch_autotune.cpp", "hydro_batch.cpp")
 
 
-@pytest.mark.parametrize("check", ["no_pinned_memory", "devices"])
+@pytest.mark.parametrize("check", ["no_pinned_memory", "devices", "busy_upload", "busy_download"])
 def test_staged_copies(tmp_path, check):
     run_check(tmp_path, "check_stage.cpp", "hydro_stage.cpp", check)
