@@ -631,7 +631,9 @@ __device__ __forceinline__ void trace_tail_scaled(const Q4<R>& q, const Q4<R>& d
   auto face = [&](R spm, R spp, R sp0, Q4<R>& x) {
     const R p = spp * ap, m = spm * am, s = p + m;  // -4 apr, -4 amr
     x.r = __builtin_fma(q4, __builtin_fma((R) 2, sp0 * a0r, s), q.r);
-    x.u = __builtin_fma(q4, (p - m) * OrOcc, q.u);
+    // (m - p, not p - m: the difference of equals is +0, as apr - amr is, and the
+    // face keeps the reference's zero where q.u is -0)
+    x.u = __builtin_fma(-q4, (m - p) * OrOcc, q.u);
     x.v = __builtin_fma(q2, sp0 * dq.v, q.v);
     x.p = __builtin_fma(q4, s * csq, q.p);
   };
@@ -691,7 +693,8 @@ __device__ __forceinline__ bool newton_step(double& pst, double pl, double pr, d
     const double h = P::divn(hr * hl, hr + hl) * (usl - usr);
     const double d = fmax(2.0 * h, -pst);
     pst += d;
-    // |d / (pst + smallpp)| > 1e-6 from products, whose error is 2^-13 of the
+    // |d / (pst + smallpp)| > 1e-6 from products: the roundings of the constant,
+    // the product and the quotient they stand for come to less than 2^-11 of the
     // margin; a wave with a lane inside the margin divides.
     const double s = pst + smallpp, a = fabs(d);
     const bool over = a > s * (1e-6 * (1.0 + 0x1p-40));
