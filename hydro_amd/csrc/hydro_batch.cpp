@@ -585,8 +585,9 @@ static int split_load(hydro_amd_batch* b) {
 }
 
 // Rebuilds the device instance array and the phase tables from the current
-// live set and their step parities (the stream must be idle).
-static int rebuild(hydro_amd_batch* b) {
+// live set and their step parities (the stream must be idle; the batch's device
+// the current one).
+static int rebuild_tables(hydro_amd_batch* b) {
   drop_graphs(b);
   b->live_ids.clear();
   b->maxid = -1;
@@ -673,6 +674,19 @@ static int rebuild(hydro_amd_batch* b) {
   b->flip = false;
   b->dirty = false;
   return 0;
+}
+
+// The same whichever device is current: what it makes on the way (task tables, the
+// second group's stream and its events) is the batch's device's.
+static int rebuild(hydro_amd_batch* b) {
+  int current = 0, own = 0;
+  BCHK(hipGetDevice(&current));
+  BCHK(hipStreamGetDevice(b->st, &own));
+  if (own == current) return rebuild_tables(b);
+  BCHK(hipSetDevice(own));
+  const int rc = rebuild_tables(b);
+  (void) hipSetDevice(current);
+  return rc;
 }
 
 static hipStream_t stream_of(const hydro_amd_batch* b, int q) { return q == 0 ? b->st : b->st2; }

@@ -35,3 +35,7 @@ def test_batch_autotune_puts_the_controls_back(tmp_path):
 @pytest.mark.parametrize("check", ["no_pinned_memory", "devices", "busy_upload", "busy_download"])
 def test_staged_copies(tmp_path, check):
     run_check(tmp_path, "check_stage.cpp", "hydro_stage.cpp", check)
+
+
+def test_batch_grows_with_another_device_current(tmp_path):
+    run_check(tmp_path, "check_batch_devices.cpp", "hydro_batch.cpp")
