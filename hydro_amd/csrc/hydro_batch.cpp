@@ -450,10 +450,13 @@ static bool folds_ghosts(const Inst& in) {
 // Large loads of the fast and mixed forms take whole steps instead (step_march;
 // for the line's reasons see step_rows, hydro_capi.cpp), in segments that fill the
 // 4096 waves the GPU holds twice, of at most 64 rows.  A step, sweeps and whole, the
-// best segment in brackets, of loads of so many wave rows: 49000 (30 grids of
-// 150-500) fast 92 and 92 us (8), mixed 67 and 65 (8); 219000 (60 of 64-1024) 364
-// and 305 (24), 224 and 209 (20-32); 1.07e6 (300 of 64-1024) 1772 and 1413 (64),
-// 1068 and 956 (96); 1.21e6 (24 of 128-4096) 2017 and 1552 (96), 1136 and 1021 (64).
+// best segment in brackets, of blasts in loads of so many wave rows: fast 46000 (30
+// grids of 150-500) 91 and 93 us (8), 68000 (40 of 150-550) 129 and 124 (8), 167000
+// (60 of 64-1024) 291 and 255 (20), 818000 (24 of 128-4096) 1365 and 1137 (64),
+// 967000 (300 of 64-1024) 1625 and 1352 (64); with flows that move everywhere 46000
+// 134 and 138, 68000 190 and 195, 167000 420 and 384.  Mixed 49000 67 and 65 (8),
+// 219000 224 and 209 (20-32), 1.07e6 1068 and 956 (96), 1.21e6 1136 and 1021 (64);
+// moving 167000 246 and 238, 818000 959 and 876.
 static void shape_by_load(hydro_amd_batch* b) {
   long segs = 0, wrows = 0, mrows = 0;
   bool fold = true;
@@ -820,7 +823,9 @@ extern "C" int hydro_amd_batch_run_async(hydro_amd_batch* b, int steps) {
   if (b->ngrp > 1) {
     // launch by launch: each group's run is one chain on its stream, met again
     // only at the run's end (two steps of both groups as one graph: 12 grids of
-    // 64-256, mixed, 43 us a step against 26; 60 of 64-1024, fast, 411 / 402)
+    // 64-256, mixed, 43 us a step against 26; 60 of 64-1024, fast, 411 / 402; two
+    // steps of each group as a graph on its own stream: half the host's time, 0.9 ms
+    // for 100 steps of those 12 instead of 2.0, but they take 2.69 ms instead of 2.50)
     if (fork_groups(b)) return -1;
     for (int k = 0; k < steps; k++) {
       for (int q = 0; q < b->ngrp; q++) enq_step(b, q, b->flip);

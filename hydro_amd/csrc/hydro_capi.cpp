@@ -462,26 +462,29 @@ static int march_rows(long ncol, long ny, long slots) {
   return (int) ((ny + nseg - 1) / nseg);
 }
 
-// How a whole step is launched on this grid (SweepTune::step).
+// How a whole step is launched on this grid (SweepTune::step).  Times below are of
+// a step, of a blast (in brackets: of a flow that moves everywhere).
 // Tiles save a launch and the y march's serial solves and pay with halo cells,
 // so they are for grids whose waves do not fill the GPU; counted in their waves,
-// the lines lie where they and the next were measured alike.  A step, tiles / two
-// sweeps, blast (a flow that moves everywhere): 250x125 FP64 20.8 / 23.5 us (17.8
-// / 21.8), fast 13.6 / 17.2, mixed 12.1 / 15.3; 500x500 (9000 waves) FP64 35.8 /
-// 41.1 (42.5 / 43.3), fast 24.8 / 27.1; 777x600 (15600) FP64 48.8 / 53.6 (58.6 /
-// 57.4), fast 32.2 / 35.6; mixed with 16 rows 500x500 18.3 / 21.5, 1021x767
-// (18400) 30.3 / 33.1, 1531x1200 (41600) 53.7 / 53.9.
+// the lines lie where they and the next were measured alike.  Tiles / two sweeps:
+// 250x125 FP64 21.3 / 23.5 us (17.4 / 21.4), fast 13.7 / 17.3 (12.6 / 16.4), mixed
+// 12.1 / 15.3; 500x500 (9000 waves) FP64 38.1 / 40.7 (48.2 / 47.6), fast 24.9 / 26.8
+// (28.8 / 30.5); 600x600 (12000) FP64 43.1 / 48.1 (55.2 / 56.5); 777x600 (15600) FP64
+// 48.6 / 51.8 (67.8 / 62.4), fast 31.2 / 34.3 (38.4 / 39.6); 850x700 (21000) fast 38.2 /
+// 39.0 (46.9 / 45.0); mixed with 16 rows 500x500 18.3 / 21.5, 1021x767 (18400) 30.3 /
+// 33.1, 1531x1200 (41600) 53.7 / 53.9.
 // The march passes over memory once a step instead of twice, which is what bounds
 // the large grids' sweeps in the fast form and half bounds them in the mixed
 // form (the FP64 form's arithmetic bounds it: no march).  March / two sweeps, fast:
-// 1021x767 (13800 wave rows) 40.7 / 40.1 (47.2 / 45.4), 1100x900 (17100) 45.7 /
-// 48.5 (53.0 / 54.6), 1400x1150 56.4 / 66.6 (67.9 / 76.8), 4099x3001 290 / 349,
-// 8192x1024 210 / 248, 8192x8192 1392 / 1794, 16384x12000 4010 / 5120; mixed:
-// 3400x2400 (137000) 144 / 144 (183 / 183), 3600x2600 (156000) 161 / 171 (206 /
-// 210), 4099x3001 204 / 219, 8192x8192 933 / 993, 16384x12000 2650 / 2810.  Its
-// waves update 60 columns, the sweeps' 63 and 64: in the mixed form, where that
-// counts, not where the grid's width makes it much worse (500x15000 145 / 142,
-// 192 / 176).
+// 1021x767 (13800 wave rows) 43.7 / 42.5 (57.3 / 50.1), 1100x900 (17100) 49.6 / 51.4
+// (65.5 / 61.0), 1150x950 (19000) 49.9 / 54.5 (64.7 / 62.9), 1400x1150 61.6 / 70.9
+// (83.3 / 85.4), 2048x1536 103 / 106 (146 / 145), 3200x2400 205 / 234 (310 / 322),
+// 4099x3001 317 / 364 (455 / 474), 8192x1024 228 / 257 (326 / 332), 8192x8192 1543 /
+// 1815 (1988 / 2077); mixed: 3400x2400 (137000) 144 / 144 (183 / 183), 3600x2600
+// (156000) 161 / 171 (206 / 210), 4099x3001 204 / 219, 8192x8192 933 / 993,
+// 16384x12000 2650 / 2810.  Its waves update 60 columns, the sweeps' 63 and 64: in
+// the mixed form, where that counts, not where the grid's width makes it much
+// worse (500x15000 145 / 142, 192 / 176).
 static int default_step(const hydro_amd_grid* g) {
   if (!folds_ghosts(g)) return 0;
   const long nx = g->p.nx, ny = g->p.ny, ncol = (nx + 59) / 60;

@@ -355,7 +355,9 @@ static int y_rows(long ncolblk, long ny, int most) {
 // at every size (8192x8192: 1.45 against 1.48 ms a sweep, 2048x1536: 200
 // against 212 us a step) and in the other forms on small and middle grids
 // (2048x1536: fast 119 against 123 us a step, mixed 85 against 88; 1021x767:
-// 68 / 71, 57 / 59); the four-wave form, with fewer halo cells, where there are
+// 68 / 71, 57 / 59; these and the four-wave form's figures are of two sweeps a
+// step, which such sizes take in a profile, with a given shape or in the mixed
+// form below its line in default_step); the four-wave form, with fewer halo cells, where there are
 // enough of its pieces to fill the GPU many times over (8192x1024, 33800
 // pieces: 285 / 288; 8192x8192 1.83 / 1.88 ms).  The number of pieces goes by
 // the square root, as y_rows; the best measured, one wave: 1 at 1021x767, 3 at
@@ -504,9 +506,13 @@ void launch_sweep(int idim, const GridGeom& g, const PhysArgs& pa, GridView<S> i
   // keeps the SIMDs busy.  A sweep of a small grid has too few waves for
   // that: each wave's march is latency-bound, and the gates' wave-wide
   // tests, branches and larger code lengthen it, so such launches run the
-  // kIeee kernels (the results are the same bits either way).  y sweep of a
-  // flow that moves everywhere, gated / IEEE, as part of a step: 250x125 22.5 /
-  // 21.8 us, 1021x767 (4096 waves) 72 / 72, 1531x1200 138 / 144, 2048x1536 218 / 229.
+  // kIeee kernels (the results are the same bits either way).  A step of a flow
+  // that moves everywhere (of a blast), every sweep gated / every sweep IEEE:
+  // 250x125 22.1 / 21.6 us (26.9 / 23.7), 500x500 45.8 / 49.3 (41.2 / 40.7), 777x600
+  // 59.9 / 66.9 (52.2 / 52.2), 1531x1200 151 / 167 (122 / 126), 2048x1536 232 / 265
+  // (178 / 188); x gated and y IEEE, as the line has it, 777x600 62.4 (51.8),
+  // 1021x767 (4096 y waves) 82.9 (67.4) against 80.6 (67.7) all gated: a lower line
+  // would gain 3 % on moving flows there and lose 1 % on blasts.
   constexpr long kFastDivWaves = 4096;  // 4 waves per SIMD on 256 CUs
   if constexpr (sizeof(S) == 8) {
     const long ncb = cdiv(g.nx, 64);

@@ -42,8 +42,8 @@ __device__ __forceinline__ void st_stream(S* p, S v) {
 // Element `off` bytes past a wave-uniform address: the address stays in scalar
 // registers and the access takes the lane's 32-bit offset (a 64-bit address a
 // lane and variable cost the y march 16 vector instructions a row of 290 in the
-// mixed form; a step of 4099x3001 without them: fast 287 and 280-285 us, mixed 202
-// and 197, FP64 567 and 563; 8192x8192 FP64 2.775 and 2.74-2.77 ms).
+// mixed form; a step of 4099x3001 with it and so: mixed 202 and 197 us, FP64 567 and
+// 563; 8192x8192 FP64 2.775 and 2.74-2.77 ms).
 template <typename S>
 __device__ __forceinline__ S ld_lane(const S* base, unsigned off) {
   return *reinterpret_cast<const S*>(reinterpret_cast<const char*>(base) + off);
@@ -931,8 +931,8 @@ __device__ __forceinline__ void tile_step(const GridGeom& g, const Phys<S>& ph,
 // same, and a row's x sweep (tile_x) comes before the row enters the window
 // (XY) or after it has left (y first).  Ghost cells as in tile_step.  The grid
 // passes through memory once a step: 64 bytes a cell in FP64 instead of the two
-// sweeps' 128, whose two passes alone took 1.76 of a step's 1.79 ms at 8192x8192
-// in the fast form; the march takes 1.39 ms.  The price is 64 / 60 in the y sweep
+// sweeps' 128, whose two passes alone took 1.76 ms of a step at 8192x8192 in the fast
+// form (with the arithmetic 1.8); the march takes 1.54 ms.  The price is 64 / 60 in the y sweep
 // and, with x first, four more rows of x sweeps a segment.
 template <typename S, bool ST1, bool COUR, bool XY, int FD>
 __device__ __forceinline__ void step_march(const GridGeom& g, const Phys<S>& ph,

@@ -154,7 +154,9 @@ int hydro_amd_batch_init_blast(hydro_amd_batch *b, int id, int bx, int by, doubl
 int hydro_amd_batch_upload(hydro_amd_batch *b, int id, const double *uold);
 int hydro_amd_batch_download(hydro_amd_batch *b, int id, double *uold);
 /* Advance every live instance by up to `steps` steps of its own time loop
- * (instances that reach tend / nstepmax stop; the rest go on). */
+ * (instances that reach tend / nstepmax stop; the rest go on).  run_async
+ * returns when the steps are queued: about 7 us of host time a step where the
+ * load is one group, 10 to 20 us where it is two. */
 int hydro_amd_batch_run(hydro_amd_batch *b, int steps);
 int hydro_amd_batch_run_async(hydro_amd_batch *b, int steps);
 int hydro_amd_batch_sync(hydro_amd_batch *b);
