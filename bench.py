@@ -18,16 +18,18 @@ reference's MC/s unit x 1e6) over the timed steps, run as the product runs
 them: replayed HIP graphs, no per-launch instrumentation, and where it is
 the faster way (large grids in the fast and mixed forms) each step in one
 launch.  `step_bytes` holds that step against the bytes it cannot do without
-(each cell read and written once).  Per-kernel
-durations come from a second, instrumented pass over the same grid (HIP
-events recorded on the grid's own stream around every launch), always of the
-two sweep kernels.  `roofline` is for the dominant one of those: algorithmic bytes (64 B per cell per sweep in
-FP64: read 4 doubles, write 4) over its average duration; its `traffic` is
-the HBM bytes the kernel really moves (two rocprofv3 --pmc passes,
-calibrated on a copy kernel), and its `copy_ceiling` the rate of a plain copy
-in the same access shape (the sweep's bytes with no arithmetic: what this
-pattern reaches on the machine, beside the published peak).  `valu` is that
-kernel's VALU work from a third counter pass.  `c2` is the 23000x23000 corner blast (50 steps).
+(each cell read and written once).  `roofline` is of the kernel that dominates
+the timed steps: where they are whole steps, of that launch (`whole_step`:
+64 B per cell in FP64, read 4 doubles, write 4, over the timed step); else of
+the longer of the two sweep kernels (64 B per cell and sweep, over its average
+launch).  Per-kernel durations (`kernels`) come from a second, instrumented
+pass over the same grid (HIP events recorded on the grid's own stream around
+every launch), always of the two sweep kernels; `sweeps` says how the longer of
+them fares.  The roofline's `traffic` is the HBM bytes its kernel really moves
+(two rocprofv3 --pmc passes, calibrated on a copy kernel), and its
+`copy_ceiling` the rate of a plain copy of the same bytes (four arrays in, four
+out, no arithmetic), beside the published peak.  `valu` is that kernel's VALU
+work from a third counter pass.  `c2` is the 23000x23000 corner blast (50 steps).
 `batched` and `serving` time the many-grid workloads (512 batched instances;
 256 Poisson arrivals at a nominal and a saturating rate, mixed precision)
 against the plain per-grid FP64 loop, timed cold (each grid created, run and
@@ -88,6 +90,7 @@ def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_
     t1 = time.perf_counter()
     assert done == steps, (done, steps)
     tstate = g.state()
+    whole = g.whole_steps()
     g.set_profile(True)
     g.run(prof_steps, log=False)
     prof = g.profile()
@@ -101,10 +104,12 @@ def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_
     ms, n = prof[kern]
     bpc = BYTES_PER_CELL_SWEEP[precision]
     per_launch_bytes = bpc * cells
-    avg_s = ms / n / 1e3
-    achieved = per_launch_bytes / avg_s / 1e9
+    achieved = per_launch_bytes / (ms / n / 1e3) / 1e9
+    step_GBps = cells * steps * bpc / elapsed / 1e9
     return {
         "tune": tune,
+        "whole": whole,
+        "launch_shape": "whole steps, by the grid's size" if whole else tune,
         "value": cells * steps / elapsed,
         "ms_per_step": elapsed / steps * 1e3,
         "elapsed_s": elapsed,
@@ -114,23 +119,26 @@ def gpu_bench(nx, ny, steps, warmup, precision, autotune=True, testcase=0, prof_
         "kernels_note": f"instrumented pass of {prof_steps} steps after the timed region, "
                         "by the two sweep kernels",
         "step_bytes": {"bytes_per_cell": bpc,
-                       "achieved_GBps": round(cells * steps * bpc / elapsed / 1e9, 1),
-                       "frac": round(cells * steps * bpc / elapsed / 1e9 / HBM_PEAK_GBS, 4)},
-        "roofline": {"bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
-                     "traffic": None, "kernel": kern,
+                       "achieved_GBps": round(step_GBps, 1),
+                       "frac": round(step_GBps / HBM_PEAK_GBS, 4)},
+        "roofline": {"bound": "hbm", "achieved": round(step_GBps if whole else achieved, 2),
+                     "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                     "frac": round((step_GBps if whole else achieved) / HBM_PEAK_GBS, 4),
+                     "traffic": None, "kernel": "whole_step" if whole else kern,
                      "algorithmic_bytes_per_launch": per_launch_bytes,
-                     "bytes_per_cell_sweep": bpc},
-        # (the bytes of two sweeps, whatever the step's launches)
-        "step_roofline_frac": round(cells * steps * 2 * bpc / elapsed / 1e9 / HBM_PEAK_GBS, 4),
+                     "bytes_per_cell_launch": bpc},
+        "sweeps": {"kernel": kern, "achieved_GBps": round(achieved, 2),
+                   "frac": round(achieved / HBM_PEAK_GBS, 4), "in_timed_steps": not whole},
+        # the timed launches' algorithmic bytes: one pass over the grid a step, or two
+        "step_roofline_frac": round((1 if whole else 2) * step_GBps / HBM_PEAK_GBS, 4),
     }
 
 
 def form_summary(r, precision):
     return {"form": FORM_NAMES[precision], "value": r["value"], "ms_per_step": r["ms_per_step"],
             "roofline_frac": r["roofline"]["frac"], "step_roofline_frac": r["step_roofline_frac"],
-            "step_bytes": r["step_bytes"],
-            "kernels": r["kernels"], "launch_shape": r["tune"]}
+            "step_bytes": r["step_bytes"], "sweeps": r["sweeps"],
+            "kernels": r["kernels"], "launch_shape": r["launch_shape"]}
 
 
 def batched_bench(n=512, steps=100):
@@ -433,7 +441,7 @@ COPY_PROBE_BYTES = 1 << 30  # each of read and written by pmc_workload's copy ke
 
 def _pmc(counters, args):
     """{counter: {kernel: mean value per dispatch}} from one rocprofv3 --pmc
-    run of this script with `args` (kernels: copy, x_sweep, y_sweep), or None
+    run of this script with `args` (kernels: copy, x_sweep, y_sweep, whole_step), or None
     if the profiler is absent or fails."""
     import csv
     import shutil
@@ -456,7 +464,8 @@ def _pmc(counters, args):
             for r in csv.DictReader(f):
                 name = r["Kernel_Name"]
                 key = ("copy" if "k_copy_probe" in name else "x_sweep" if "k_sweep_x" in name
-                       else "y_sweep" if "k_sweep_y" in name else None)
+                       else "y_sweep" if "k_sweep_y" in name
+                       else "whole_step" if "k_step" in name else None)
                 if key and r.get("Counter_Name") in counters:
                     acc.setdefault(r["Counter_Name"], {}).setdefault(key, []).append(
                         float(r["Counter_Value"]))
@@ -469,8 +478,8 @@ def _pmc_kib(counter, args):
 
 
 def measured_traffic(nx, precision, tune):
-    """HBM bytes per launch of each sweep kernel: rocprofv3 FETCH_SIZE and
-    WRITE_SIZE passes over pmc_workload, each scaled by what the same counter
+    """HBM bytes per launch of each kernel of a step (tune None: the grid's own
+    launches): rocprofv3 FETCH_SIZE and WRITE_SIZE passes over pmc_workload, each scaled by what the same counter
     reads for the copy kernel (COPY_PROBE_BYTES read and written)."""
     args = ["--steps", "2", "--nx", str(nx), "--precision", PREC_ARG[precision]]
     if tune:
@@ -480,7 +489,7 @@ def measured_traffic(nx, precision, tune):
         return None
     out = {"fetch_scale": COPY_PROBE_BYTES / (fetch["copy"] * 1024),
            "write_scale": COPY_PROBE_BYTES / (write["copy"] * 1024)}
-    for k in ("x_sweep", "y_sweep"):
+    for k in ("x_sweep", "y_sweep", "whole_step"):
         if k in fetch and k in write:
             out[k] = (fetch[k] * 1024 * out["fetch_scale"] + write[k] * 1024 * out["write_scale"])
     return out
@@ -494,7 +503,7 @@ XCDS = 8                  # GRBM_GUI_ACTIVE is summed over the XCDs
 
 
 def measured_valu(nx, precision, tune, kern, avg_s):
-    """VALU work of the sweep kernel `kern` from one rocprofv3 --pmc pass over
+    """VALU work of the kernel `kern` from one rocprofv3 --pmc pass over
     pmc_workload: VALU instructions per cell, FP64 FLOP/s (FMA = 2) over the
     kernel's measured duration `avg_s`, and the share of SIMD cycles issuing
     VALU, counting each wave64 instruction at 4 cycles (a 16-lane SIMD; the
@@ -586,10 +595,11 @@ def main():
                                f"{FORM_NAMES[prec]}, CFL 0.8, reflective walls",
                    "form": FORM_NAMES[prec], "nx": a.nx, "ny": ny, "testcase": a.testcase,
                    "steps_timed": a.steps, "first_timed_step": a.warmup,
-                   "launch_shape": r["tune"], "timed_path": "replayed HIP graphs"},
+                   "launch_shape": r["launch_shape"], "timed_path": "replayed HIP graphs"},
         "roofline": r["roofline"],
         "step_roofline_frac": r["step_roofline_frac"],
         "step_bytes": r["step_bytes"],
+        "sweeps": r["sweeps"],
         "kernels": r["kernels"],
         "kernels_note": r["kernels_note"],
     }
@@ -599,7 +609,7 @@ def main():
     ceil = hydro_amd.stream_probe((a.nx + 4) * (ny + 4), 10)
     line["roofline"]["copy_ceiling"] = {
         "GBps": round(ceil, 1), "frac": round(line["roofline"]["achieved"] / ceil, 4),
-        "kernel": "k_stream_probe: a copy in the sweep's access shape (4 arrays of "
+        "kernel": "k_stream_probe: a plain copy of the same bytes (4 arrays of "
                   f"{(a.nx + 4) * (ny + 4)} doubles in, 4 out, one cell per thread, "
                   "non-temporal loads and stores), 64 bytes per cell"}
     progress(f"streaming-copy ceiling {ceil:.0f} GB/s")
@@ -621,14 +631,16 @@ def main():
         line["c2"] = {"workload": "23000x23000 corner blast, 50 steps (33.9 GB of FP64 state "
                                   "in HBM)", **c2}
     if not a.no_traffic:
-        tr = measured_traffic(a.nx, prec, r["tune"])
+        shape = None if r["whole"] else r["tune"]
+        tr = measured_traffic(a.nx, prec, shape)
         kern = line["roofline"]["kernel"]
         if tr and kern in tr:
             line["roofline"]["traffic"] = round(tr[kern])
             line["roofline"]["traffic_note"] = (
                 "HBM bytes per launch from rocprofv3 FETCH_SIZE + WRITE_SIZE, scaled by "
                 f"{tr['fetch_scale']:.3f} / {tr['write_scale']:.3f} (copy-kernel calibration)")
-        va = measured_valu(a.nx, prec, r["tune"], kern, r["kernels"][kern]["avg_ms"] / 1e3)
+        va = measured_valu(a.nx, prec, shape, kern,
+                           (r["ms_per_step"] if r["whole"] else r["kernels"][kern]["avg_ms"]) / 1e3)
         if va:
             line["valu"] = va
         progress("rocprofv3 traffic and VALU passes done")

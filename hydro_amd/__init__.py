@@ -147,6 +147,7 @@ def lib() -> C.CDLL:
                        ("hydro_amd_grid_set_tune", [G, C.c_int, C.c_int, C.c_int, C.c_int]),
                        ("hydro_amd_grid_set_profile", [G, C.c_int]),
                        ("hydro_amd_grid_autotune", [G, C.c_int, C.c_void_p]),
+                       ("hydro_amd_grid_whole_steps", [G]),
                        ("hydro_amd_grid_profile", [G, _dp, C.POINTER(C.c_longlong)])]:
         fn = getattr(L, name)
         fn.argtypes = args
@@ -322,6 +323,10 @@ class Grid:
         best = (C.c_int * 4)()
         _check(lib().hydro_amd_grid_autotune(self._h, reps, C.cast(best, C.c_void_p)))
         return dict(zip(("yseg", "ywaves", "xwaves", "xiter"), list(best)))
+
+    def whole_steps(self) -> bool:
+        """Whether runs of this grid take each step in one launch."""
+        return bool(lib().hydro_amd_grid_whole_steps(self._h))
 
     def set_profile(self, on: bool) -> None:
         _check(lib().hydro_amd_grid_set_profile(self._h, int(on)))

@@ -503,9 +503,16 @@ static int default_step(const hydro_amd_grid* g) {
              : 0;
 }
 
-static int step_rows(const hydro_amd_grid* g) {
-  if (g->prof) return 0;  // (profiles are of the sweeps)
+static int unprofiled_rows(const hydro_amd_grid* g) {
   return g->tune.step >= 0 ? g->tune.step : default_step(g);
+}
+
+static int step_rows(const hydro_amd_grid* g) {
+  return g->prof ? 0 : unprofiled_rows(g);  // (profiles are of the sweeps)
+}
+
+extern "C" int hydro_amd_grid_whole_steps(const hydro_amd_grid* g) {
+  return g && unprofiled_rows(g) > 0;
 }
 
 // hydro_godunov.c:98-237: both directions, ghosts refilled before each, on the

@@ -118,6 +118,9 @@ int hydro_amd_grid_set_tune(hydro_amd_grid *g, int yseg, int ywaves, int xwaves,
  * steps, keeps the fastest and caches it per (nx, ny, precision) for the process.  best[4] (may be NULL)
  * receives yseg, ywaves, xwaves, xiter. */
 int hydro_amd_grid_autotune(hydro_amd_grid *g, int reps, int *best);
+/* 1 if runs of this grid take each step in one launch (whole steps), 0 if in two
+ * sweeps. */
+int hydro_amd_grid_whole_steps(const hydro_amd_grid *g);
 /* Kernel timing with HIP events recorded on the grid's own stream around
  * every x-sweep, y-sweep, ghost-fill and CFL launch (graph replay and whole
  * steps are off while enabled; ghosts are filled by launches of their own only
@@ -155,7 +158,7 @@ int hydro_amd_batch_upload(hydro_amd_batch *b, int id, const double *uold);
 int hydro_amd_batch_download(hydro_amd_batch *b, int id, double *uold);
 /* Advance every live instance by up to `steps` steps of its own time loop
  * (instances that reach tend / nstepmax stop; the rest go on).  run_async
- * returns when the steps are queued: about 7 us of host time a step where the
+ * returns when the steps are queued: about 6 us of host time a step where the
  * load is one group, 10 to 20 us where it is two. */
 int hydro_amd_batch_run(hydro_amd_batch *b, int steps);
 int hydro_amd_batch_run_async(hydro_amd_batch *b, int steps);
